@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 #include <atomic>
 #include <cstdint>
+#include <type_traits>
 
 #include "ckr_internal.h"
 #include "ckr_table.h"
@@ -1279,73 +1280,109 @@ struct FastEncParams {
 
 // Encode table entry in LDS, 16 bytes, every field ready for its instruction
 // (one ds_read_b128 per symbol): x = rcp; y = cmpl | rsh << 24 (the 24-bit
-// multiply reads cmpl, the shift reads byte 3); z = bias; w = 8f (the
-// renormalisation compares read it against bytes of the state).  See EncSym:
-// cmpl = M - f, rsh < 12, bias < 8192; w = 0 marks f == 0.
+// multiply reads cmpl, the shift reads byte 3); z = bias; w = D, from which the
+// emitted bytes follow without a comparison (enc_bytes).  See EncSym: cmpl = M
+// - f, rsh < 12, bias < 8192.
+//
+// n, the bytes a state x in [2^23, 2^31 + 2^13) emits before a symbol of count
+// f, is (x >= f << 19) + (x >= f << 27).  Only one of the two is ever open: for
+// f > 16 the second bound is above every x, for f <= 16 the first is at most
+// every x.  So n = base + (x >> 16 >= T), base = 0, T = 8f or base = 1, T = 2048f,
+// and, x >> 16 being below 2^16, n = (x >> 16) + D >> 16 with D = (base + 1) *
+// 65536 - T.  D = 65536 (n = 1 for every x) marks f == 0, the raw-byte escape.
+constexpr uint32_t ENC_ESC = 65536u;
 __device__ __forceinline__ uint4 enc_quad(const EncSym& e) {
-    return make_uint4(e.rcp, (e.cmpl_rsh & 0xFFFu) | ((e.cmpl_rsh >> 16) << 24), e.bias, e.xmax >> 16);
+    const uint32_t f = e.xmax >> 19;
+    const uint32_t d = f > 16u ? 65536u - 8u * f : (f ? 131072u - 2048u * f : ENC_ESC);
+    return make_uint4(e.rcp, (e.cmpl_rsh & 0xFFFu) | ((e.cmpl_rsh >> 16) << 24), e.bias, d);
+}
+__device__ __forceinline__ uint32_t enc_bytes(uint32_t x, uint32_t d) { return ((x >> 16) + d) >> 16; }
+// The state after a symbol, from the state xr its n bytes left.
+__device__ __forceinline__ uint32_t enc_next(uint32_t xr, uint4 t) {
+    const uint32_t q = __umulhi(xr, t.x) >> (t.y >> 24);
+    return __umul24(q, t.y) + (xr + t.z);
+}
+
+// LDS by address (byte offset in the workgroup's LDS), for values that an
+// instruction computed whole: no base is added.
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+__device__ __forceinline__ void lds_put(uint32_t a, uint32_t v) { *(lds_u32*)(uintptr_t)a = v; }
+// Entry 16 * (byte SH / 8 of w) of the table at LDS address 0: the entry's
+// address is one SDWA shift (the compiler's own form is two instructions).
+template <uint32_t SH>
+__device__ __forceinline__ uint4 enc_entry_of(uint32_t w) {
+    uint32_t a;
+    if constexpr (SH == 8) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(a) : "v"(4u), "v"(w));
+    else if constexpr (SH == 16) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(a) : "v"(4u), "v"(w));
+    else asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3" : "=v"(a) : "v"(4u), "v"(w));
+    const u32x4 t = *(lds_u32x4*)(uintptr_t)a;
+    return make_uint4(t.x, t.y, t.z, t.w);
 }
 
 // Lane coder state.  x: rANS state.  {hi, lo}: the last 8 bytes emitted, the
-// newest in the top byte of hi.  sel: v_perm selector 0x08090A0B - P*0x01010101
-// with P (0..7) the emitted bytes not yet flushed (the top P bytes of the
-// window).  ptr: LDS byte address of the lane's next flushed dword.
+// newest in the top byte of hi.  a: LDS address of the newest byte (the slot's
+// end before the first): the stream grows downward.
+//
+// The slot holds the stream with the bytes of each aligned dword in reverse
+// order (the byte of address a is at a ^ 3), as they lie in the window, so that
+// a dword is stored as it is shifted out; the packer waves turn them round
+// (lds_read16).
+//
+// Instruction issue bounds the coder waves (a wave issues one instruction in
+// about 4.2 cycles whether or not it depends on the one before; v_mul_hi_u32
+// takes 6.5), so the row's instruction count is its time: 12 a row here
+// (address, 2 for n, 3 window shifts, 5 for the state, and half of the 5 of
+// enc_flush) against 20 with two comparisons per row and a selector that
+// tracked the pending bytes.  Measured: a 64 KiB unit coded in 12.7 us instead
+// of 14.8; the encode of a 436 MB bf16 layer 231 -> 202 us, of a 67 MB fp32
+// tensor 57 -> 52, pass 2 of a 1 GiB fp32 tensor in 1 MiB units 761 -> 650 and
+// pass 1 288 -> 246.  The packer waves are then as slow as the coders.
 struct EncLane {
-    uint32_t x, hi, lo, sel, ptr;
+    uint32_t x, hi, lo, a;
 };
 
 // One symbol of rans_encode_kernel's loop body (ANSCompressor.cpp:180-202)
-// without branches, from the table entry t (see enc_quad).  Renormalisation
-// emits n in {0,1,2} bytes: x >= f*2^19 and x >= f*2^27 are (x >> 16) >= 8f
-// and (x >> 24) >= 8f.  The n low bytes of x, low byte first (the reference's
-// emission order), enter the window from the top: one v_alignbyte per register
-// shifts by n bytes.  ESC: the table may give f == 0 to a symbol of the data
-// (raw-byte escape, no state update, :185-192); tables built from the data
-// itself never do.
+// without branches, from the table entry t (see enc_quad).  The n low bytes of
+// x, low byte first (the reference's emission order), enter the window from the
+// top: one v_alignbyte per register shifts by n bytes.  ESC: the table may give
+// f == 0 to a symbol of the data (raw-byte escape, no state update, :185-192);
+// tables built from the data itself never do.  Returns n.
+template <bool ESC>
+__device__ __forceinline__ uint32_t enc_window(uint32_t& x, uint32_t& hi, uint32_t& lo, uint32_t sym, uint4 t) {
+    const uint32_t n = enc_bytes(x, t.w);
+    const bool esc = ESC && t.w == ENC_ESC;
+    const uint32_t ins = esc ? sym : x;
+    const uint32_t xr = __builtin_amdgcn_alignbyte(0u, x, n);
+    lo = __builtin_amdgcn_alignbyte(hi, lo, n);
+    hi = __builtin_amdgcn_alignbyte(ins, hi, n);
+    const uint32_t xn = enc_next(xr, t);
+    x = esc ? x : xn;
+    return n;
+}
 template <bool ESC>
 __device__ __forceinline__ void enc_step(EncLane& s, uint32_t sym, uint4 t) {
-    const uint32_t f8 = t.w;
-    const uint32_t x = s.x;
-    uint32_t n4 = ((x >> 24) >= f8) ? 0x02020202u : (((x >> 16) >= f8) ? 0x01010101u : 0u);
-    uint32_t ins = x;
-    bool esc = false;
-    if (ESC) {
-        esc = f8 == 0u;
-        n4 = esc ? 0x01010101u : n4;
-        ins = esc ? sym : x;
-    }
-    const uint32_t xr = __builtin_amdgcn_alignbyte(0u, x, n4);
-    s.lo = __builtin_amdgcn_alignbyte(s.hi, s.lo, n4);
-    s.hi = __builtin_amdgcn_alignbyte(ins, s.hi, n4);
-    s.sel -= n4;
-    const uint32_t q = __umulhi(xr, t.x) >> (t.y >> 24);
-    const uint32_t xn = xr + t.z + __umul24(q, t.y);
-    s.x = (ESC && esc) ? x : xn;
+    s.a -= enc_window<ESC>(s.x, s.hi, s.lo, sym, t);
 }
 
-// Flush the 4 oldest pending bytes when P >= 4 (called at least every 2
-// symbols, so P <= 7).  The dword holds them in stream order (the newest at the
-// lowest address): a byte-reversing select out of the 8-byte window.
-// The dword is stored whatever P: with P < 4 it lands at the lane's next
-// flush position, which a later flush or the final partial dword overwrites,
-// or, when the stream ends on a dword boundary, just below the stream (in the
-// slot, its padding or the guard).  P >= 4 exactly when bit 3 of the
-// selector's low byte (0x0B - P) is clear.
-__device__ __forceinline__ void enc_flush(EncLane& s, uint8_t* lds8) {
-    *reinterpret_cast<uint32_t*>(lds8 + s.ptr) = __builtin_amdgcn_perm(s.hi, s.lo, s.sel);
-    const bool fl = (s.sel & 8u) == 0u;
-    s.ptr -= fl ? 4u : 0u;
-    s.sel += fl ? 0x04040404u : 0u;
+// After at most two symbols (4 bytes): store the lowest dword that lies wholly
+// above the newest byte's own dword, (a & ~3) + 4, whose bytes begin 4 - (a & 3)
+// behind the newest.  At most one new dword has got there since the last call;
+// when none has, the same dword is stored again, unchanged (before the first
+// byte, the 4 bytes from slot end + 4, in the slot's padding).  The newest
+// byte's own dword, whole or partial, is left to a later flush or enc_finish.
+__device__ __forceinline__ void enc_flush(const EncLane& s) {
+    lds_put((s.a & ~3u) + 4u, __builtin_amdgcn_alignbyte(s.hi, s.lo, s.a));
 }
 
-// End of the lane: the remaining P (< 4 after a flush) bytes go into the top of
-// one more dword (its lower bytes lie before the stream's start).  Returns the
-// byte count; the stream then occupies [slot_end - count, slot_end).
-__device__ __forceinline__ uint32_t enc_finish(EncLane& s, uint8_t* lds8, uint32_t slot_end) {
-    enc_flush(s, lds8);
-    const uint32_t P = 0x0Bu - (s.sel & 0xFFu);
-    *reinterpret_cast<uint32_t*>(lds8 + s.ptr) = __builtin_amdgcn_perm(s.hi, s.lo, s.sel);
-    return (slot_end - 4u - s.ptr) + P;
+// End of the lane: the newest byte's dword (the bytes of it below the stream
+// are not part of it).  Returns the byte count; the stream then occupies
+// [slot_end - count, slot_end).
+__device__ __forceinline__ uint32_t enc_finish(EncLane& s, uint32_t slot_end) {
+    enc_flush(s);
+    lds_put(s.a & ~3u, __builtin_amdgcn_alignbyte(0u, s.hi, s.a));
+    return slot_end - s.a;
 }
 
 // Look-back status words.  Their values carry everything the protocol needs
@@ -1438,13 +1475,16 @@ __device__ uint64_t lookback_wave(uint64_t* status, uint64_t n_units, uint64_t u
     return excl;
 }
 
-// 16 LDS bytes from an arbitrary byte address (5 aligned 32-bit reads).
+// 16 stream bytes from LDS byte address a of a slot, whose aligned dwords hold
+// their bytes in reverse order (EncLane): 5 dwords, then one byte select per
+// dword out of two neighbours, the stream's next bytes from the top of the
+// first down.
 __device__ __forceinline__ uint4 lds_read16(const uint8_t* lds8, uint32_t a) {
     const uint32_t* w = reinterpret_cast<const uint32_t*>(lds8 + (a & ~3u));
-    const uint32_t sh = a & 3u;
+    const uint32_t sel = 0x04050607u - (a & 3u) * 0x01010101u;
     const uint32_t d0 = w[0], d1 = w[1], d2 = w[2], d3 = w[3], d4 = w[4];
-    return make_uint4(__builtin_amdgcn_alignbyte(d1, d0, sh), __builtin_amdgcn_alignbyte(d2, d1, sh),
-                      __builtin_amdgcn_alignbyte(d3, d2, sh), __builtin_amdgcn_alignbyte(d4, d3, sh));
+    return make_uint4(__builtin_amdgcn_perm(d0, d1, sel), __builtin_amdgcn_perm(d1, d2, sel),
+                      __builtin_amdgcn_perm(d2, d3, sel), __builtin_amdgcn_perm(d3, d4, sel));
 }
 
 // Bytes [s, 16) of r over those of v (0 <= s < 16): one bitfield insert per
@@ -1459,42 +1499,36 @@ __device__ __forceinline__ uint4 merge16_from(uint4 v, uint4 r, uint32_t s) {
 }
 
 
-// Coding of the live lanes of every column of a unit whose rows are all full
+// Coding of one live lane of every column of a unit whose rows are all full
 // (length a multiple of 256, so every column has the same nrows rows).  P = 0:
-// byte FL of each column (chain c0); P = 1: byte 3 (chain c0); P = 2: both
-// (c0: byte FL, c1: byte 3, interleaved).  Rows are taken from the top down.
+// byte FL of each column; P = 1: byte 3.  Rows are taken from the top down.
 // The rows above the highest multiple of GR go one at a time; then groups of
 // GR rows, the next group's loads in flight while the current one is coded
-// (loads and table reads are unconditional, so the waits stay exact), and each
-// TB-row batch's table entries read while the batch before it is coded.
-// Pending bytes are flushed after every second row.  The sidecar rows are
-// written by the thread coding plane 0 and 1 alternately (row k by P == k & 1),
-// or all of them when P = 2.
-template <int SPE, bool ESC, bool SIDE, int P, int GR, int TB, int NBUF>
-__device__ __forceinline__ void enc_full_rows(EncLane& c0, EncLane& c1, const uint8_t* ucol, uint8_t* sidecar,
-                                              uint64_t ubase, uint32_t j, uint32_t nrows, const uint4* tab,
-                                              uint8_t* lds8) {
+// (loads and table reads are unconditional, so the waits stay exact), and a
+// row's table entry read TR - 1 rows before it is coded, through a ring of TR
+// entries that carries over from group to group (the LDS serves it in about 50
+// cycles when idle, 100 and more beside the packers' reads; a row takes about
+// 55).  Emitted bytes are stored after every second row.  The sidecar rows are
+// written by the thread coding plane 0 and 1 alternately (row k by P == k & 1).
+template <int SPE, bool ESC, bool SIDE, int P, int GR, int TR>
+__device__ __forceinline__ void enc_full_rows(EncLane& c, const uint8_t* ucol, uint8_t* sidecar, uint64_t ubase,
+                                              uint32_t j, uint32_t nrows) {
     constexpr int FL = SPE == 2 ? 2 : 1;
-    constexpr uint32_t SH0 = P == 1 ? 24u : 8u * FL;  // byte of chain c0
-    constexpr uint32_t SH1 = 24u;                     // byte of chain c1 (P = 2)
+    constexpr uint32_t SH = P == 1 ? 24u : 8u * FL;   // this lane's byte of the column
     const uint32_t* in32 = reinterpret_cast<const uint32_t*>(ucol);          // row k at in32[64 k]
     uint16_t* sc16 = SIDE ? reinterpret_cast<uint16_t*>(sidecar + (ubase >> 1) + 2 * j) : nullptr;  // row k at sc16[64 k]
     auto side = [&](uint16_t* p, uint32_t wd) {
         if (SIDE) *p = (uint16_t)(SPE == 2 ? (wd & 0xFFFFu) : ((wd & 0xFFu) | ((wd >> 8) & 0xFF00u)));
     };
-    auto mine = [&](uint32_t k) { return P == 2 || (k & 1u) == (uint32_t)P; };  // sidecar row k written here
-    static_assert(GR % TB == 0 && TB % 2 == 0 && GR % 2 == 0, "row groups of whole table batches");
+    static_assert(GR % TR == 0 && GR % 2 == 0, "row groups of whole turns of the ring");
     const uint32_t ng = nrows / GR;  // full groups: rows [0, GR ng)
     for (int32_t k = (int32_t)nrows - 1; k >= (int32_t)(GR * ng); k--) {
         const uint32_t wd = in32[64 * k];
-        if (mine((uint32_t)k)) side(sc16 + 64 * k, wd);
-        const uint32_t s0 = (wd >> SH0) & 255u;
-        enc_step<ESC>(c0, s0, tab[s0]);
-        if (P == 2) { const uint32_t s1 = wd >> SH1; enc_step<ESC>(c1, s1, tab[s1]); }
-        if ((k & 1) == 0) { enc_flush(c0, lds8); if (P == 2) enc_flush(c1, lds8); }
+        if (((uint32_t)k & 1u) == (uint32_t)P) side(sc16 + 64 * k, wd);
+        enc_step<ESC>(c, (wd >> SH) & 255u, enc_entry_of<SH>(wd));
+        if ((k & 1) == 0) enc_flush(c);
     }
-    enc_flush(c0, lds8);
-    if (P == 2) enc_flush(c1, lds8);
+    enc_flush(c);
     if (ng == 0) return;
     // group g: rows GR g + GR - 1 (r[0]) down to GR g (r[GR - 1])
     auto load = [&](uint32_t (&r)[GR], uint32_t g) {
@@ -1502,67 +1536,35 @@ __device__ __forceinline__ void enc_full_rows(EncLane& c0, EncLane& c1, const ui
 #pragma unroll
         for (int i = 0; i < GR; i++) r[i] = p[-64 * i];
     };
-    auto code = [&](const uint32_t (&r)[GR], uint32_t g) {
-        uint4 t0[2][TB], t1[2][TB];
-        (void)t1;
-        auto fetch = [&](int buf, int i0) {
-#pragma unroll
-            for (int i = 0; i < TB; i++) {
-                t0[buf][i] = tab[(r[i0 + i] >> SH0) & 255u];
-                if (P == 2) t1[buf][i] = tab[r[i0 + i] >> SH1];
-            }
-        };
+    uint4 t[TR];  // entry of row i of a group at t[i % TR]
+    // rn: the next group's rows (the group's own again when it is the last)
+    auto code = [&](const uint32_t (&r)[GR], const uint32_t (&rn)[GR], uint32_t g) {
         uint16_t* scp = SIDE ? sc16 + 64 * (GR * g + GR - 1) : nullptr;
-        constexpr int NB = GR / TB;
-        fetch(0, 0);
 #pragma unroll
-        for (int bt = 0; bt < NB; bt++) {
-            if (bt < NB - 1) fetch((bt + 1) & 1, TB * (bt + 1));
-#pragma unroll
-            for (int i = 0; i < TB; i++) {
-                const int ii = TB * bt + i;              // row GR g + GR - 1 - ii: parity (ii & 1) ^ 1
-                if (P == 2 || ((ii & 1) ^ 1) == P) side(scp - 64 * ii, r[ii]);
-                enc_step<ESC>(c0, (r[ii] >> SH0) & 255u, t0[bt & 1][i]);
-                if (P == 2) enc_step<ESC>(c1, r[ii] >> SH1, t1[bt & 1][i]);
-                if (i & 1) { enc_flush(c0, lds8); if (P == 2) enc_flush(c1, lds8); }
-            }
+        for (int i = 0; i < GR; i++) {  // row GR g + GR - 1 - i: parity (i & 1) ^ 1
+            constexpr int A = TR - 1;
+            t[(i + A) % TR] = enc_entry_of<SH>(i + A < GR ? r[i + A] : rn[i + A - GR]);
+            if (((i & 1) ^ 1) == P) side(scp - 64 * i, r[i]);
+            // the scheduler would move the read down to just before its use
+            __builtin_amdgcn_sched_barrier(0);
+            enc_step<ESC>(c, (r[i] >> SH) & 255u, t[i % TR]);
+            if (i & 1) enc_flush(c);
         }
     };
-    if (NBUF == 2) {
-        uint32_t ra[GR], rb[GR];
-        uint32_t g = ng - 1;
-        load(ra, g);
-        for (;;) {
-            if (g == 0) { code(ra, 0); break; }
-            load(rb, g - 1);
-            code(ra, g);
-            g--;
-            if (g == 0) { code(rb, 0); break; }
-            load(ra, g - 1);
-            code(rb, g);
-            g--;
-        }
-    } else {
-        // three buffers: group g - 2's loads issued while group g is coded (the
-        // last groups load group 0 again, so that every load is unconditional)
-        uint32_t ra[GR], rb[GR], rc[GR];
-        int32_t g = (int32_t)ng - 1;
-        load(ra, (uint32_t)g);
-        load(rb, (uint32_t)max(g - 1, 0));
-        for (;;) {
-            load(rc, (uint32_t)max(g - 2, 0));
-            code(ra, (uint32_t)g);
-            if (g == 0) break;
-            g--;
-            load(ra, (uint32_t)max(g - 2, 0));
-            code(rb, (uint32_t)g);
-            if (g == 0) break;
-            g--;
-            load(rb, (uint32_t)max(g - 2, 0));
-            code(rc, (uint32_t)g);
-            if (g == 0) break;
-            g--;
-        }
+    uint32_t ra[GR], rb[GR];
+    uint32_t g = ng - 1;
+    load(ra, g);
+#pragma unroll
+    for (int i = 0; i < TR - 1; i++) t[i] = enc_entry_of<SH>(ra[i]);
+    for (;;) {
+        if (g == 0) { code(ra, ra, 0); break; }
+        load(rb, g - 1);
+        code(ra, rb, g);
+        g--;
+        if (g == 0) { code(rb, rb, 0); break; }
+        load(ra, g - 1);
+        code(rb, ra, g);
+        g--;
     }
 }
 
@@ -1592,8 +1594,8 @@ __device__ __forceinline__ void enc_full_rows(EncLane& c0, EncLane& c1, const ui
 // by the general kernels) and, for the lowest slot, into the lane tables (at
 // most 2 bytes per symbol, 256 symbols: 516 bytes), never out of its region.
 static constexpr uint32_t FE_TABSZ = 4096, FE_CHDR = FE_TABSZ, FE_CBYTES = FE_TABSZ + 48;
-// Rows per load group and per table batch of the fast encoder's coders.
-static constexpr int ENC_GR = 32, ENC_TB = 2, ENC_NBUF = 2;
+// Rows per load group of the fast encoder's coders, entries of their table ring.
+static constexpr int ENC_GR = 32, ENC_TR = 4;
 // Packer waves per coder pair.  With four, a workgroup of two pairs is 12
 // waves (3 per SIMD); the coders are held to 128 VGPRs (4 waves per SIMD) so
 // that the overlapped histogram's wave still fits on every SIMD beside them.
@@ -1627,9 +1629,9 @@ __device__ __forceinline__ void ws_signal(uint32_t* p, uint32_t v, uint32_t lane
     if (lane == 0) (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// 4 bytes between slots: a stream that fills its slot exactly still writes one
-// dword below its start (the final partial dword, empty)
-__host__ __device__ constexpr uint32_t slot_stride(uint32_t sl) { return sl + 4; }
+// 8 bytes of padding above each slot, where a lane that has emitted nothing yet
+// stores (enc_flush, enc_finish)
+__host__ __device__ constexpr uint32_t slot_stride(uint32_t sl) { return sl + 8; }
 __host__ __device__ constexpr uint32_t ws_ctl_offset(uint32_t canon_bytes) {
     return (FE_CBYTES + 3 * canon_bytes + 15u) & ~15u;
 }
@@ -1688,7 +1690,8 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
         uint32_t* cb32 = reinterpret_cast<uint32_t*>(lds8 + cb_off);
         const uint32_t ncb = 3 * fp.canon_bytes / 4;
         const uint32_t cb_per = fp.canon_bytes / 4;
-        for (uint32_t i = tid; i < ncb; i += NT) cb32[i] = cs[(i / cb_per) * fp.cw + (i % cb_per)];
+        // (as in the slots, the bytes of each dword in reverse order)
+        for (uint32_t i = tid; i < ncb; i += NT) cb32[i] = __builtin_bswap32(cs[(i / cb_per) * fp.cw + (i % cb_per)]);
         if (tid < 12) chdr[tid] = canon[(tid >> 2) * (4 + fp.cw) + (tid & 3)];
         uint32_t* c32 = reinterpret_cast<uint32_t*>(lds8 + ctl_off);
         for (uint32_t i = tid; i < PAIRS * (uint32_t)sizeof(WsPairCtl) / 4; i += NT) c32[i] = 0;
@@ -1736,12 +1739,11 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
             const uint32_t rb = reg0 + (2 * pr + s) * rbytes;
             const uint32_t endw = rl ? rb + R_SLOTS + 64 * fp.stride0 + j * fp.stride1 + fp.sl1
                                      : rb + R_SLOTS + j * fp.stride0 + fp.sl0;
-            EncLane c{L, 0u, 0u, 0x08090A0Bu, endw - 4u};
-            EncLane c_unused = c;
+            EncLane c{L, 0u, 0u, endw};
             const uint32_t K = len > col ? (len - col + 255) / 256 : 0u;
             if ((len & 255u) == 0) {
-                if (rl == 0) enc_full_rows<SPE, ESC, SIDE, 0, ENC_GR, ENC_TB, ENC_NBUF>(c, c_unused, usrc + col, sidecar, ubase, j, len >> 8, tab, lds8);
-                else enc_full_rows<SPE, ESC, SIDE, 1, ENC_GR, ENC_TB, ENC_NBUF>(c, c_unused, usrc + col, sidecar, ubase, j, len >> 8, tab, lds8);
+                if (rl == 0) enc_full_rows<SPE, ESC, SIDE, 0, ENC_GR, ENC_TR>(c, usrc + col, sidecar, ubase, j, len >> 8);
+                else enc_full_rows<SPE, ESC, SIDE, 1, ENC_GR, ENC_TR>(c, usrc + col, sidecar, ubase, j, len >> 8);
             } else {
                 // A tensor's last unit: rows from the top down, one at a time; the top
                 // row may be partial (bf16: lane 4j+3 has one symbol fewer).
@@ -1755,10 +1757,10 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
                     v &= lm;
                     const uint32_t sy = (v >> sh) & 255u;
                     if (rl == 0 || nvalid == 4) enc_step<ESC>(c, sy, tab[sy]);
-                    if ((k & 1) == 0) enc_flush(c, lds8);
+                    if ((k & 1) == 0) enc_flush(c);
                 }
             }
-            const uint32_t e = enc_finish(c, lds8, endw);
+            const uint32_t e = enc_finish(c, endw);
             // per column: count FL, state FL, count 3, state 3, in the set's lane-record
             // area (the records are written only after every packer wave has read
             // them; it lies below the guard that an outgrown lowest slot may write into)
@@ -2229,18 +2231,9 @@ __host__ __device__ constexpr uint32_t seg_count(uint64_t unit) {
 // enc_step's state update without the bytes: returns how many it emits.
 template <bool ESC>
 __device__ __forceinline__ uint32_t seg_size_step(uint32_t& x, uint4 t) {
-    const uint32_t f8 = t.w;
-    uint32_t n = ((x >> 24) >= f8) ? 2u : (((x >> 16) >= f8) ? 1u : 0u);
-    const uint32_t xr = x >> (8u * n);
-    const uint32_t q = __umulhi(xr, t.x) >> (t.y >> 24);
-    const uint32_t xn = xr + t.z + __umul24(q, t.y);
-    if (ESC) {
-        const bool esc = f8 == 0u;
-        n = esc ? 1u : n;
-        x = esc ? x : xn;
-    } else {
-        x = xn;
-    }
+    const uint32_t n = enc_bytes(x, t.w);
+    const uint32_t xn = enc_next(__builtin_amdgcn_alignbyte(0u, x, n), t);
+    x = ESC && t.w == ENC_ESC ? x : xn;
     return n;
 }
 
@@ -2393,7 +2386,8 @@ __global__ void __launch_bounds__(256) seg_size_kernel(const uint8_t* __restrict
 static constexpr uint32_t SEG_LINE = 64;  // bytes a line buffer holds (a multiple of 16)
 
 struct SegLane {
-    EncLane c;
+    uint32_t x, hi, lo;  // state and window (EncLane)
+    uint32_t sel;        // v_perm selector 0x08090A0B - P * 0x01010101, P (0..7) the bytes not yet flushed
     int32_t go;    // next dword to flush (offset from the unit's output base, aligned in memory)
     int32_t rs;    // the run's first byte
     int32_t e;     // one past its last byte
@@ -2403,11 +2397,10 @@ struct SegLane {
 
 __device__ __forceinline__ void seg_lane_init(SegLane& l, uint32_t x, int32_t rs, int32_t e, uint32_t ua, uint32_t lb) {
     const uint32_t a = (0u - (ua + (uint32_t)e)) & 3u;
-    l.c.x = x;
-    l.c.hi = 0;
-    l.c.lo = 0;
-    l.c.sel = 0x08090A0Bu - a * 0x01010101u;
-    l.c.ptr = 0;
+    l.x = x;
+    l.hi = 0;
+    l.lo = 0;
+    l.sel = 0x08090A0Bu - a * 0x01010101u;
     l.go = e + (int32_t)a - 4;
     l.rs = rs;
     l.e = e;
@@ -2428,16 +2421,23 @@ __device__ __attribute__((noinline)) void seg_line_bytes(const uint8_t* lds8, ui
     }
 }
 
-// One flush.  Returns the line start (offset) when this flush completed a
-// line (wrote its first dword), else INT32_MIN.
+template <bool ESC>
+__device__ __forceinline__ void seg_step(SegLane& l, uint32_t sym, uint4 t) {
+    l.sel -= enc_window<ESC>(l.x, l.hi, l.lo, sym, t) * 0x01010101u;
+}
+
+// One flush: the 4 oldest pending bytes when P >= 4 (bit 3 of the selector's low
+// byte, 0x0B - P, is then clear), in stream order.  Returns the line start
+// (offset) when this flush completed a line (wrote its first dword), else
+// INT32_MIN.
 __device__ __forceinline__ int32_t seg_flush(SegLane& l, uint8_t* lds8, uint32_t ua) {
-    const uint32_t v = __builtin_amdgcn_perm(l.c.hi, l.c.lo, l.c.sel);
-    const bool fl = (l.c.sel & 8u) == 0u;
+    const uint32_t v = __builtin_amdgcn_perm(l.hi, l.lo, l.sel);
+    const bool fl = (l.sel & 8u) == 0u;
     const uint32_t o = (ua + (uint32_t)l.go) & (SEG_LINE - 1);
     *reinterpret_cast<uint32_t*>(lds8 + l.lb + o) = v;
     const int32_t done = (fl && o == 0u) ? l.go : INT32_MIN;
     l.go -= fl ? 4 : 0;
-    l.c.sel += fl ? 0x04040404u : 0u;
+    l.sel += fl ? 0x04040404u : 0u;
     return done;
 }
 
@@ -2479,8 +2479,8 @@ __device__ __forceinline__ void seg_lines_out(SegLane& l0, SegLane& l1, int32_t 
 // into the buffer, and the bytes below the lowest line written out.  True when
 // they end exactly at the run start.
 __device__ __forceinline__ bool seg_finish_lane(SegLane& l, uint8_t* lds8, uint32_t ua, uint8_t* ud) {
-    const uint32_t P = 0x0Bu - (l.c.sel & 0xFFu);  // < 4 after the last flush
-    const uint32_t v = __builtin_amdgcn_perm(l.c.hi, l.c.lo, l.c.sel);  // its top P bytes
+    const uint32_t P = 0x0Bu - (l.sel & 0xFFu);  // < 4 after the last flush
+    const uint32_t v = __builtin_amdgcn_perm(l.hi, l.lo, l.sel);  // its top P bytes
     *reinterpret_cast<uint32_t*>(lds8 + l.lb + ((ua + (uint32_t)l.go) & (SEG_LINE - 1))) = v;
     const bool ok = l.go + 4 - (int32_t)P == l.rs && l.lc - l.rs <= (int32_t)SEG_LINE;
     if (ok && l.rs < l.lc) seg_line_bytes(lds8, l.lb, ua, ud, l.rs, l.lc);
@@ -2609,14 +2609,14 @@ __device__ void seg_code_item(const uint8_t* __restrict__ src, const EncodeGeom&
                 for (uint32_t b = 0; b < nv; b++) wd |= (uint32_t)p[b] << (8 * b);
                 write_sidecar_row<SPE>(sidecar, ubase + 256ull * kf + 4 * j, wd, nv);
             }
-            if (4 * j + FL < r) { const uint32_t sy = p[FL]; enc_step<ESC>(l0.c, sy, tab[sy]); }
-            if (4 * j + 3 < r) { const uint32_t sy = p[3]; enc_step<ESC>(l1.c, sy, tab[sy]); }
+            if (4 * j + FL < r) { const uint32_t sy = p[FL]; seg_step<ESC>(l0, sy, tab[sy]); }
+            if (4 * j + 3 < r) { const uint32_t sy = p[3]; seg_step<ESC>(l1, sy, tab[sy]); }
             flush2();
         }
         auto row = [&](uint32_t k, uint32_t wd, uint4 t0, uint4 t1) {
             side(k, wd);
-            enc_step<ESC>(l0.c, (wd >> SH0) & 255u, t0);
-            enc_step<ESC>(l1.c, wd >> 24, t1);
+            seg_step<ESC>(l0, (wd >> SH0) & 255u, t0);
+            seg_step<ESC>(l1, wd >> 24, t1);
         };
         const uint32_t nf = fhi - lo, ng = nf >> 4;
         for (int32_t k = (int32_t)fhi - 1; k >= (int32_t)(lo + 16 * ng); k--) {
@@ -2666,8 +2666,8 @@ __device__ void seg_code_item(const uint8_t* __restrict__ src, const EncodeGeom&
             }
         }
         flush2();
-        const bool ok0 = seg_finish_lane(l0, lds8, ua, ud) && l0.c.x == n0.x;
-        const bool ok1 = seg_finish_lane(l1, lds8, ua, ud) && l1.c.x == n1.x;
+        const bool ok0 = seg_finish_lane(l0, lds8, ua, ud) && l0.x == n0.x;
+        const bool ok1 = seg_finish_lane(l1, lds8, ua, ud) && l1.x == n1.x;
         if (!(ok0 && ok1)) atomicOr(aux, 1u);
     }
     // the zero-plane lanes copy their canonical stream: thread j those of
@@ -2776,7 +2776,7 @@ seg_fast_kernel(const uint8_t* __restrict__ src, EncodeGeom g, const EncSym* __r
     const uint32_t lm = live_mask32<SPE>();
     const uint32_t Kf = (uint32_t)(g.unit >> 8);  // rows of a whole unit: every lane's symbol count
     {   // table (EncSym → enc_quad), the canonical stream of Kf zero symbols (byte
-        // order, at FE_CBYTES), control blocks
+        // order, each dword's bytes reversed as in the slots, at FE_CBYTES), control blocks
         const uint4* d_tab = reinterpret_cast<const uint4*>(d_enc);
         uint4* wt = reinterpret_cast<uint4*>(lds8);
         for (uint32_t k = tid; k < 256; k += NT) {
@@ -2786,7 +2786,7 @@ seg_fast_kernel(const uint8_t* __restrict__ src, EncodeGeom g, const EncSym* __r
         }
         const uint32_t* cs = canon + 3 * (4 + cw) + canon_index(canon, cw, Kf) * cw;
         uint32_t* cb32 = reinterpret_cast<uint32_t*>(lds8 + FE_CBYTES);
-        for (uint32_t i = tid; i < fp.canon_bytes / 4; i += NT) cb32[i] = cs[i];
+        for (uint32_t i = tid; i < fp.canon_bytes / 4; i += NT) cb32[i] = __builtin_bswap32(cs[i]);
         uint32_t* c32 = reinterpret_cast<uint32_t*>(lds8 + ctl_off);
         for (uint32_t i = tid; i < PAIRS * (uint32_t)sizeof(WsPairCtl) / 4; i += NT) c32[i] = 0;
     }
@@ -2882,12 +2882,11 @@ seg_fast_kernel(const uint8_t* __restrict__ src, EncodeGeom g, const EncSym* __r
                 } else {
                     const uint32_t endw = rl ? rb + R_SLOTS + 64 * fp.stride0 + j * fp.stride1 + fp.sl1
                                              : rb + R_SLOTS + j * fp.stride0 + fp.sl0;
-                    EncLane c{x0, 0u, 0u, 0x08090A0Bu, endw - 4u};
-                    EncLane c_unused = c;
+                    EncLane c{x0, 0u, 0u, endw};
                     if (full) {
                         const uint8_t* ucol = src + ubase + col;
-                        if (rl == 0) enc_full_rows<SPE, ESC, true, 0, ENC_GR, ENC_TB, ENC_NBUF>(c, c_unused, ucol, sidecar, ubase, j, 256, tab, lds8);
-                        else enc_full_rows<SPE, ESC, true, 1, ENC_GR, ENC_TB, ENC_NBUF>(c, c_unused, ucol, sidecar, ubase, j, 256, tab, lds8);
+                        if (rl == 0) enc_full_rows<SPE, ESC, true, 0, ENC_GR, ENC_TR>(c, ucol, sidecar, ubase, j, 256);
+                        else enc_full_rows<SPE, ESC, true, 1, ENC_GR, ENC_TR>(c, ucol, sidecar, ubase, j, 256);
                     } else {
                         // the top segment of a partial last unit: rows from the top down,
                         // one at a time (as in encode_fast_kernel); the top row may be
@@ -2906,10 +2905,10 @@ seg_fast_kernel(const uint8_t* __restrict__ src, EncodeGeom g, const EncSym* __r
                             v &= lm;
                             const uint32_t sy = (v >> sh) & 255u;
                             if (rl == 0 || nvalid == 4) enc_step<ESC>(c, sy, tab[sy]);
-                            if ((k & 1) == 0) enc_flush(c, lds8);
+                            if ((k & 1) == 0) enc_flush(c);
                         }
                     }
-                    e = enc_finish(c, lds8, endw);
+                    e = enc_finish(c, endw);
                     flag = (e == xch[X_LEN + li] && c.x == xch[X_FLAG + li]) ? 0u : 2u;
                     if (flag) e = 0;  // nothing is copied from a lane off its checkpoints
                 }
@@ -3750,6 +3749,54 @@ __global__ void __launch_bounds__(256) dec_setup_multi_kernel(DecSetupJobs J, Ch
 static constexpr uint32_t LU_SEG = 1024;  // rows per segment (a multiple of 32)
 static constexpr uint32_t LU_CH = 130;    // chains per unit: 64 columns x 2 live lanes, 2 zero-plane counts
 
+// The chain of one lane (byte SH / 8 of its column) over the 32 ng rows at
+// in32, from the top down: groups of 32 rows, the next two groups' loads in
+// flight while one is coded, and each row's table entry read 7 rows ahead.
+// record(s) at the entry of every segment.  A row is 9.5 VALU instructions and
+// one LDS read, all on one wave: instruction issue (about 4.2 cycles each) is
+// what bounds the chain.  A 33.5 MB bf16 tensor (131072 rows): 4.90 ms with
+// enc_step's earlier form (15 instructions) and entries 4 rows ahead in the
+// source but sunk to their use, 4.18 with 9.5 instructions, 3.2 with this ring.
+template <bool ESC, uint32_t SH, typename R>
+__device__ __forceinline__ void lu_chain_rows(uint32_t& x, uint32_t& e, const uint32_t* in32, uint32_t ng, R&& record) {
+    constexpr int TR = 8;
+    auto load = [&](uint32_t (&rr)[32], uint32_t gi) __attribute__((always_inline)) {
+        const uint32_t* p = in32 + 64 * (32 * (uint64_t)gi + 31);
+#pragma unroll
+        for (int i = 0; i < 32; i++) rr[i] = p[-64 * i];
+    };
+    uint4 t[TR];  // entry of row i of a group at t[i % TR]
+    // rn: the rows of the group after (its own again for the last)
+    auto code = [&](const uint32_t (&rr)[32], const uint32_t (&rn)[32], uint32_t gi) __attribute__((always_inline)) {
+        if ((32 * gi + 32) % LU_SEG == 0) record((32 * gi + 31) / LU_SEG);
+#pragma unroll
+        for (int i = 0; i < 32; i++) {
+            constexpr int A = TR - 1;
+            t[(i + A) % TR] = enc_entry_of<SH>(i + A < 32 ? rr[i + A] : rn[i + A - 32]);
+            // the scheduler would move the read down to just before its use
+            __builtin_amdgcn_sched_barrier(0);
+            e += seg_size_step<ESC>(x, t[i % TR]);
+        }
+    };
+    uint32_t ra[32], rb[32], rc[32];
+    int32_t gi = (int32_t)ng - 1;
+    load(ra, (uint32_t)gi);
+    load(rb, (uint32_t)max(gi - 1, 0));
+#pragma unroll
+    for (int i = 0; i < TR - 1; i++) t[i] = enc_entry_of<SH>(ra[i]);
+    for (;;) {
+        load(rc, (uint32_t)max(gi - 2, 0));
+        code(ra, rb, (uint32_t)gi);
+        if (--gi < 0) break;
+        load(ra, (uint32_t)max(gi - 2, 0));
+        code(rb, rc, (uint32_t)gi);
+        if (--gi < 0) break;
+        load(rb, (uint32_t)max(gi - 2, 0));
+        code(rc, ra, (uint32_t)gi);
+        if (--gi < 0) break;
+    }
+}
+
 // Record slots: rec[(u * S + s) * LU_CH + c] = {state, bytes emitted so far}
 // of chain c of unit u at the entry of segment s (before its top row is
 // coded); c = 64 p + j for live lane p (0: byte FL, 1: byte 3) of column j,
@@ -3759,7 +3806,8 @@ __global__ void __launch_bounds__(64) lu_chain_kernel(const uint8_t* __restrict_
                                                       const EncSym* __restrict__ d_enc, uint32_t S,
                                                       uint2* __restrict__ rec, ckr_stream_header* __restrict__ hdrs,
                                                       uint32_t* __restrict__ err) {
-    __shared__ uint4 tab[256];
+    extern __shared__ uint4 lu_tab[];  // at LDS address 0 (enc_entry_of)
+    uint4* tab = lu_tab;
     for (uint32_t i = threadIdx.x; i < 256; i += 64) tab[i] = enc_quad(d_enc[i]);
     if (blockIdx.x == 0 && threadIdx.x == 0) *err = 0;  // pass 2 runs after this grid
     __syncthreads();
@@ -3817,44 +3865,12 @@ __global__ void __launch_bounds__(64) lu_chain_kernel(const uint8_t* __restrict_
         if ((uint32_t)(k + 1) % LU_SEG == 0) record((uint32_t)k / LU_SEG);
         e += seg_size_step<ESC>(x, tab[(in32[64 * (uint64_t)k] >> sh) & 255u]);
     }
-    // groups of 32 rows from the top down, the next two groups' loads in flight
-    // while one is coded; table entries read 4 rows ahead
-    auto load = [&](uint32_t (&rr)[32], uint32_t gi) __attribute__((always_inline)) {
-        const uint32_t* p = in32 + 64 * (32 * (uint64_t)gi + 31);
-#pragma unroll
-        for (int i = 0; i < 32; i++) rr[i] = p[-64 * i];
-    };
-    auto code = [&](const uint32_t (&rr)[32], uint32_t gi) __attribute__((always_inline)) {
-        if ((32 * gi + 32) % LU_SEG == 0) record((32 * gi + 31) / LU_SEG);
-        uint4 ta[2][4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) ta[0][i] = tab[(rr[i] >> sh) & 255u];
-#pragma unroll
-        for (int bt = 0; bt < 8; bt++) {
-            if (bt < 7) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) ta[(bt + 1) & 1][i] = tab[(rr[4 * (bt + 1) + i] >> sh) & 255u];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) e += seg_size_step<ESC>(x, ta[bt & 1][i]);
-        }
-    };
     if (ng) {
-        uint32_t ra[32], rb[32], rc[32];
-        int32_t gi = (int32_t)ng - 1;
-        load(ra, (uint32_t)gi);
-        if (gi >= 1) load(rb, (uint32_t)gi - 1);
-        for (;;) {
-            if (gi >= 2) load(rc, (uint32_t)gi - 2);
-            code(ra, (uint32_t)gi);
-            if (--gi < 0) break;
-            if (gi >= 2) load(ra, (uint32_t)gi - 2);
-            code(rb, (uint32_t)gi);
-            if (--gi < 0) break;
-            if (gi >= 2) load(rb, (uint32_t)gi - 2);
-            code(rc, (uint32_t)gi);
-            if (--gi < 0) break;
-        }
+        auto run = [&](auto sh_c) __attribute__((always_inline)) {
+            lu_chain_rows<ESC, decltype(sh_c)::value>(x, e, in32, ng, record);
+        };
+        if (role == 0) run(std::integral_constant<uint32_t, 8u * FL>{});
+        else run(std::integral_constant<uint32_t, 24u>{});
     }
     ckr_stream_header h;
     h.final_state = x;
@@ -3948,17 +3964,14 @@ __global__ void __launch_bounds__(256) lu_code_kernel(const uint8_t* __restrict_
         if (live) sym = (uint32_t)k < kf ? (*reinterpret_cast<const uint32_t*>(us + 256ull * k + 4 * j) >> sh) & 255u
                                          : us[256ull * k + l];
         const uint4 t = tab[sym];
-        const uint32_t f8 = t.w;
-        if (ESC && f8 == 0u) {  // raw-byte escape (ANSCompressor.cpp:185-192)
+        if (ESC && t.w == ENC_ESC) {  // raw-byte escape (ANSCompressor.cpp:185-192)
             put(sym);
             continue;
         }
-        const uint32_t n = ((x >> 24) >= f8) ? 2u : (((x >> 16) >= f8) ? 1u : 0u);
+        const uint32_t n = enc_bytes(x, t.w);
         if (n >= 1) put(x & 255u);
         if (n == 2) put((x >> 8) & 255u);
-        const uint32_t xr = x >> (8 * n);
-        const uint32_t q = __umulhi(xr, t.x) >> (t.y >> 24);
-        x = xr + t.z + __umul24(q, t.y);
+        x = enc_next(x >> (8 * n), t);
     }
     if (hi - pos != (uintptr_t)(e1 - st.y) || x != xend) atomicOr(err, 1u);
 }
@@ -3973,7 +3986,7 @@ static hipError_t encode_long_t(const uint8_t* src, const EncodeGeom& g, const E
                                 ckr_stream_header* hdrs, uint32_t* unit_size, uint64_t* unit_off, uint8_t* sidecar,
                                 uint8_t* out, uint32_t* err, hipStream_t s) {
     const uint32_t S = encode_long_segments(g.unit);
-    CKR_LAUNCH("lu_chain_kernel", s, lu_chain_kernel<SPE, ESC><<<(uint32_t)(3 * g.n_units), 64, 0, s>>>(src, g, d_enc, S, rec, hdrs, err));
+    CKR_LAUNCH("lu_chain_kernel", s, lu_chain_kernel<SPE, ESC><<<(uint32_t)(3 * g.n_units), 64, 4096, s>>>(src, g, d_enc, S, rec, hdrs, err));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     CKR_LAUNCH("unit_finalize_kernel", s, unit_finalize_kernel<<<(uint32_t)g.n_units, 256, 0, s>>>(g, 0, hdrs, unit_size, nullptr));
