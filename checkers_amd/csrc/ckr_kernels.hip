@@ -3746,7 +3746,12 @@ __global__ void __launch_bounds__(256) dec_setup_multi_kernel(DecSetupJobs J, Ch
 // and writes the sidecar.  A zero-plane lane codes K zeros from state L: its
 // stream depends on K alone, which takes two values in a unit (the lanes
 // inside the partial top row and the others), so two chains serve them all.
-static constexpr uint32_t LU_SEG = 1024;  // rows per segment (a multiple of 32)
+// Rows per segment (a multiple of 32) and rows loaded ahead in pass 2.  Pass 2
+// waits for memory, so it needs many segments and loads in flight: a 33.5 MB
+// bf16 tensor in 1024-row segments (128 blocks), one row at a time, took 505
+// us, in 256-row segments with 16 rows ahead 87 us (records: 1.6% of the input).
+static constexpr uint32_t LU_SEG = 256;
+static constexpr int LU_ROWS = 16;
 static constexpr uint32_t LU_CH = 130;    // chains per unit: 64 columns x 2 live lanes, 2 zero-plane counts
 
 // The chain of one lane (byte SH / 8 of its column) over the 32 ng rows at
@@ -3959,19 +3964,48 @@ __global__ void __launch_bounds__(256) lu_code_kernel(const uint8_t* __restrict_
     };
     uint32_t x = st.x;
     const uint32_t sh = 8 * b;
-    for (int32_t k = (int32_t)kl - 1; k >= (int32_t)k0; k--) {
-        uint32_t sym = 0;
-        if (live) sym = (uint32_t)k < kf ? (*reinterpret_cast<const uint32_t*>(us + 256ull * k + 4 * j) >> sh) & 255u
-                                         : us[256ull * k + l];
-        const uint4 t = tab[sym];
+    auto step = [&](uint32_t sym, uint4 t) __attribute__((always_inline)) {
         if (ESC && t.w == ENC_ESC) {  // raw-byte escape (ANSCompressor.cpp:185-192)
             put(sym);
-            continue;
+            return;
         }
         const uint32_t n = enc_bytes(x, t.w);
         if (n >= 1) put(x & 255u);
         if (n == 2) put((x >> 8) & 255u);
         x = enc_next(x >> (8 * n), t);
+    };
+    int32_t k = (int32_t)kl - 1;
+    if (k >= (int32_t)kf) {  // the partial row
+        const uint32_t sym = live ? us[256ull * k + l] : 0u;
+        step(sym, tab[sym]);
+        k--;
+    }
+    // groups of LU_ROWS rows from the top down, the next group's loads in flight
+    // while one is coded (rows below the segment are clamped to its first)
+    uint32_t ra[LU_ROWS], rb[LU_ROWS];
+    auto load = [&](uint32_t (&r)[LU_ROWS], int32_t kt) __attribute__((always_inline)) {
+        if (!live) return;
+#pragma unroll
+        for (int i = 0; i < LU_ROWS; i++)
+            r[i] = *reinterpret_cast<const uint32_t*>(us + 256ull * (uint32_t)max(kt - i, (int32_t)k0) + 4 * j);
+    };
+    auto code = [&](const uint32_t (&r)[LU_ROWS], int32_t kt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < LU_ROWS; i++) {
+            if (kt - i < (int32_t)k0) break;
+            const uint32_t sym = live ? (r[i] >> sh) & 255u : 0u;
+            step(sym, tab[sym]);
+        }
+    };
+    if (k >= (int32_t)k0) load(ra, k);
+    while (k >= (int32_t)k0) {
+        if (k - LU_ROWS >= (int32_t)k0) load(rb, k - LU_ROWS);
+        code(ra, k);
+        k -= LU_ROWS;
+        if (k < (int32_t)k0) break;
+        if (k - LU_ROWS >= (int32_t)k0) load(ra, k - LU_ROWS);
+        code(rb, k);
+        k -= LU_ROWS;
     }
     if (hi - pos != (uintptr_t)(e1 - st.y) || x != xend) atomicOr(err, 1u);
 }
@@ -4145,6 +4179,35 @@ __device__ __forceinline__ uint32_t lu_decode_lane(const uint8_t* data, uint64_t
     return nbad;
 }
 
+// A unit stored raw: masked bytes | sidecar, its rows shared by the 4 *
+// LU_RAW_BLOCKS waves of its raw blocks.
+template <int SPE>
+__device__ __forceinline__ void lu_copy_raw(const uint8_t* ud, uint32_t len, uint64_t ubase, const uint8_t* sidecar,
+                                            uint8_t* dst, uint32_t wave, uint32_t j) {
+    for (uint32_t k = wave; 256ull * k < len; k += 4 * LU_RAW_BLOCKS) {
+        const uint32_t p = 256 * k + 4 * j;
+        if (p >= len) continue;
+        const uint32_t nvalid = min(len - p, 4u);
+        uint32_t v = 0;
+        for (uint32_t q = 0; q < nvalid; q++) v |= (uint32_t)ud[p + q] << (8 * q);
+        v = merge_sidecar_row<SPE>(sidecar, ubase + p, v, nvalid);
+        uint8_t* dd = dst + ubase + p;
+        if (nvalid == 4) *reinterpret_cast<uint32_t*>(dd) = v;
+        else for (uint32_t q = 0; q < nvalid; q++) dd[q] = (uint8_t)(v >> (8 * q));
+    }
+}
+template <int SPE>
+__global__ void __launch_bounds__(256) decode_long_raw_kernel(const uint8_t* __restrict__ data,
+                                                              const ckr_stream_header* __restrict__ hdrs,
+                                                              const uint64_t* __restrict__ unit_off, EncodeGeom g,
+                                                              const uint8_t* __restrict__ sidecar,
+                                                              uint8_t* __restrict__ dst) {
+    const uint64_t u = blockIdx.x, ubase = u * g.unit, uoff = unit_off[u];
+    const uint32_t len = unit_len(g, ubase);
+    if (unit_off[u + 1] - uoff == len && hdrs[u * 256].byte_count == len)
+        lu_copy_raw<SPE>(data + uoff, len, ubase, sidecar, dst, blockIdx.y * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+}
+
 template <int SPE>
 __global__ void __launch_bounds__(256) decode_long_kernel(const uint8_t* __restrict__ data,
                                                           const ckr_stream_header* __restrict__ hdrs,
@@ -4162,20 +4225,8 @@ __global__ void __launch_bounds__(256) decode_long_kernel(const uint8_t* __restr
     const uint64_t usize = unit_off[u + 1] - uoff;
     const ckr_stream_header* uh = hdrs + u * 256;
     const bool raw = usize == len && uh[0].byte_count == len;
-    if (blockIdx.y) {  // a raw unit: masked bytes | sidecar, rows shared by the blocks' waves
-        if (!raw) return;
-        const uint32_t W = 4 * LU_RAW_BLOCKS;
-        for (uint32_t k = (blockIdx.y - 1) * 4 + wv; 256ull * k < len; k += W) {
-            const uint32_t p = 256 * k + 4 * j;
-            if (p >= len) continue;
-            const uint32_t nvalid = min(len - p, 4u);
-            uint32_t v = 0;
-            for (uint32_t q = 0; q < nvalid; q++) v |= (uint32_t)ud[p + q] << (8 * q);
-            v = merge_sidecar_row<SPE>(sidecar, ubase + p, v, nvalid);
-            uint8_t* dd = dst + ubase + p;
-            if (nvalid == 4) *reinterpret_cast<uint32_t*>(dd) = v;
-            else for (uint32_t q = 0; q < nvalid; q++) dd[q] = (uint8_t)(v >> (8 * q));
-        }
+    if (blockIdx.y) {
+        if (raw) lu_copy_raw<SPE>(ud, len, ubase, sidecar, dst, (blockIdx.y - 1) * 4 + wv, j);
         return;
     }
     if (raw) return;
@@ -4197,11 +4248,281 @@ __global__ void __launch_bounds__(256) decode_long_kernel(const uint8_t* __restr
     if (nbad) atomicAdd(bad, (unsigned long long)nbad);
 }
 
+// The same decode when there are no more units than CUs, so that each block has
+// a CU to itself and only the length of a lane's chain counts (the one-stream
+// layout: one unit per tensor).  A symbol is then the latency of one table read
+// and the instructions between its arrival and the next symbol's address:
+// - the table has 8-byte entries {f | sym << 24, slot - cum}, ready for one
+//   multiply-add, and is laid out twice (64 KiB), so that an entry's address, the
+//   low 16 bits of 8x, is one SDWA shift with no mask;
+// - the stream window is off the chain: while a pair of symbols is decoded from
+//   the window at its position, the 8 bytes from there are read again, and one
+//   64-bit shift by the bits the pair took makes the next pair's window;
+// - a lane's ring is 256 consecutive LDS bytes (four 64-byte chunks, 16-byte
+//   writes) and a copy of its first 48, so that those 8 bytes lie together
+//   wherever they begin; the position wraps between groups of 16 rows.
+// On entering chunk ch the lane fetches chunk ch + 2, written to the ring
+// DL_PUT_AFTER group ends later (a fetch takes about 1 us behind the stores).
+// 33.5 MB bf16 (131072 rows): 8.6 ms against 10.1 for decode_long_kernel, which
+// stays the better one for many units (three of its blocks share a CU).
+static constexpr uint32_t DL_TAB_BYTES = 65536;
+static constexpr uint32_t DL_LANE = 256 + 48;             // a lane's ring and the copy of its start
+static constexpr uint32_t DL_RING_BYTES = 64 * DL_LANE;   // a wave's
+static constexpr uint32_t DL_LDS = DL_TAB_BYTES + 4 * DL_RING_BYTES + 64;
+static constexpr uint32_t DL_ROWS = 16;  // rows per group
+static constexpr uint32_t DL_AHEAD = 2;  // groups of sidecar bytes loaded ahead (zero-plane lanes)
+static constexpr uint32_t DL_PUT_AFTER = 2;
+// A group takes at most 2 DL_ROWS bytes of a lane, and its last pair's (4 at most)
+// are counted in the next: chunk ch is entered at 64 ch + 2 DL_ROWS + 3 at most, ch + 1
+// two groups later at the earliest, when the registers of the chunk fetched on
+// entering ch are free again; that chunk, ch + 2, is in the ring before a window
+// (12 bytes with its dwords) reaches it.
+static_assert(2 * DL_ROWS * DL_PUT_AFTER <= 64, "one chunk in flight per lane");
+static_assert(2 * DL_ROWS * (DL_PUT_AFTER + 1) + 4 + 12 <= 128, "a chunk must be in the ring before it is read");
+static_assert(2 * DL_ROWS + 4 + 12 <= DL_LANE - 256, "windows of a group end within the copy of the ring's start");
+
+struct DlLane {
+    uint32_t x, w;      // state; window (next 4 stream bytes, the first on top)
+    uint32_t ra, off;   // LDS address of the next stream byte; position = ra + off
+    uint32_t end;       // LDS address of the ring's end
+    uint32_t ch, last;  // as DfLane
+    uint32_t age;       // chunk ch + 2 in flight in c[]: 0 none, else group ends since its fetch
+    uint4 c[4];
+};
+
+__device__ __forceinline__ void lds_put16(uint32_t a, uint4 v) {
+    *(lds_u32x4*)(uintptr_t)a = u32x4{v.x, v.y, v.z, v.w};
+}
+// Chunk k of the lane whose ring begins at tb.
+__device__ __forceinline__ void dl_put(uint32_t tb, uint32_t k, const uint4 (&c)[4]) {
+    const uint32_t a = tb + ((k & 3u) << 6);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) lds_put16(a + 16 * i, c[i]);
+    if ((k & 3u) == 0) {
+#pragma unroll
+        for (uint32_t i = 0; i < 3; i++) lds_put16(tb + 256 + 16 * i, c[i]);
+    }
+}
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+// The three dwords around the 8 stream bytes at LDS address a, and those bytes
+// with the first on top (unaligned 8-byte reads, one instruction in place of
+// the seven here, take LDS so long that the chain was 1.5x as slow).
+struct DlWindow {
+    uint32_t d0, d1, d2;
+};
+__device__ __forceinline__ DlWindow dl_window_read(uint32_t a) {
+    const uint32_t w = a & ~3u;
+    return {*(lds_u32*)(uintptr_t)w, *(lds_u32*)(uintptr_t)(w + 4), *(lds_u32*)(uintptr_t)(w + 8)};
+}
+__device__ __forceinline__ uint64_t dl_window_form(const DlWindow& r, uint32_t a) {
+    const uint32_t hi = __builtin_bswap32(__builtin_amdgcn_alignbyte(r.d1, r.d0, a));
+    const uint32_t lo = __builtin_bswap32(__builtin_amdgcn_alignbyte(r.d2, r.d1, a));
+    return (uint64_t)hi << 32 | lo;
+}
+// The table entry of state x's slot (table at LDS address 0).
+__device__ __forceinline__ u32x2 dl_entry(uint32_t x) {
+    uint32_t a;
+    asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:DWORD" : "=v"(a) : "v"(3u), "v"(x));
+    return *(lds_u32x2*)(uintptr_t)a;
+}
+// The state update and renormalisation of df_sym; returns the bits taken.
+__device__ __forceinline__ uint32_t dl_next(uint32_t& x, uint32_t& w, u32x2 e) {
+    const uint32_t y = __umul24(e.x, x >> 12) + e.y;
+    const uint32_t sh = ((uint32_t)__builtin_clz(y) - 1u) & 24u;
+    const uint64_t v = (((uint64_t)y << 32) | w) << sh;
+    x = (uint32_t)(v >> 32);
+    w = (uint32_t)v;
+    return sh;
+}
+// End of a group.
+__device__ __forceinline__ void dl_step(DlLane& d, const DfSrc& sr) {
+    if (d.age == DL_PUT_AFTER) { dl_put(d.end - 256, d.ch + 2u, d.c); d.age = 0; }
+    else if (d.age) d.age++;
+    const bool adv = ((d.ra + d.off) >> 6) > d.ch;
+    d.ch += adv ? 1u : 0u;
+    if (adv && d.ch + 2u <= d.last) { df_fetch(sr, d.ch + 2u, d.c); d.age = 1; }
+    const uint32_t wrap = d.ra >= d.end ? 256u : 0u;
+    d.ra -= wrap;
+    d.off += wrap;
+}
+
+template <int SPE, int B>
+__device__ __forceinline__ uint32_t dl_decode_lane(const uint8_t* data, uint64_t data_len,
+                                                   const ckr_stream_header* uh, const uint8_t* ud, uint64_t usize,
+                                                   uint32_t len, uint64_t ubase, uint32_t tb, const uint8_t* sidecar,
+                                                   uint8_t* dst, uint32_t j) {
+    constexpr bool LIVE = lane_is_live<SPE>(B);
+    uint32_t nbad = 0, z = 0, ge8;
+    DlLane d;
+    DfSrc sr;
+    {
+        DfLane f;
+        lu_lane_init(f, sr, ge8, uh[4 * j + B], data, data_len, ud, usize, nbad);
+        d.x = f.x;
+        d.ch = 0;
+        d.last = f.last;
+        d.age = 0;
+        d.ra = tb + (f.p8 >> 3);
+        d.off = 0u - tb;
+        d.end = tb + 256;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 3; k++)
+        if (k <= d.last) {
+            df_fetch(sr, k, d.c);
+            dl_put(tb, k, d.c);
+        }
+    const uint32_t K = len >> 8;  // full rows; a partial row K follows when len % 256 != 0
+    uint8_t* o8 = dst + ubase + 4 * j + B;  // row k at o8[256 k]
+    // the zero planes' output bytes are the sidecar's: fp32 bytes 0, 1 of the
+    // element; bf16 byte 0 of each of the column's two elements
+    const uint8_t* s8 = sidecar + ((ubase + 4 * j) >> 1) + (SPE == 2 ? B : B / 2);  // row k at s8[128 k]
+    // What a pair hands on: the read of the next symbol's entry, in flight; the
+    // 8 bytes its window began with and the bits it took (the next window and
+    // position are formed while that read is under way).  The scheduling
+    // barriers keep everything else behind the reads' issue.
+    u32x2 en = dl_entry(d.x);
+    DlWindow v = dl_window_read(d.ra);
+    uint64_t vf = dl_window_form(v, d.ra);
+    uint32_t h = 0;
+    auto settle = [&]() __attribute__((always_inline)) {
+        d.w = (uint32_t)((vf << h) >> 32);
+        d.ra += h >> 3;
+    };
+    auto pair = [&](uint8_t* o, uint32_t sv0, uint32_t sv1) __attribute__((always_inline)) {
+        const u32x2 e0 = en;
+        settle();
+        v = dl_window_read(d.ra);
+        __builtin_amdgcn_sched_barrier(0);
+        h = dl_next(d.x, d.w, e0);
+        const u32x2 e1 = dl_entry(d.x);
+        __builtin_amdgcn_sched_barrier(0);
+        if (LIVE) o[0] = (uint8_t)(e0.x >> 24);
+        else { z |= e0.x; o[0] = (uint8_t)sv0; }
+        vf = dl_window_form(v, d.ra);
+        __builtin_amdgcn_sched_barrier(0);
+        h += dl_next(d.x, d.w, e1);
+        en = dl_entry(d.x);
+        __builtin_amdgcn_sched_barrier(0);
+        if (LIVE) o[256] = (uint8_t)(e1.x >> 24);
+        else { z |= e1.x; o[256] = (uint8_t)sv1; }
+    };
+    const uint32_t ng = K / DL_ROWS;
+    if (ng) {
+        const uint32_t gl = ng - 1;
+        uint32_t sb[DL_AHEAD + 1][DL_ROWS];
+        auto load = [&](uint32_t (&b)[DL_ROWS], uint32_t g) __attribute__((always_inline)) {
+            if (!LIVE) {
+#pragma unroll
+                for (uint32_t r = 0; r < DL_ROWS; r++) b[r] = s8[128ull * (DL_ROWS * g + r)];
+            }
+        };
+#pragma unroll
+        for (uint32_t q = 0; q < DL_AHEAD; q++) load(sb[q], min(q, gl));
+        uint32_t gi = 0;
+        uint8_t* o = o8;
+        auto group = [&](const uint32_t (&b)[DL_ROWS]) __attribute__((always_inline)) {
+#pragma unroll
+            for (uint32_t r = 0; r < DL_ROWS; r += 2) pair(o + 256 * r, b[r], b[r + 1]);
+            o += 256 * DL_ROWS;
+            dl_step(d, sr);
+        };
+        for (; gi + DL_AHEAD + 1 <= ng; gi += DL_AHEAD + 1) {
+#pragma unroll
+            for (uint32_t q = 0; q <= DL_AHEAD; q++) {
+                load(sb[(q + DL_AHEAD) % (DL_AHEAD + 1)], min(gi + q + DL_AHEAD, gl));
+                group(sb[q]);
+            }
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < DL_AHEAD; q++)
+            if (gi + q < ng) group(sb[q]);
+    }
+    // at most 15 rows and the partial one: 32 bytes at most
+    uint32_t k = DL_ROWS * ng;
+    for (; k + 2 <= K; k += 2) pair(o8 + 256ull * k, LIVE ? 0u : s8[128ull * k], LIVE ? 0u : s8[128ull * (k + 1)]);
+    settle();
+    uint32_t p8 = (d.ra + d.off) << 3;
+    const bool top = 4 * j + B < (len & 255u);  // this lane holds a byte of the partial row K
+    auto one = [&](uint32_t kr) __attribute__((always_inline)) {
+        const u32x2 e = dl_entry(d.x);
+        p8 += dl_next(d.x, d.w, e);
+        if (LIVE) o8[256ull * kr] = (uint8_t)(e.x >> 24);
+        else { z |= e.x; o8[256ull * kr] = s8[128ull * kr]; }
+    };
+    if (k < K) one(k);  // the window's 4 bytes serve this row and the partial one
+    if (top) one(K);
+    // bad: not ending at state L with every byte consumed, or, in a zero
+    // plane, a nonzero symbol
+    nbad += (d.x != L || p8 != ge8 || (!LIVE && (z >> 24))) ? 1u : 0u;
+    return nbad;
+}
+
+template <int SPE>
+__global__ void __launch_bounds__(256) decode_chain_kernel(const uint8_t* __restrict__ data,
+                                                           const ckr_stream_header* __restrict__ hdrs,
+                                                           const uint64_t* __restrict__ unit_off,
+                                                           const uint32_t* __restrict__ d_dec, EncodeGeom g,
+                                                           const uint8_t* __restrict__ sidecar,
+                                                           uint8_t* __restrict__ dst, unsigned long long* bad) {
+    extern __shared__ uint32_t lds[];  // at LDS address 0 (dl_entry)
+    const uint64_t u = blockIdx.x;
+    const uint32_t j = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t ubase = u * g.unit;
+    const uint32_t len = unit_len(g, ubase);
+    const uint64_t uoff = unit_off[u];
+    const uint8_t* ud = data + uoff;
+    const uint64_t usize = unit_off[u + 1] - uoff;
+    const ckr_stream_header* uh = hdrs + u * 256;
+    if (usize == len && uh[0].byte_count == len) return;  // stored raw: decode_long_raw_kernel's
+    for (uint32_t i = threadIdx.x; i < 8192; i += 256) {
+        const uint32_t slot = i & 4095u, e = d_dec[slot];  // sym | (f - 1) << 8 | cum << 20
+        lds[2 * i] = (((e >> 8) & 4095u) + 1u) | (e & 255u) << 24;
+        lds[2 * i + 1] = slot - (e >> 20);
+    }
+    __syncthreads();
+    const uint64_t data_len = unit_off[g.n_units];
+    const uint32_t tb = DL_TAB_BYTES + wv * DL_RING_BYTES + j * DL_LANE;
+    uint32_t nbad;
+    switch (wv) {
+        case 0: nbad = dl_decode_lane<SPE, 0>(data, data_len, uh, ud, usize, len, ubase, tb, sidecar, dst, j); break;
+        case 1: nbad = dl_decode_lane<SPE, 1>(data, data_len, uh, ud, usize, len, ubase, tb, sidecar, dst, j); break;
+        case 2: nbad = dl_decode_lane<SPE, 2>(data, data_len, uh, ud, usize, len, ubase, tb, sidecar, dst, j); break;
+        default: nbad = dl_decode_lane<SPE, 3>(data, data_len, uh, ud, usize, len, ubase, tb, sidecar, dst, j); break;
+    }
+    if (nbad) atomicAdd(bad, (unsigned long long)nbad);
+}
+
 hipError_t launch_decode_long(const uint8_t* data, const ckr_stream_header* hdrs, const uint64_t* unit_off,
                               const uint32_t* d_dec, const EncodeGeom& g, const uint8_t* sidecar, uint8_t* dst,
                               unsigned long long* bad, hipStream_t s) {
     if (g.n_units == 0) return hipSuccess;
     if (g.spe != 1 && g.spe != 2) return hipErrorInvalidValue;
+    // a block per CU at most: the kernel with the shorter chain (its LDS takes the CU)
+    int dev = 0, ncu = 0;
+    hipError_t e;
+    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+    if ((e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+    if (g.n_units <= (uint64_t)ncu) {
+        const void* kf = g.spe == 2 ? reinterpret_cast<const void*>(decode_chain_kernel<2>)
+                                    : reinterpret_cast<const void*>(decode_chain_kernel<1>);
+        if (hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)DL_LDS) == hipSuccess) {
+            const uint32_t n = (uint32_t)g.n_units;
+            const dim3 rg(n, LU_RAW_BLOCKS);
+            if (g.spe == 2) {
+                CKR_LAUNCH("decode_chain_kernel", s, decode_chain_kernel<2><<<n, 256, DL_LDS, s>>>(data, hdrs, unit_off, d_dec, g, sidecar, dst, bad));
+                if ((e = hipGetLastError()) != hipSuccess) return e;
+                CKR_LAUNCH("decode_long_raw_kernel", s, decode_long_raw_kernel<2><<<rg, 256, 0, s>>>(data, hdrs, unit_off, g, sidecar, dst));
+            } else {
+                CKR_LAUNCH("decode_chain_kernel", s, decode_chain_kernel<1><<<n, 256, DL_LDS, s>>>(data, hdrs, unit_off, d_dec, g, sidecar, dst, bad));
+                if ((e = hipGetLastError()) != hipSuccess) return e;
+                CKR_LAUNCH("decode_long_raw_kernel", s, decode_long_raw_kernel<1><<<rg, 256, 0, s>>>(data, hdrs, unit_off, g, sidecar, dst));
+            }
+            return hipGetLastError();
+        }
+        (void)hipGetLastError();  // LDS too small on this device
+    }
     const uint32_t lb = DF_TAB_BYTES + 4 * DF_RING_BYTES;
     const dim3 grid((uint32_t)g.n_units, 1 + LU_RAW_BLOCKS);
     if (g.spe == 2) CKR_LAUNCH("decode_long_kernel", s, decode_long_kernel<2><<<grid, 256, lb, s>>>(data, hdrs, unit_off, d_dec, g, sidecar, dst, bad));
