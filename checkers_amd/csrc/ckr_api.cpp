@@ -249,7 +249,9 @@ hipError_t canon_launch(const ckr_freq_table* t, const CanonKs& ck, uint32_t* ca
     return hipSuccess;
 }
 
-bool use_fast_encode(const ckr::EncodeGeom& g) { return use_dedup(g) && (g.unit + 255) / 256 <= kFastMaxK; }
+bool use_fast_encode(const ckr::EncodeGeom& g) {
+    return g_fast_paths && g.n_units > 0 && (g.unit + 255) / 256 <= kFastMaxK;
+}
 // Units above 64 KiB (up to the dedup limit): the two-pass kernels.
 bool use_seg_encode(const ckr::EncodeGeom& g) { return use_dedup(g) && (g.unit + 255) / 256 > kFastMaxK; }
 // Units above the dedup limit (the one-stream layout of a tensor above 1 MiB):
@@ -361,12 +363,14 @@ EncodeLayout encode_layout(const ckr::EncodeGeom& g) {
 // Decode workspace: enc table, canonical streams, decode table, bad-lane counter.
 struct DecodeLayout {
     uint64_t off_canon, off_dec, off_bad, total;
-    bool fast;
+    bool fast;      // the fast decoder with canonical streams (masked dtypes)
+    bool fast_any;  // the fast decoder (int8 and int32 included)
 };
 DecodeLayout decode_layout(const ckr::EncodeGeom& g) {
     DecodeLayout L{};
     const CanonKs ck = canon_ks(g);
     L.fast = g_fast_paths != 0 && g.spe > 0 && g.n_units > 0 && use_dedup(g);
+    L.fast_any = L.fast || (g_fast_paths != 0 && g.spe == 0 && g.n_units > 0 && (g.unit + 255) / 256 <= kDedupMaxK);
     uint64_t o = 0;
     L.off_canon = o; o = align_up(o + (L.fast ? 3ull * (4 + 2 * ck.cw) * 4 : 0), kAlign);
     L.off_dec = o;   o = align_up(o + 4096 * 4, kAlign);
@@ -825,12 +829,17 @@ int encode_impl(const void* d_src, uint64_t n_elems, int dtype, const ckr_freq_t
     if (fast) {
         fp.escapes = escapes;
         const uint32_t K = (uint32_t)((g.unit + 255) / 256);
-        fp.cw = ck.cw;
-        const uint32_t cbmax = std::max(canon_stream_bytes(h_table, ck.k0),
-                                        std::max(canon_stream_bytes(h_table, ck.k1), canon_stream_bytes(h_table, ck.k2)));
-        fp.canon_bytes = std::min<uint32_t>((cbmax + 3) & ~3u, 4 * ck.cw);
+        fp.unmasked = g.spe == 0;
+        fp.cw = dedup ? ck.cw : 0;
+        const uint32_t cbmax = !dedup ? 0u
+                                      : std::max(canon_stream_bytes(h_table, ck.k0),
+                                                 std::max(canon_stream_bytes(h_table, ck.k1),
+                                                          canon_stream_bytes(h_table, ck.k2)));
+        fp.canon_bytes = std::min<uint32_t>((cbmax + 3) & ~3u, 4 * fp.cw);
         if (g_fast_paths >= 2) {
             fp.sl0 = fp.sl1 = 8;
+        } else if (fp.unmasked) {  // (all four planes alike; 0: no slot fits)
+            fp.sl0 = fp.sl1 = std::max(8u, ckr::encode_fast_max_slot(0, K, (uint32_t)max_lds_per_block(), true));
         } else {
             fp.sl0 = lane_slot_bytes(h_planes, h_table, K);
             fp.sl1 = lane_slot_bytes(h_planes ? h_planes + 256 : nullptr, h_table, K);
@@ -1227,9 +1236,10 @@ bool dev_enc_setup(DevEnc& d, const void* src, const ckr::EncodeGeom& g, uint8_t
     d.pin = pin;
     const uint32_t K = (uint32_t)((g.unit + 255) / 256);
     d.fp.escapes = false;  // the table is the data's own: every symbol present has a slot
-    d.fp.cw = d.ck.cw;
-    d.fp.canon_bytes = 4 * d.ck.cw;
-    const uint32_t smax = ckr::encode_fast_max_slot(d.fp.canon_bytes, K, (uint32_t)max_lds_per_block());
+    d.fp.unmasked = g.spe == 0;
+    d.fp.cw = g.spe ? d.ck.cw : 0;
+    d.fp.canon_bytes = 4 * d.fp.cw;
+    const uint32_t smax = ckr::encode_fast_max_slot(d.fp.canon_bytes, K, (uint32_t)max_lds_per_block(), d.fp.unmasked);
     if (!smax || d.ck.cw > ckr::kCanonMaxCw) return false;
     d.fp.sl0 = d.fp.sl1 = smax;
     return ckr::encode_fast_lds_bytes(d.fp, (uint32_t)max_lds_per_block()) != 0;
@@ -1244,7 +1254,7 @@ ckr::TableEncJob dev_enc_table_job(const DevEnc& d, int ensure_full) {
     t.status = reinterpret_cast<uint64_t*>(d.ws + d.L.off_status);
     t.n_status = ckr::encode_fast_status_words(d.g.n_units);
     t.ctl = d.dctl;
-    t.a = ckr::TableEncArg{(uint32_t)((d.g.unit + 255) / 256), d.ck.k0, d.ck.k1, d.ck.k2, d.ck.cw, d.fp.sl0, ensure_full};
+    t.a = ckr::TableEncArg{(uint32_t)((d.g.unit + 255) / 256), d.ck.k0, d.ck.k1, d.ck.k2, d.fp.cw, d.fp.sl0, ensure_full};
     return t;
 }
 
@@ -1658,7 +1668,7 @@ int ckr_compress_many(ckr_compress_job* jobs, uint64_t n, uint64_t unit_bytes, i
                 if (rc == CKR_OK)
                     rc = encode_impl(staged[i].p, jb.n_elems, jb.dtype, t, unit_bytes, jb.d_out, jb.out_capacity,
                                      jb.d_headers, jb.d_unit_offsets, jb.d_sidecar, jb.d_workspace, jb.workspace_bytes,
-                                     &jb.total, hh + 256, s);
+                                     &jb.total, geo[i].spe ? hh + 256 : nullptr, s);
             }
             if (rc) return rc;
         }
@@ -1718,11 +1728,11 @@ int ckr_compress_many(ckr_compress_job* jobs, uint64_t n, uint64_t unit_bytes, i
             // the encodes of all jobs of one kind (spe, sidecar) in one launch
             // behind the tables, at most kMaxFastJobs a launch
             {
-                std::vector<ckr::FastJob> fj[4];
+                std::vector<ckr::FastJob> fj[6];
                 for (uint64_t i = 0; i < n; i++) {
                     if (!geo[i].n_units) continue;
                     const ckr::FastJob f = dev_fast_job(dv[i]);
-                    fj[(f.g.spe == 2 ? 2 : 0) + (f.sidecar ? 1 : 0)].push_back(f);
+                    fj[2 * f.g.spe + (f.sidecar ? 1 : 0)].push_back(f);
                 }
                 for (auto& v : fj)
                     for (size_t o = 0; o < v.size(); o += ckr::kMaxFastJobs)
@@ -1926,7 +1936,7 @@ int decode_impl(const uint8_t* d_data, const ckr_stream_header* d_headers, const
     hipError_t de = use_long_units(g)
                         ? ckr::launch_decode_long(d_data, d_headers, d_unit_offsets, dec, g, d_sidecar, out, bad, s)
                         : ckr::launch_decode(d_data, d_headers, d_unit_offsets, dec, g, d_sidecar, out, bad,
-                                             L.fast ? canon : nullptr, ck.cw, s, counted);
+                                             L.fast ? canon : nullptr, ck.cw, L.fast_any, s, counted);
     if (tmp) {
         if (de == hipSuccess) de = hipMemcpyAsync(d_dst, tmp, g.n_bytes, hipMemcpyDeviceToDevice, s);
         (void)hipFreeAsync(tmp, s);

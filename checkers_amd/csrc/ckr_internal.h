@@ -128,13 +128,14 @@ hipError_t launch_encode_batch(const uint8_t* src, const EncodeGeom& g, uint64_t
                                uint32_t* unit_size, uint64_t* unit_off, uint8_t* out, const uint32_t* ulist,
                                hipStream_t s);
 
-// LDS-staged encode of all units (masked dtypes, units <= 64 KiB).  status:
+// LDS-staged encode of all units (units <= 64 KiB).  status:
 // encode_fast_status_words(n_units) u64, ctl: 6 u32 ({ticket, redo count, error, 0, total lo, total hi}),
 // both cleared beforehand by launch_build_enc_table_reset; redo_list: n_units u32 — units whose bytes
 // must then be produced by launch_encode_batch.
 struct FastEncParamsHost {
     uint32_t sl0, sl1, cw, canon_bytes;
     bool escapes;  // the data may hold symbols with f == 0 (table not built from it)
+    bool unmasked = false;  // int8, int32: four live lanes per column (sl0 == sl1, no canonical streams)
 };
 // LDS bytes of the fast encoder's workgroup within lds_limit (0: it does not fit).
 uint32_t encode_fast_lds_bytes(const FastEncParamsHost& p, uint32_t lds_limit);
@@ -187,7 +188,8 @@ hipError_t launch_tables(const uint32_t* hists, uint64_t n, int ensure_full, uin
 // by ranks, encode entries, canonical zero-plane streams for lane counts k0,
 // k1, k2 (cw dwords), the fast encoder's slot sizes (each at most smax, their
 // sum at most 2 smax), and its status and control words cleared.  tinfo:
-// norm[256], sum, ambiguity, sl0, sl1.
+// norm[256], sum, ambiguity, sl0, sl1.  cw 0: an unmasked dtype (no canonical
+// streams, both slots smax).
 struct TableEncArg {
     uint32_t K, k0, k1, k2, cw, smax;
     int ensure_full;
@@ -222,9 +224,9 @@ constexpr uint64_t kChainBytes = (4ull + 2ull) * (kChainSteps + 1) * kChainRows 
 hipError_t launch_canon_chains(void* chains, hipStream_t s);
 constexpr uint32_t kTinfoWords = 260;
 constexpr uint32_t kCanonMaxCw = 136;  // canonical stream dwords table_enc handles (K <= 256)
-// The largest slot (multiple of 4, at most 2K + 8) whose two-pair layout of the
-// fast encoder fits lds_cap (0: none).
-uint32_t encode_fast_max_slot(uint32_t canon_bytes, uint32_t K, uint32_t lds_cap);
+// The largest slot (multiple of 4, at most 2K + 8) whose two-pair layout (unmasked:
+// the one unit of four coder waves) of the fast encoder fits lds_cap (0: none).
+uint32_t encode_fast_max_slot(uint32_t canon_bytes, uint32_t K, uint32_t lds_cap, bool unmasked);
 
 // Units above 64 KiB of masked dtypes, in two passes (no lane scratch): rec
 // holds n_units * encode_seg_segments(unit) * 128 checkpoint records, unit_size
@@ -310,8 +312,8 @@ hipError_t launch_dec_setup_multi(const DecSetupJob* jobs, uint32_t n, const voi
 // them one by one).
 hipError_t launch_decode_fast_multi(DecJob* jobs, uint32_t n, hipStream_t s);
 
-// Decode; with canon (masked dtypes) the fast kernel decodes every unit,
-// otherwise the general kernel does.
+// Decode; with fast_ok (and canon, for masked dtypes) the fast kernel decodes
+// every unit, otherwise the general kernel does.
 uint32_t decode_fast_lds_bytes();
 // zero_bytes: the fast decoder also compares the zero-plane lanes' bytes with
 // their canonical streams (their headers are checked either way); those bytes
@@ -319,7 +321,7 @@ uint32_t decode_fast_lds_bytes();
 // needs them read.
 hipError_t launch_decode(const uint8_t* data, const ckr_stream_header* hdrs, const uint64_t* unit_off,
                          const uint32_t* d_dec, const EncodeGeom& g, const uint8_t* sidecar, uint8_t* dst,
-                         unsigned long long* bad, const uint32_t* canon, uint32_t cw, hipStream_t s,
+                         unsigned long long* bad, const uint32_t* canon, uint32_t cw, bool fast_ok, hipStream_t s,
                          bool zero_bytes = true);
 
 // Analyzer (ckr_analyzer.hip): every record in one grid per pass.

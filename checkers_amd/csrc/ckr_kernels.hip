@@ -309,11 +309,23 @@ __device__ void table_enc_body(const uint32_t* __restrict__ hist, const TableEnc
     rank_table(hist, a.ensure_full != 0, T);
     const uint32_t s = threadIdx.x;
     // the chain data of the canonical streams, loaded now and used at the end
-    const CanonLoad cl = canon_load(T.norm[0], a.k0, a.k1, a.k2, ch);
+    const bool masked = a.cw != 0;  // int8, int32: no zero planes, every lane's slot as large as the LDS allows
+    CanonLoad cl{};
+    if (masked) cl = canon_load(T.norm[0], a.k0, a.k1, a.k2, ch);
     const uint32_t nm = T.norm[s];
     enc[s] = enc_entry_fc(nm, T.cum[s]);
     tinfo[s] = nm;
     if (s < 6) ctl[s] = s == 2 ? flags : 0u;
+    if (!masked) {
+        if (s == 0) {
+            tinfo[256] = T.cum[256];
+            tinfo[257] = T.amb;
+            tinfo[258] = tinfo[259] = a.smax;
+            ctl[6] = (uint32_t)epoch;
+            ctl[7] = (uint32_t)(epoch >> 32);
+        }
+        return;
+    }
     // slot sizes: per plane p, n = sum h_p, m = sum h_p cost / n, v = sum h_p cost^2 / n - m^2
     const float cost = nm ? 12.0f - log2f((float)nm) : 8.0f;  // log2(M / norm)
     float v[6];
@@ -726,6 +738,7 @@ struct HistTableJobs {
 };
 __global__ void __launch_bounds__(256) hist_table_kernel(HistTableJobs J, Chains ch) {
     __shared__ __align__(16) uint32_t sh[512 * 16];
+    static_assert(256 * HIST_COPIES <= 512 * 16, "unmasked dtypes' copies");
     static_assert(sizeof(TableLds) <= sizeof(sh), "the table set-up reuses the histogram's LDS");
     __shared__ uint32_t last;
     uint32_t k = 0;
@@ -747,6 +760,8 @@ __global__ void __launch_bounds__(256) hist_table_kernel(HistTableJobs J, Chains
     }
     if (j.spe == 2)
         masked_hist_share<2, 16>(sh, j.src, j.n_bytes, j.es, j.hist, j.hist + 256, j.head_n, b, j.nblk, gate, J.epoch, gate_err);
+    else if (j.spe == 0)
+        masked_hist_share<0, 16>(sh, j.src, j.n_bytes, j.es, j.hist, nullptr, j.head_n, b, j.nblk, gate, J.epoch, gate_err);
     else
         masked_hist_share<1, 16>(sh, j.src, j.n_bytes, j.es, j.hist, j.hist + 256, j.head_n, b, j.nblk, gate, J.epoch, gate_err);
     // this workgroup's adds complete (every wave waits for its own) before its
@@ -1314,7 +1329,8 @@ __device__ __forceinline__ void lds_put(uint32_t a, uint32_t v) { *(lds_u32*)(ui
 template <uint32_t SH>
 __device__ __forceinline__ uint4 enc_entry_of(uint32_t w) {
     uint32_t a;
-    if constexpr (SH == 8) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(a) : "v"(4u), "v"(w));
+    if constexpr (SH == 0) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0" : "=v"(a) : "v"(4u), "v"(w));
+    else if constexpr (SH == 8) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(a) : "v"(4u), "v"(w));
     else if constexpr (SH == 16) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(a) : "v"(4u), "v"(w));
     else asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3" : "=v"(a) : "v"(4u), "v"(w));
     const u32x4 t = *(lds_u32x4*)(uintptr_t)a;
@@ -1499,9 +1515,9 @@ __device__ __forceinline__ uint4 merge16_from(uint4 v, uint4 r, uint32_t s) {
 }
 
 
-// Coding of one live lane of every column of a unit whose rows are all full
-// (length a multiple of 256, so every column has the same nrows rows).  P = 0:
-// byte FL of each column; P = 1: byte 3.  Rows are taken from the top down.
+// Coding of one live lane of every column, byte SH / 8 of it, of a unit whose
+// rows are all full (length a multiple of 256, so every column has the same
+// nrows rows).  Rows are taken from the top down.
 // The rows above the highest multiple of GR go one at a time; then groups of
 // GR rows, the next group's loads in flight while the current one is coded
 // (loads and table reads are unconditional, so the waits stay exact), and a
@@ -1509,12 +1525,10 @@ __device__ __forceinline__ uint4 merge16_from(uint4 v, uint4 r, uint32_t s) {
 // entries that carries over from group to group (the LDS serves it in about 50
 // cycles when idle, 100 and more beside the packers' reads; a row takes about
 // 55).  Emitted bytes are stored after every second row.  The sidecar rows are
-// written by the thread coding plane 0 and 1 alternately (row k by P == k & 1).
-template <int SPE, bool ESC, bool SIDE, int P, int GR, int TR>
+// written by the two coder waves alternately (row k by the one with P == k & 1).
+template <int SPE, bool ESC, bool SIDE, uint32_t SH, int P, int GR, int TR>
 __device__ __forceinline__ void enc_full_rows(EncLane& c, const uint8_t* ucol, uint8_t* sidecar, uint64_t ubase,
                                               uint32_t j, uint32_t nrows) {
-    constexpr int FL = SPE == 2 ? 2 : 1;
-    constexpr uint32_t SH = P == 1 ? 24u : 8u * FL;   // this lane's byte of the column
     const uint32_t* in32 = reinterpret_cast<const uint32_t*>(ucol);          // row k at in32[64 k]
     uint16_t* sc16 = SIDE ? reinterpret_cast<uint16_t*>(sidecar + (ubase >> 1) + 2 * j) : nullptr;  // row k at sc16[64 k]
     auto side = [&](uint16_t* p, uint32_t wd) {
@@ -1635,13 +1649,15 @@ __host__ __device__ constexpr uint32_t slot_stride(uint32_t sl) { return sl + 8;
 __host__ __device__ constexpr uint32_t ws_ctl_offset(uint32_t canon_bytes) {
     return (FE_CBYTES + 3 * canon_bytes + 15u) & ~15u;
 }
-__host__ __device__ constexpr uint32_t ws_region_bytes(uint32_t stride0, uint32_t stride1) {
-    return (R_SLOTS + 64 * stride0 + 64 * stride1 + 15u) & ~15u;
+// nc: live lanes of a column, 2 (masked dtypes) or 4 (int8, int32; stride0 ==
+// stride1 then): a coder wave and 64 slots for each.
+__host__ __device__ constexpr uint32_t ws_region_bytes(uint32_t stride0, uint32_t stride1, uint32_t nc = 2) {
+    return (R_SLOTS + 32 * nc * stride0 + 32 * nc * stride1 + 15u) & ~15u;
 }
 __host__ __device__ constexpr uint32_t ws_lds_bytes(uint32_t pairs, uint32_t canon_bytes, uint32_t stride0,
-                                                    uint32_t stride1) {
+                                                    uint32_t stride1, uint32_t nc = 2) {
     return ws_ctl_offset(canon_bytes) + pairs * (uint32_t)sizeof(WsPairCtl) +
-           2 * pairs * ws_region_bytes(stride0, stride1) + 32;
+           2 * pairs * ws_region_bytes(stride0, stride1, nc) + 32;
 }
 
 // LIST: the units a previous launch put on the redo list (ctl[1] of them in
@@ -1666,12 +1682,13 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
     }
     extern __shared__ uint32_t lds[];
     uint8_t* lds8 = reinterpret_cast<uint8_t*>(lds);
-    constexpr uint32_t NT = 64 * (2 + NPK) * PAIRS;
+    constexpr uint32_t NC = SPE == 0 ? 4 : 2;  // coder waves of a pair, one per live byte of a column
+    constexpr uint32_t NT = 64 * (NC + NPK) * PAIRS;
     const uint4* tab = reinterpret_cast<const uint4*>(lds8 + 0);
     uint32_t* chdr = reinterpret_cast<uint32_t*>(lds8 + FE_CHDR);
     const uint32_t cb_off = FE_CBYTES;
     const uint32_t ctl_off = ws_ctl_offset(fp.canon_bytes);
-    const uint32_t rbytes = ws_region_bytes(fp.stride0, fp.stride1);
+    const uint32_t rbytes = ws_region_bytes(fp.stride0, fp.stride1, NC);
     const uint32_t reg0 = ctl_off + PAIRS * (uint32_t)sizeof(WsPairCtl);
     const uint32_t tid = threadIdx.x;
     const uint32_t j = tid & 63;  // column
@@ -1686,13 +1703,15 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
             const EncSym e = {tv.x, tv.y, tv.z, tv.w};
             wt[k] = enc_quad(e);
         }
-        const uint32_t* cs = canon + 3 * (4 + fp.cw);
-        uint32_t* cb32 = reinterpret_cast<uint32_t*>(lds8 + cb_off);
-        const uint32_t ncb = 3 * fp.canon_bytes / 4;
-        const uint32_t cb_per = fp.canon_bytes / 4;
-        // (as in the slots, the bytes of each dword in reverse order)
-        for (uint32_t i = tid; i < ncb; i += NT) cb32[i] = __builtin_bswap32(cs[(i / cb_per) * fp.cw + (i % cb_per)]);
-        if (tid < 12) chdr[tid] = canon[(tid >> 2) * (4 + fp.cw) + (tid & 3)];
+        if constexpr (SPE > 0) {
+            const uint32_t* cs = canon + 3 * (4 + fp.cw);
+            uint32_t* cb32 = reinterpret_cast<uint32_t*>(lds8 + cb_off);
+            const uint32_t ncb = 3 * fp.canon_bytes / 4;
+            const uint32_t cb_per = fp.canon_bytes / 4;
+            // (as in the slots, the bytes of each dword in reverse order)
+            for (uint32_t i = tid; i < ncb; i += NT) cb32[i] = __builtin_bswap32(cs[(i / cb_per) * fp.cw + (i % cb_per)]);
+            if (tid < 12) chdr[tid] = canon[(tid >> 2) * (4 + fp.cw) + (tid & 3)];
+        }
         uint32_t* c32 = reinterpret_cast<uint32_t*>(lds8 + ctl_off);
         for (uint32_t i = tid; i < PAIRS * (uint32_t)sizeof(WsPairCtl) / 4; i += NT) c32[i] = 0;
     }
@@ -1701,15 +1720,20 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     // waves 0 .. 2 PAIRS - 1 code, the others pack, NPK per pair (wave w runs on
     // SIMD w mod 4, so the coders are on four different SIMDs)
-    const bool coder = wv < 2 * PAIRS;
-    const uint32_t pr = coder ? (wv >> 1) : (wv - 2 * PAIRS) / NPK;  // pair
-    const uint32_t rl = wv & 1;  // coder: 0 byte FL, 1 byte 3
-    const uint32_t pw = coder ? 0u : (wv - 2 * PAIRS) % NPK;  // packer: 0 look-back, 1 headers, all pack
+    const bool coder = wv < NC * PAIRS;
+    const uint32_t pr = coder ? wv / NC : (wv - NC * PAIRS) / NPK;  // pair
+    const uint32_t rl = wv % NC;  // coder: 0 byte FL, 1 byte 3 (SPE 0: byte rl)
+    const uint32_t pw = coder ? 0u : (wv - NC * PAIRS) % NPK;  // packer: 0 look-back, 1 headers, all pack
     WsPairCtl& pc = *reinterpret_cast<WsPairCtl*>(lds8 + ctl_off + pr * (uint32_t)sizeof(WsPairCtl));
     const uint32_t col = 4 * j;
+    // LDS address of the end of column j's slot of coder r in the region at rb
+    auto slot_end = [&](uint32_t rb, uint32_t r) {
+        if constexpr (SPE == 0) return rb + R_SLOTS + (64 * r + j) * fp.stride0 + fp.sl0;
+        else return r ? rb + R_SLOTS + 64 * fp.stride0 + j * fp.stride1 + fp.sl1 : rb + R_SLOTS + j * fp.stride0 + fp.sl0;
+    };
 
     if (coder) {
-        const uint32_t sh = rl ? 24u : 8u * FL;  // this wave's byte of the column
+        const uint32_t cb = SPE == 0 ? rl : (rl ? 3u : (uint32_t)FL);  // this wave's byte of the column
         for (uint32_t i = 0;; i++) {
             const uint32_t s = i & 1;
             const uint64_t t_wait = phase ? wall_clock64() : 0;
@@ -1737,16 +1761,29 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
             const uint32_t len = (uint32_t)((g.n_bytes - ubase < g.unit) ? (g.n_bytes - ubase) : g.unit);
             const uint8_t* usrc = src + ubase;
             const uint32_t rb = reg0 + (2 * pr + s) * rbytes;
-            const uint32_t endw = rl ? rb + R_SLOTS + 64 * fp.stride0 + j * fp.stride1 + fp.sl1
-                                     : rb + R_SLOTS + j * fp.stride0 + fp.sl0;
+            const uint32_t endw = slot_end(rb, rl);
             EncLane c{L, 0u, 0u, endw};
             const uint32_t K = len > col ? (len - col + 255) / 256 : 0u;
             if ((len & 255u) == 0) {
-                if (rl == 0) enc_full_rows<SPE, ESC, SIDE, 0, ENC_GR, ENC_TR>(c, usrc + col, sidecar, ubase, j, len >> 8);
-                else enc_full_rows<SPE, ESC, SIDE, 1, ENC_GR, ENC_TR>(c, usrc + col, sidecar, ubase, j, len >> 8);
+                auto rows = [&](auto sh_c, auto p_c) __attribute__((always_inline)) {
+                    enc_full_rows<SPE, ESC, SIDE, decltype(sh_c)::value, decltype(p_c)::value, ENC_GR, ENC_TR>(
+                        c, usrc + col, sidecar, ubase, j, len >> 8);
+                };
+                using p0 = std::integral_constant<int, 0>;
+                using p1 = std::integral_constant<int, 1>;
+                if constexpr (SPE == 0) {
+                    if (rl == 0) rows(std::integral_constant<uint32_t, 0>{}, p0{});
+                    else if (rl == 1) rows(std::integral_constant<uint32_t, 8>{}, p0{});
+                    else if (rl == 2) rows(std::integral_constant<uint32_t, 16>{}, p0{});
+                    else rows(std::integral_constant<uint32_t, 24>{}, p0{});
+                } else {
+                    if (rl == 0) rows(std::integral_constant<uint32_t, 8u * FL>{}, p0{});
+                    else rows(std::integral_constant<uint32_t, 24>{}, p1{});
+                }
             } else {
                 // A tensor's last unit: rows from the top down, one at a time; the top
-                // row may be partial (bf16: lane 4j+3 has one symbol fewer).
+                // row may be partial (16-bit elements: lane 4j+3 may have one symbol
+                // fewer than 4j+1; bytes: any lane of the last column).
                 for (int32_t k = (int32_t)K - 1; k >= 0; k--) {
                     const uint32_t p = 256 * (uint32_t)k + col;
                     const uint32_t nvalid = (len - p) < 4 ? (len - p) : 4;
@@ -1755,13 +1792,13 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
                     else for (uint32_t b = 0; b < nvalid; b++) v |= (uint32_t)usrc[p + b] << (8 * b);
                     if (SIDE && (uint32_t)(k & 1) == rl) write_sidecar_row<SPE>(sidecar, ubase + p, v, nvalid);
                     v &= lm;
-                    const uint32_t sy = (v >> sh) & 255u;
-                    if (rl == 0 || nvalid == 4) enc_step<ESC>(c, sy, tab[sy]);
+                    const uint32_t sy = (v >> (8 * cb)) & 255u;
+                    if (nvalid > cb) enc_step<ESC>(c, sy, tab[sy]);
                     if ((k & 1) == 0) enc_flush(c);
                 }
             }
             const uint32_t e = enc_finish(c, endw);
-            // per column: count FL, state FL, count 3, state 3, in the set's lane-record
+            // per column and coder: count, state, in the set's lane-record
             // area (the records are written only after every packer wave has read
             // them; it lies below the guard that an outgrown lowest slot may write into)
             uint32_t* xch = reinterpret_cast<uint32_t*>(lds8 + rb + R_REC);
@@ -1785,7 +1822,7 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
     };
     for (uint32_t i = 0;; i++) {
         const uint32_t s = i & 1;
-        ws_wait_ge(&pc.coded[s], 2 * ((i >> 1) + 1));
+        ws_wait_ge(&pc.coded[s], NC * ((i >> 1) + 1));
         const uint32_t u = __builtin_amdgcn_readfirstlane(ws_load(&pc.unit[s]));
         if (u >= g.n_units) break;
         const uint64_t t_seen = phase ? wall_clock64() : 0;
@@ -1794,21 +1831,26 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
         const uint8_t* usrc = src + ubase;
         const uint32_t rb = reg0 + (2 * pr + s) * rbytes;
         uint2* lrec = reinterpret_cast<uint2*>(lds8 + rb + R_REC);  // per lane {LDS address of unit byte 0, lane end}
-        static_assert(R_REC + 1024 <= R_SLOTS - 516, "exchange words below the guard of the lowest slot");
+        static_assert(R_REC + 512 * NC <= R_SLOTS - 516, "exchange words below the guard of the lowest slot");
         uint8_t* bmap_w = lds8 + rb + R_MAP;                           // 64-byte block → lane (1025)
-        const uint32_t end0 = rb + R_SLOTS + j * fp.stride0 + fp.sl0;
-        const uint32_t end1 = rb + R_SLOTS + 64 * fp.stride0 + j * fp.stride1 + fp.sl1;
         const uint32_t* xch = reinterpret_cast<const uint32_t*>(lds8 + rb + R_REC);
-        const uint32_t e0 = xch[j], x0 = xch[64 + j];
-        const uint32_t e1 = xch[128 + j], x1 = xch[192 + j];
+        uint32_t le[NC], lx[NC];
+        bool over = false;  // the lowest dword a lane wrote must lie in its slot
+#pragma unroll
+        for (uint32_t r = 0; r < NC; r++) {
+            le[r] = xch[128 * r + j];
+            lx[r] = xch[128 * r + 64 + j];
+            over |= ((le[r] + 3u) & ~3u) > (SPE > 0 && r ? fp.sl1 : fp.sl0);
+        }
         ws_signal(&pc.xread, 1u, j);  // once all NPK have, the records may overwrite them
         // byte counts, final states and LDS stream starts of the four lanes of column j
         uint32_t cnt[4], fs[4], sa[4];
 #pragma unroll
         for (int b = 0; b < 4; b++) {
-            if (b == FL) { cnt[b] = e0; fs[b] = x0; sa[b] = end0 - e0; }
-            else if (b == 3) { cnt[b] = e1; fs[b] = x1; sa[b] = end1 - e1; }
-            else {
+            if (lane_is_live<SPE>(b)) {
+                const uint32_t r = SPE == 0 ? b : (b == 3 ? 1 : 0);
+                cnt[b] = le[r]; fs[b] = lx[r]; sa[b] = slot_end(rb, r) - le[r];
+            } else {
                 const uint32_t pb = col + b;
                 const uint32_t Kb = len > pb ? (len - pb + 255) / 256 : 0u;
                 const uint32_t ent = (chdr[0] == Kb) ? 0u : ((chdr[4] == Kb) ? 1u : 2u);
@@ -1828,8 +1870,6 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
         const uint32_t excl = incl - tsum;
         const bool raw = total >= len;
         const uint32_t size = raw ? len : total;
-        // the lowest dword a lane wrote must lie in its slot
-        const bool over = ((e0 + 3u) & ~3u) > fp.sl0 || ((e1 + 3u) & ~3u) > fp.sl1;
         const bool any_over = __ballot(over) != 0;
 
         uint64_t t_off = 0;
@@ -2019,7 +2059,7 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
 
 
 template <int SPE, bool ESC, bool SIDE, int PAIRS, int NPK, bool LIST = false>
-__global__ void __launch_bounds__(64 * (2 + NPK) * PAIRS) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(64 * ((SPE ? 2 : 4) + NPK) * PAIRS) __attribute__((amdgpu_waves_per_eu(4)))
 encode_fast_kernel(const uint8_t* __restrict__ src, EncodeGeom g, const EncSym* __restrict__ d_enc,
                    const uint32_t* __restrict__ canon, FastEncParams fp, ckr_stream_header* __restrict__ hdrs,
                    uint8_t* __restrict__ sidecar, uint8_t* __restrict__ out, uint64_t* __restrict__ unit_off,
@@ -2035,7 +2075,7 @@ encode_fast_kernel(const uint8_t* __restrict__ src, EncodeGeom g, const EncSym* 
 // own tickets, look-back and outputs.  One launch instead of one per tensor,
 // and no tensor waits for another's workgroups to leave the CUs.
 template <int SPE, bool SIDE, int PAIRS, int NPK>
-__global__ void __launch_bounds__(64 * (2 + NPK) * PAIRS) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(64 * ((SPE ? 2 : 4) + NPK) * PAIRS) __attribute__((amdgpu_waves_per_eu(4)))
 encode_fast_multi_kernel(FastJobs J) {
     uint32_t k = 0;
     while (k + 1 < J.n && J.j[k + 1].wg0 <= blockIdx.x) k++;
@@ -2051,14 +2091,15 @@ uint64_t encode_fast_status_words(uint64_t n_units) { return n_units + 2 * ((n_u
 
 // Coder pairs per workgroup that fit the LDS limit (0: none).
 static uint32_t fast_enc_pairs(const FastEncParamsHost& p, uint32_t lds_limit) {
-    for (uint32_t pairs = 2; pairs >= 1; pairs--)
-        if (ws_lds_bytes(pairs, p.canon_bytes, slot_stride(p.sl0), slot_stride(p.sl1)) <= lds_limit) return pairs;
+    const uint32_t nc = p.unmasked ? 4 : 2;
+    for (uint32_t pairs = p.unmasked ? 1 : 2; pairs >= 1; pairs--)
+        if (ws_lds_bytes(pairs, p.canon_bytes, slot_stride(p.sl0), slot_stride(p.sl1), nc) <= lds_limit) return pairs;
     return 0;
 }
 
 uint32_t encode_fast_lds_bytes(const FastEncParamsHost& p, uint32_t lds_limit) {
     const uint32_t pairs = fast_enc_pairs(p, lds_limit);
-    return pairs ? ws_lds_bytes(pairs, p.canon_bytes, slot_stride(p.sl0), slot_stride(p.sl1)) : 0u;
+    return pairs ? ws_lds_bytes(pairs, p.canon_bytes, slot_stride(p.sl0), slot_stride(p.sl1), p.unmasked ? 4 : 2) : 0u;
 }
 
 hipError_t launch_encode_fast(const uint8_t* src, const EncodeGeom& g, const EncSym* d_enc, const uint32_t* canon,
@@ -2071,7 +2112,7 @@ hipError_t launch_encode_fast(const uint8_t* src, const EncodeGeom& g, const Enc
     fp.stride0 = slot_stride(hp.sl0); fp.stride1 = slot_stride(hp.sl1);
     const uint32_t pairs = fast_enc_pairs(hp, lds_limit);
     if (!pairs) return hipErrorInvalidValue;
-    const uint32_t lb = ws_lds_bytes(pairs, fp.canon_bytes, fp.stride0, fp.stride1);
+    const uint32_t lb = ws_lds_bytes(pairs, fp.canon_bytes, fp.stride0, fp.stride1, g.spe ? 2 : 4);
     const uint64_t n = g.n_units;
     hipError_t e = hipSuccess;
     // persistent grid: as many workgroups as fit on the device at once (more
@@ -2098,7 +2139,10 @@ hipError_t launch_encode_fast(const uint8_t* src, const EncodeGeom& g, const Enc
                 : run(encode_fast_kernel<SPE_, ESC_, SIDE_, 1, NPK_>, 64u * (2 + NPK_)))
 #define CKR_FAST_ENC(SPE_, ESC_, SIDE_) CKR_FAST_ENC_P(SPE_, ESC_, SIDE_, ENC_NPK)
     const bool side = sidecar != nullptr;
-    if (g.spe == 2) {
+    if (g.spe == 0) {  // one unit's four coder waves per CU, eight packers
+        e = hp.escapes ? run(encode_fast_kernel<0, true, false, 1, 2 * ENC_NPK>, 64u * (4 + 2 * ENC_NPK))
+                       : run(encode_fast_kernel<0, false, false, 1, 2 * ENC_NPK>, 64u * (4 + 2 * ENC_NPK));
+    } else if (g.spe == 2) {
         if (hp.escapes) e = side ? CKR_FAST_ENC(2, true, true) : CKR_FAST_ENC(2, true, false);
         else e = side ? CKR_FAST_ENC(2, false, true) : CKR_FAST_ENC(2, false, false);
     } else {
@@ -2118,16 +2162,17 @@ hipError_t launch_encode_fast_multi(const FastJob* jobs, uint32_t n, uint32_t ld
     uint32_t pairs = 2, lb = 0;
     uint64_t units = 0;
     for (uint32_t i = 0; i < n; i++) {
-        if (jobs[i].g.spe != spe || (jobs[i].sidecar != nullptr) != side || (spe != 1 && spe != 2))
+        if (jobs[i].g.spe != spe || (jobs[i].sidecar != nullptr) != side || spe < 0 || spe > 2)
             return hipErrorInvalidValue;
-        const FastEncParamsHost hp{jobs[i].sl0, jobs[i].sl1, jobs[i].cw, jobs[i].canon_bytes, false};
+        const FastEncParamsHost hp{jobs[i].sl0, jobs[i].sl1, jobs[i].cw, jobs[i].canon_bytes, false, spe == 0};
         const uint32_t pj = fast_enc_pairs(hp, lds_limit);
         if (!pj) return hipErrorInvalidValue;
         pairs = std::min(pairs, pj);
         units += jobs[i].g.n_units;
     }
     for (uint32_t i = 0; i < n; i++)
-        lb = std::max(lb, ws_lds_bytes(pairs, jobs[i].canon_bytes, slot_stride(jobs[i].sl0), slot_stride(jobs[i].sl1)));
+        lb = std::max(lb, ws_lds_bytes(pairs, jobs[i].canon_bytes, slot_stride(jobs[i].sl0), slot_stride(jobs[i].sl1),
+                                       spe ? 2 : 4));
     int dev = 0, ncu = 0;
     hipError_t e;
     if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
@@ -2155,6 +2200,7 @@ hipError_t launch_encode_fast_multi(const FastJob* jobs, uint32_t n, uint32_t ld
         CKR_LAUNCH("encode_fast_kernel", s, kern<<<wg, nthreads, lb, s>>>(J));
         return hipGetLastError();
     };
+    if (spe == 0) return run(encode_fast_multi_kernel<0, false, 1, 2 * ENC_NPK>, 64u * (4 + 2 * ENC_NPK));
     if (spe == 2)
         return pairs == 2 ? (side ? run(encode_fast_multi_kernel<2, true, 2, ENC_NPK>, 128u * (2 + ENC_NPK))
                                   : run(encode_fast_multi_kernel<2, false, 2, ENC_NPK>, 128u * (2 + ENC_NPK)))
@@ -2174,6 +2220,7 @@ static uint32_t encode_fast_list_slot(const EncodeGeom& g) {
 }
 
 bool encode_fast_list_fits(const FastEncParamsHost& hp, const EncodeGeom& g, uint32_t lds_limit) {
+    if (g.spe == 0) return false;  // 256 such slots, twice, never fit: the general kernels redo those units
     const uint32_t st = slot_stride(encode_fast_list_slot(g));
     return ws_lds_bytes(1, hp.canon_bytes, st, st) <= lds_limit;
 }
@@ -2885,8 +2932,8 @@ seg_fast_kernel(const uint8_t* __restrict__ src, EncodeGeom g, const EncSym* __r
                     EncLane c{x0, 0u, 0u, endw};
                     if (full) {
                         const uint8_t* ucol = src + ubase + col;
-                        if (rl == 0) enc_full_rows<SPE, ESC, true, 0, ENC_GR, ENC_TR>(c, ucol, sidecar, ubase, j, 256);
-                        else enc_full_rows<SPE, ESC, true, 1, ENC_GR, ENC_TR>(c, ucol, sidecar, ubase, j, 256);
+                        if (rl == 0) enc_full_rows<SPE, ESC, true, 8u * FL, 0, ENC_GR, ENC_TR>(c, ucol, sidecar, ubase, j, 256);
+                        else enc_full_rows<SPE, ESC, true, 24u, 1, ENC_GR, ENC_TR>(c, ucol, sidecar, ubase, j, 256);
                     } else {
                         // the top segment of a partial last unit: rows from the top down,
                         // one at a time (as in encode_fast_kernel); the top row may be
@@ -3427,28 +3474,29 @@ __device__ __forceinline__ uint32_t df_sel(uint32_t o) {
     return SPE == 2 ? 0x07060100u + o * 0x0101u : 0x07010500u + o * 0x00010001u;
 }
 
-// Two rows: one window read per lane, two symbols from it.
-template <int SPE>
-__device__ __forceinline__ void df_pair(DfLane& a, DfLane& b, const uint8_t* lds8, const uint32_t* tab, uint32_t* out,
-                                        uint32_t sv0, uint32_t sv1, uint32_t sel) {
+// Two rows: one window read per lane, two symbols from it; emit(r, ea, eb) takes
+// row r's table words.
+template <typename E>
+__device__ __forceinline__ void df_pair(DfLane& a, DfLane& b, const uint8_t* lds8, const uint32_t* tab, uint32_t r,
+                                        E&& emit) {
     uint32_t wa = df_window(a, lds8), wb = df_window(b, lds8);
     uint32_t ha0, ha1, hb0, hb1;
     const uint32_t a0 = df_sym(a.x, wa, ha0, tab);
     const uint32_t b0 = df_sym(b.x, wb, hb0, tab);
-    df_store(out, df_pack<SPE>(a0, b0, sv0, sel));
+    emit(r, a0, b0);
     const uint32_t a1 = df_sym(a.x, wa, ha1, tab);
     const uint32_t b1 = df_sym(b.x, wb, hb1, tab);
-    df_store(out + 64, df_pack<SPE>(a1, b1, sv1, sel));
+    emit(r + 1, a1, b1);
     a.p8 += ha0 + ha1;
     b.p8 += hb0 + hb1;
 }
 
-// Eight rows (sidecar words sc), then the window step.
-template <int SPE>
-__device__ __forceinline__ void df_group(DfLane& a, DfLane& b, uint8_t* lds8, const uint32_t* tab, uint32_t* out,
-                                         const uint32_t (&sc)[8], uint32_t sel, const DfSrc& sr) {
+// Eight rows, then the window step.
+template <typename E>
+__device__ __forceinline__ void df_group(DfLane& a, DfLane& b, uint8_t* lds8, const uint32_t* tab, const DfSrc& sr,
+                                         E&& emit) {
 #pragma unroll
-    for (int r = 0; r < 8; r += 2) df_pair<SPE>(a, b, lds8, tab, out + 64 * r, sc[r], sc[r + 1], sel);
+    for (uint32_t r = 0; r < 8; r += 2) df_pair(a, b, lds8, tab, r, emit);
     df_step(a, lds8, sr);
     df_step(b, lds8, sr);
 }
@@ -3616,6 +3664,11 @@ __device__ __forceinline__ void decode_fast_body(const uint8_t* __restrict__ dat
         // (one in-order counter), so the loads of group g + DF_AHEAD are issued
         // before group g's output stores and wait only for stores DF_AHEAD groups old.  Loads are
         // unconditional (indices clamped to the last group) so the waits stay exact.
+        auto masked_rows = [&](uint32_t* out, const uint32_t (&sc)[8]) __attribute__((always_inline)) {
+            df_group(da, db, lds8, tab, sr, [&](uint32_t r, uint32_t ea, uint32_t eb) __attribute__((always_inline)) {
+                df_store(out + 64 * r, df_pack<SPE>(ea, eb, sc[r], sel));
+            });
+        };
         const uint32_t ng = K >> 3;  // full groups
         if (ng) {
             constexpr uint32_t A = DF_AHEAD;
@@ -3628,16 +3681,19 @@ __device__ __forceinline__ void decode_fast_body(const uint8_t* __restrict__ dat
 #pragma unroll
                 for (uint32_t q = 0; q <= A; q++) {
                     df_load_sc(sb[(q + A) % (A + 1)], sc32 + 256 * min(gi + q + A, gl));
-                    df_group<SPE>(da, db, lds8, tab, out32 + 512 * (gi + q), sb[q], sel, sr);
+                    masked_rows(out32 + 512 * (gi + q), sb[q]);
                 }
             }
 #pragma unroll
             for (uint32_t q = 0; q < A; q++)
-                if (gi + q < ng) df_group<SPE>(da, db, lds8, tab, out32 + 512 * (gi + q), sb[q], sel, sr);
+                if (gi + q < ng) masked_rows(out32 + 512 * (gi + q), sb[q]);
         }
         // at most 7 rows left: no window step needed
         uint32_t k = 8 * ng;
-        for (; k + 2 <= K; k += 2) df_pair<SPE>(da, db, lds8, tab, out32 + 64 * k, sc32[32 * k], sc32[32 * (k + 1)], sel);
+        for (; k + 2 <= K; k += 2)
+            df_pair(da, db, lds8, tab, k, [&](uint32_t r, uint32_t ea, uint32_t eb) __attribute__((always_inline)) {
+                df_store(out32 + 64 * r, df_pack<SPE>(ea, eb, sc32[32 * r], sel));
+            });
         if (k < K) {
             uint32_t wa = df_window(da, lds8), wb = df_window(db, lds8);
             uint32_t ha, hb;
@@ -3669,6 +3725,123 @@ __device__ __forceinline__ void decode_fast_body(const uint8_t* __restrict__ dat
         nbad_total += nbad;
     }
     if (nbad_total) atomicAdd(bad, nbad_total);
+}
+
+// The same for int8 and int32, whose four lanes per column are all live: a unit
+// is two waves' work, wave half h decoding lanes 4j + 2h and 4j + 2h + 1 and
+// storing those two bytes of every row (the halves meet in L2).
+__device__ __forceinline__ void decode_fast_unmasked(const uint8_t* __restrict__ data,
+                                                     const ckr_stream_header* __restrict__ hdrs,
+                                                     const uint64_t* __restrict__ unit_off,
+                                                     const uint32_t* __restrict__ d_dec, EncodeGeom g,
+                                                     uint8_t* __restrict__ dst, unsigned long long* bad) {
+    extern __shared__ uint32_t lds[];
+    uint8_t* lds8 = reinterpret_cast<uint8_t*>(lds);
+    const uint32_t* tab = reinterpret_cast<const uint32_t*>(lds);
+    for (uint32_t i = threadIdx.x; i < 4096; i += 64 * DF_WAVES) {
+        const uint32_t e = d_dec[i];  // sym | (f - 1) << 8 | cum << 20
+        lds[i] = (e & 0x000FFF00u) << 4 | (i - (e >> 20)) | (e & 255u) << 24;  // sym<<24 | (f-1)<<12 | slot-cum
+    }
+    __syncthreads();
+    const uint32_t j = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t data_len = unit_off[g.n_units];
+    const uintptr_t d0 = reinterpret_cast<uintptr_t>(data), d1 = d0 + data_len;
+    const uint32_t tb0 = DF_TAB_BYTES + wv * DF_WAVE_BYTES + 4 * j;
+    unsigned long long nbad_total = 0;
+    const uint64_t n_items = 2 * g.n_units;
+    for (uint64_t it = (uint64_t)blockIdx.x * DF_WAVES + wv; it < n_items; it += (uint64_t)gridDim.x * DF_WAVES) {
+        const uint64_t u = it >> 1;
+        const uint32_t bA = 2 * (uint32_t)(it & 1);  // first byte of this wave's half of a column
+        const uint64_t ubase = u * g.unit;
+        const uint32_t len = unit_len(g, ubase);
+        const uint64_t uoff = unit_off[u];
+        const uint8_t* ud = data + uoff;
+        const uint32_t usize = (uint32_t)(unit_off[u + 1] - uoff);
+        const ckr_stream_header* uh = hdrs + u * 256;
+        if (usize == len && uh[0].byte_count == len) {
+            if (bA == 0) decode_raw_unit<0>(ud, ubase, len, j, nullptr, dst);
+            continue;
+        }
+        const ckr_stream_header h0 = uh[4 * j + bA], h1 = uh[4 * j + bA + 1];
+        // chunks are read from the unit's 64-byte aligned base
+        const uintptr_t ua = reinterpret_cast<uintptr_t>(ud) & ~(uintptr_t)63;
+        const uint32_t g0 = (uint32_t)(reinterpret_cast<uintptr_t>(ud) - ua);
+        DfSrc sr;
+        sr.d0 = data;
+        sr.dlen = data_len;
+        sr.ua = (int64_t)ua - (int64_t)d0;
+        sr.k_lo = ua >= d0 ? 0u : 1u;
+        const int64_t k_end = min<int64_t>(((int64_t)d1 - (int64_t)ua) >> DF_CH_LOG, 0x40000000ll);
+        sr.n_in = k_end > (int64_t)sr.k_lo ? (uint32_t)(k_end - (int64_t)sr.k_lo) : 0u;
+        uint32_t nbad = 0, gea8, geb8;
+        DfLane da, db;
+        auto init = [&](DfLane& d, uint32_t& ge8, const ckr_stream_header& h, uint32_t tb) __attribute__((always_inline)) {
+            const bool ok = (uint64_t)h.buf_offset + h.byte_count <= usize;
+            nbad += ok ? 0u : 1u;
+            const uint32_t p = g0 + (ok ? h.buf_offset : 0u), pe = p + (ok ? h.byte_count : 0u);
+            d.x = h.final_state;
+            d.p8 = p << 3;
+            ge8 = pe << 3;
+            d.ch = p >> DF_CH_LOG;
+            d.last = pe > p ? (pe - 1u) >> DF_CH_LOG : d.ch;
+            d.age = 0;
+            d.tb = tb;
+        };
+        init(da, gea8, h0, tb0);
+        init(db, geb8, h1, tb0 + DF_RING_BYTES);
+        {   // the first two chunks of each stream (the second only if the stream reaches it)
+            uint4 ca[DF_CQ], cb[DF_CQ];
+            df_fetch(sr, da.ch, ca);
+            df_fetch(sr, db.ch, cb);
+            const bool a2nd = da.ch + 1u <= da.last, b2nd = db.ch + 1u <= db.last;
+            if (a2nd) df_fetch(sr, da.ch + 1u, da.c);
+            if (b2nd) df_fetch(sr, db.ch + 1u, db.c);
+            df_put(lds8, da.tb, da.ch, ca);
+            df_put(lds8, db.tb, db.ch, cb);
+            if (a2nd) df_put(lds8, da.tb, da.ch + 1u, da.c);
+            if (b2nd) df_put(lds8, db.tb, db.ch + 1u, db.c);
+        }
+        const uint32_t K = len >> 8;  // full rows; a partial row K follows when len % 256 != 0
+        uint16_t* out = reinterpret_cast<uint16_t*>(dst + ubase + 4 * j + bA);  // row k at out[128 k]
+        auto put2 = [&](uint32_t r, uint32_t ea, uint32_t eb) __attribute__((always_inline)) {
+            out[128 * r] = (uint16_t)__builtin_amdgcn_perm(eb, ea, 0x0C0C0703u);
+        };
+        uint32_t k = 0;
+        for (; k + 8 <= K; k += 8) {
+            df_group(da, db, lds8, tab, sr, put2);
+            out += 1024;
+        }
+        const uint32_t rest = K - k;  // at most 7 rows left: no window step needed
+        uint32_t q = 0;
+        for (; q + 2 <= rest; q += 2) df_pair(da, db, lds8, tab, q, put2);
+        const uint32_t r = len & 255u, nv = r > 4 * j ? min(r - 4 * j, 4u) : 0u;  // bytes of the partial row in this column
+        auto one = [&](DfLane& d) __attribute__((always_inline)) {
+            uint32_t w = df_window(d, lds8), h;
+            const uint32_t e = df_sym(d.x, w, h, tab);
+            d.p8 += h;
+            return e;
+        };
+        if (q < rest) {
+            const uint32_t ea = one(da), eb = one(db);
+            put2(q, ea, eb);
+        }
+        uint8_t* d8 = dst + ubase + 256ull * K + 4 * j;
+        if (nv > bA) d8[bA] = (uint8_t)(one(da) >> 24);
+        if (nv > bA + 1) d8[bA + 1] = (uint8_t)(one(db) >> 24);
+        nbad += (da.x != L || da.p8 != gea8) ? 1u : 0u;
+        nbad += (db.x != L || db.p8 != geb8) ? 1u : 0u;
+        nbad_total += nbad;
+    }
+    if (nbad_total) atomicAdd(bad, nbad_total);
+}
+
+__global__ void __launch_bounds__(64 * DF_WAVES) decode_fast_unmasked_kernel(const uint8_t* __restrict__ data,
+                                                                            const ckr_stream_header* __restrict__ hdrs,
+                                                                            const uint64_t* __restrict__ unit_off,
+                                                                            const uint32_t* __restrict__ d_dec,
+                                                                            EncodeGeom g, uint8_t* __restrict__ dst,
+                                                                            unsigned long long* bad) {
+    decode_fast_unmasked(data, hdrs, unit_off, d_dec, g, dst, bad);
 }
 
 template <int SPE>
@@ -4578,7 +4751,7 @@ hipError_t launch_hist_table(const HistSrc* srcs, uint32_t* const* hists, const 
         J.epoch = next_epoch();
         HistJob hj[kMaxHistJobs];
         for (uint32_t k = 0; k < m; k++)
-            if (srcs[j0 + k].spe != 1 && srcs[j0 + k].spe != 2) return hipErrorInvalidValue;
+            if (srcs[j0 + k].spe < 0 || srcs[j0 + k].spe > 2) return hipErrorInvalidValue;
         const uint32_t nb = hist_shares(srcs + j0, m, hj, hists + j0);
         for (uint32_t k = 0; k < m; k++) {
             J.j[k].h = hj[k];
@@ -4593,10 +4766,11 @@ hipError_t launch_hist_table(const HistSrc* srcs, uint32_t* const* hists, const 
 }
 // The largest slot (bytes, a multiple of 4, at most 2K + 8) whose two-pair
 // layout fits lds_cap.
-uint32_t encode_fast_max_slot(uint32_t canon_bytes, uint32_t K, uint32_t lds_cap) {
+uint32_t encode_fast_max_slot(uint32_t canon_bytes, uint32_t K, uint32_t lds_cap, bool unmasked) {
+    const uint32_t pairs = unmasked ? 1 : 2, nc = unmasked ? 4 : 2;
     uint32_t sl = (2 * K + 8 + 3) & ~3u;
-    while (sl > 8 && ws_lds_bytes(2, canon_bytes, slot_stride(sl), slot_stride(sl)) > lds_cap) sl -= 4;
-    return ws_lds_bytes(2, canon_bytes, slot_stride(sl), slot_stride(sl)) <= lds_cap ? sl : 0u;
+    while (sl > 8 && ws_lds_bytes(pairs, canon_bytes, slot_stride(sl), slot_stride(sl), nc) > lds_cap) sl -= 4;
+    return ws_lds_bytes(pairs, canon_bytes, slot_stride(sl), slot_stride(sl), nc) <= lds_cap ? sl : 0u;
 }
 hipError_t launch_build_dec_table(const TableArg& t, uint32_t* d_dec, unsigned long long* bad, hipStream_t s) {
     CKR_LAUNCH("build_dec_table_kernel", s, build_dec_table_kernel<<<16, 256, 0, s>>>(t, d_dec, bad));
@@ -4650,16 +4824,18 @@ hipError_t launch_decode_fast_multi(DecJob* jobs, uint32_t n, hipStream_t s) {
 }
 hipError_t launch_decode(const uint8_t* data, const ckr_stream_header* hdrs, const uint64_t* unit_off,
                          const uint32_t* d_dec, const EncodeGeom& g, const uint8_t* sidecar, uint8_t* dst,
-                         unsigned long long* bad, const uint32_t* canon, uint32_t cw, hipStream_t s, bool zero_bytes) {
+                         unsigned long long* bad, const uint32_t* canon, uint32_t cw, bool fast_ok, hipStream_t s,
+                         bool zero_bytes) {
     const uint32_t grid = (uint32_t)((g.n_units + 3) / 4);
     if (grid == 0) return hipSuccess;
     hipError_t e;
     bool fast_ran = false;
-    if (canon && g.spe > 0) {  // fast path
+    if (fast_ok && (canon || g.spe == 0)) {  // fast path
         const uint32_t lb = decode_fast_lds_bytes();
         int dev = 0, ncu = 0;
         if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
         if ((e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+        const uint64_t items = g.spe ? g.n_units : 2 * g.n_units;  // waves' worth of work
         auto fast = [&](auto kern) -> hipError_t {
             int per_cu = 0;
             if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lb) != hipSuccess ||
@@ -4668,13 +4844,16 @@ hipError_t launch_decode(const uint8_t* data, const ckr_stream_header* hdrs, con
                 return hipSuccess;  // LDS too small on this device: the general kernel takes every unit
             }
             // persistent: the blocks that fit at once, never more than needed
-            const uint64_t need = (g.n_units + DF_WAVES - 1) / DF_WAVES;
+            const uint64_t need = (items + DF_WAVES - 1) / DF_WAVES;
             const uint32_t fg = (uint32_t)std::min<uint64_t>(need, (uint64_t)per_cu * (uint64_t)std::max(ncu, 1));
-            CKR_LAUNCH("decode_fast_kernel", s, kern<<<fg, 64 * DF_WAVES, lb, s>>>(data, hdrs, unit_off, d_dec, canon, cw, g, sidecar, dst, bad, zero_bytes ? 1u : 0u));
+            if constexpr (std::is_same_v<decltype(kern), decltype(&decode_fast_unmasked_kernel)>)
+                CKR_LAUNCH("decode_fast_kernel", s, kern<<<fg, 64 * DF_WAVES, lb, s>>>(data, hdrs, unit_off, d_dec, g, dst, bad));
+            else
+                CKR_LAUNCH("decode_fast_kernel", s, kern<<<fg, 64 * DF_WAVES, lb, s>>>(data, hdrs, unit_off, d_dec, canon, cw, g, sidecar, dst, bad, zero_bytes ? 1u : 0u));
             fast_ran = true;
             return hipGetLastError();
         };
-        if ((e = (g.spe == 2 ? fast(decode_fast_kernel<2>) : fast(decode_fast_kernel<1>))) != hipSuccess) return e;
+        if ((e = (g.spe == 0 ? fast(decode_fast_unmasked_kernel) : g.spe == 2 ? fast(decode_fast_kernel<2>) : fast(decode_fast_kernel<1>))) != hipSuccess) return e;
         if (fast_ran) return hipSuccess;  // the fast kernel decodes every unit
     }
     if (g.spe == 2) CKR_LAUNCH("decode_kernel", s, decode_kernel<2><<<grid, 256, 0, s>>>(data, hdrs, unit_off, d_dec, g, sidecar, dst, bad));
