@@ -1,14 +1,14 @@
 // checkers_amd/csrc/ckr_analyzer.hip — the statistics pass of TensorAnalyzer
 // (src/TensorAnalyzer.cpp:64-198 compute_tensor_stats, :200-229
 // tensor_stats_kernel, :281-290 the fingerprint) for any number of records in
-// four launches: every record's blocks share one grid per pass.
+// two launches behind the records' descriptors: every record's blocks share one
+// grid per pass, and a record's last block to finish closes the pass for it.
 //
-//   pass 1  min, max and the fp64 sum of each block's share of its record
-//   mid     per record: min, max, mean and the histogram scale
+//   pass 1  min, max and the fp64 sum of each block's share of its record;
+//           last block: the record's min, max, mean and histogram scale
 //   pass 2  per block: the 256-bin histogram (LDS, 16 copies, then added to
 //           the record's histogram with global atomics) and the fp64 central
-//           power sums 2..4
-//   final   per record: moments, min/max and fingerprint
+//           power sums 2..4; last block: moments, min/max and fingerprint
 //
 // Each block reads its share with 16-byte loads; the elements before the
 // first 16-byte boundary of a record and those after its last whole vector
@@ -32,15 +32,24 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kHistCopies = 16;  // 8, 16, 32 within 2%; 64 (a copy per lane) 35% slower
-// Loads in flight per thread, and the grid: at most 256 workgroups per record,
-// so that pass 2's closing global atomics (one per histogram bin and
-// workgroup) stay few.  Measured on the cfg3 shard (4 records of 1G elements):
-// 2048 workgroups per record and 2 loads in pass 2, 5.18 ms per call; 512,
-// 4.95; 256, 4.70; 256 with 4 loads in pass 2, 4.61 (passes at 6.27 and 6.01
-// TB/s); 128, 6.34 (pass 2 then lacks waves to hide its latency).
-constexpr int kUnroll1 = 4, kUnroll2 = 4;
-constexpr uint64_t kBytesPerBlock = 128 * 1024;
-constexpr uint32_t kMaxBlocksPerRecord = 256;
+// Loads in flight per thread.  Pass 2 with 4 takes 103 VGPRs, so half the waves
+// fit; with 2, held to 64 VGPRs, all 8 per SIMD.  For 144 records of 1.53 GB in
+// all the whole call takes 592 us with 2 and 650 with 4 (721 with 4, 128 KiB
+// blocks and closing kernels of their own); for four records of 1G elements
+// (long loops per thread) 4742 us with 2 and 4650 with 4.  So 4 from
+// kLongBlock bytes per block (about 4 GB a call) on.
+constexpr int kUnroll1 = 4;
+constexpr uint64_t kLongBlock = 2 << 20;
+// At most 256 workgroups per record, so that pass 2's closing global atomics
+// (one per histogram bin and workgroup) stay few (four records of 1G elements:
+// 2048 workgroups per record 5.18 ms per call; 512, 4.95; 256, 4.70; 128, 6.34).
+constexpr uint32_t kMaxBlocksPerRecord = 256;  // at most kThreads: the last block reduces one partial per thread
+// Bytes per block: the records' total over about what the device holds at once
+// (256 CUs, 8 blocks each by LDS), so that a call is one round of blocks and a
+// block's fixed costs (clearing and flushing the LDS histogram, up to 256 global
+// atomics) are paid as rarely as the parallelism allows; at least 32 KiB, below
+// which they outweigh the reading.
+constexpr uint64_t kBlocksPerCall = 1900, kMinBytesPerBlock = 32 * 1024;
 constexpr uint32_t kDescPerStore = 40;
 
 // A record as the kernels see it.
@@ -50,6 +59,7 @@ struct StatsDesc {
     uint32_t dt, bins;   // dtype tag; bins requested
     uint32_t blk0, nblk; // first block of the record in the grid, its block count
     uint32_t head;       // elements before the first 16-byte boundary
+    uint32_t done[2];    // blocks that have finished pass 1, pass 2
     uint32_t pad;
     uint32_t* hist;
     float *mom, *mm, *fp;
@@ -168,6 +178,36 @@ __device__ __forceinline__ T block_reduce(T v, T* sh, Op op) {
     return r;
 }
 
+// A block's partial result, read by another block of the same launch (on another
+// XCD perhaps): device-scope stores, complete before the block takes its ticket,
+// and device-scope loads by the record's last block.
+template <typename T>
+__device__ __forceinline__ void partial_store(T* p, const T& v) {
+    static_assert(sizeof(T) % 8 == 0, "whole 64-bit words");
+    const auto* w = reinterpret_cast<const unsigned long long*>(&v);
+    auto* q = reinterpret_cast<unsigned long long*>(p);
+    for (uint32_t i = 0; i < sizeof(T) / 8; i++) __hip_atomic_store(q + i, w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T partial_load(const T* p) {
+    T v;
+    auto* w = reinterpret_cast<unsigned long long*>(&v);
+    auto* q = reinterpret_cast<unsigned long long*>(const_cast<T*>(p));
+    for (uint32_t i = 0; i < sizeof(T) / 8; i++) w[i] = __hip_atomic_load(q + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return v;
+}
+// Thread 0 has stored the block's partial: true in every thread of the record's
+// last block.
+__device__ __forceinline__ bool last_block(uint32_t* done, uint32_t nblk) {
+    __shared__ uint32_t last;
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_s_waitcnt(0);  // the partial's stores are complete
+        last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nblk - 1;
+    }
+    __syncthreads();
+    return last;
+}
+
 // The sum of one vector's elements in fp32 (at most 16 terms), then into the
 // fp64 total.
 template <uint32_t DT>
@@ -186,8 +226,9 @@ __device__ void pass1_share(const StatsDesc& d, uint32_t lb, float& mn, float& m
         });
 }
 
-__global__ void __launch_bounds__(kThreads) stats_pass1_kernel(const StatsDesc* __restrict__ desc, uint32_t n_rec,
-                                                               StatsPartial1* __restrict__ out) {
+__global__ void __launch_bounds__(kThreads) stats_pass1_kernel(StatsDesc* __restrict__ desc, uint32_t n_rec,
+                                                               StatsPartial1* __restrict__ out,
+                                                               StatsParams* __restrict__ prm) {
     __shared__ float shf[kThreads];
     __shared__ double shd[kThreads];
     const uint32_t r = record_of(desc, n_rec, blockIdx.x);
@@ -205,19 +246,13 @@ __global__ void __launch_bounds__(kThreads) stats_pass1_kernel(const StatsDesc* 
     mn = block_reduce(mn, shf, [](float a, float b) { return fminf(a, b); });
     mx = block_reduce(mx, shf, [](float a, float b) { return fmaxf(a, b); });
     sm = block_reduce(sm, shd, [](double a, double b) { return a + b; });
-    if (threadIdx.x == 0) out[blockIdx.x] = StatsPartial1{mn, mx, sm};
-}
-
-__global__ void __launch_bounds__(kThreads) stats_mid_kernel(const StatsDesc* __restrict__ desc,
-                                                             const StatsPartial1* __restrict__ p1,
-                                                             StatsParams* __restrict__ prm) {
-    __shared__ float shf[kThreads];
-    __shared__ double shd[kThreads];
-    const StatsDesc d = desc[blockIdx.x];
-    float mn = 1e37f, mx = -1e37f;
-    double sm = 0.0;
-    for (uint32_t b = threadIdx.x; b < d.nblk; b += kThreads) {
-        const StatsPartial1 q = p1[d.blk0 + b];
+    if (threadIdx.x == 0) partial_store(out + blockIdx.x, StatsPartial1{mn, mx, sm});
+    if (!last_block(&desc[r].done[0], d.nblk)) return;
+    mn = 1e37f;
+    mx = -1e37f;
+    sm = 0.0;
+    if (threadIdx.x < d.nblk) {
+        const StatsPartial1 q = partial_load(out + d.blk0 + threadIdx.x);
         mn = fminf(mn, q.mn);
         mx = fmaxf(mx, q.mx);
         sm += q.sum;
@@ -237,13 +272,13 @@ __global__ void __launch_bounds__(kThreads) stats_mid_kernel(const StatsDesc* __
         q.scale = q.use_range ? (float)((double)((float)bins - 1.0f) / (double)range) : 0.0f;
         q.bins = bins;
         q.pad[0] = q.pad[1] = 0;
-        prm[blockIdx.x] = q;
+        prm[r] = q;
     }
 }
 
 // Central powers as the reference forms them (float d = x - mean), summed in
 // fp32 over one vector's elements, then into fp64 totals.
-template <uint32_t DT>
+template <uint32_t DT, int kUnroll2>
 __device__ void pass2_share(const StatsDesc& d, uint32_t lb, const StatsParams& q, uint32_t* sh, double& a2,
                             double& a3, double& a4) {
     const uint32_t c = threadIdx.x & (kHistCopies - 1);
@@ -273,7 +308,8 @@ __device__ void pass2_share(const StatsDesc& d, uint32_t lb, const StatsParams& 
         });
 }
 
-__global__ void __launch_bounds__(kThreads) stats_pass2_kernel(const StatsDesc* __restrict__ desc, uint32_t n_rec,
+template <int U>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(U == 2 ? 8 : 4))) stats_pass2_kernel(StatsDesc* __restrict__ desc, uint32_t n_rec,
                                                                const StatsParams* __restrict__ prm,
                                                                StatsPartial2* __restrict__ out) {
     __shared__ uint32_t sh[256 * kHistCopies];
@@ -286,11 +322,11 @@ __global__ void __launch_bounds__(kThreads) stats_pass2_kernel(const StatsDesc* 
     const uint32_t lb = blockIdx.x - d.blk0;
     double a2 = 0, a3 = 0, a4 = 0;
     switch (d.dt) {
-        case CKR_F32: pass2_share<CKR_F32>(d, lb, q, sh, a2, a3, a4); break;
-        case CKR_BF16: pass2_share<CKR_BF16>(d, lb, q, sh, a2, a3, a4); break;
-        case CKR_F16: pass2_share<CKR_F16>(d, lb, q, sh, a2, a3, a4); break;
-        case CKR_I8: pass2_share<CKR_I8>(d, lb, q, sh, a2, a3, a4); break;
-        default: pass2_share<CKR_I32>(d, lb, q, sh, a2, a3, a4); break;
+        case CKR_F32: pass2_share<CKR_F32, U>(d, lb, q, sh, a2, a3, a4); break;
+        case CKR_BF16: pass2_share<CKR_BF16, U>(d, lb, q, sh, a2, a3, a4); break;
+        case CKR_F16: pass2_share<CKR_F16, U>(d, lb, q, sh, a2, a3, a4); break;
+        case CKR_I8: pass2_share<CKR_I8, U>(d, lb, q, sh, a2, a3, a4); break;
+        default: pass2_share<CKR_I32, U>(d, lb, q, sh, a2, a3, a4); break;
     }
     const auto add = [](double a, double b) { return a + b; };
     a2 = block_reduce(a2, shd, add);
@@ -301,24 +337,16 @@ __global__ void __launch_bounds__(kThreads) stats_pass2_kernel(const StatsDesc* 
         for (int k = 0; k < kHistCopies; k++) hs += sh[threadIdx.x * kHistCopies + k];
         if (hs) atomicAdd(&d.hist[threadIdx.x], hs);
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = StatsPartial2{a2, a3, a4, 0.0};
-}
-
-__global__ void __launch_bounds__(kThreads) stats_final_kernel(const StatsDesc* __restrict__ desc,
-                                                               const StatsPartial2* __restrict__ p2,
-                                                               const StatsParams* __restrict__ prm) {
-    __shared__ double shd[kThreads];
-    const StatsDesc d = desc[blockIdx.x];
-    const StatsParams q = prm[blockIdx.x];
+    if (threadIdx.x == 0) partial_store(out + blockIdx.x, StatsPartial2{a2, a3, a4, 0.0});
+    if (!last_block(&desc[r].done[1], d.nblk)) return;
     const uint32_t t = threadIdx.x;
     double m2 = 0, m3 = 0, m4 = 0;
-    for (uint32_t b = t; b < d.nblk; b += kThreads) {
-        const StatsPartial2 v = p2[d.blk0 + b];
+    if (t < d.nblk) {
+        const StatsPartial2 v = partial_load(out + d.blk0 + t);
         m2 += v.m2;
         m3 += v.m3;
         m4 += v.m4;
     }
-    const auto add = [](double a, double b) { return a + b; };
     m2 = block_reduce(m2, shd, add);
     m3 = block_reduce(m3, shd, add);
     m4 = block_reduce(m4, shd, add);
@@ -342,9 +370,18 @@ bool analyzable(const ckr_stats_record& r) {
                                          r.data_type == CKR_F16 || r.data_type == CKR_I8 || r.data_type == CKR_I32);
 }
 
-uint32_t blocks_for(const ckr_stats_record& r) {
-    const uint64_t bytes = r.num_elements * (uint64_t)ckr_element_size((int)r.data_type);
-    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((bytes + kBytesPerBlock - 1) / kBytesPerBlock, 1),
+uint64_t record_bytes(const ckr_stats_record& r) {
+    return r.num_elements * (uint64_t)ckr_element_size((int)r.data_type);
+}
+uint64_t bytes_per_block(const ckr_stats_record* recs, uint64_t n) {
+    uint64_t total = 0;
+    for (uint64_t i = 0; i < n; i++)
+        if (analyzable(recs[i])) total += record_bytes(recs[i]);
+    return std::max(kMinBytesPerBlock, (total / kBlocksPerCall + 4095) / 4096 * 4096);
+}
+uint32_t blocks_for(const ckr_stats_record& r, uint64_t per_block) {
+    static_assert(kMaxBlocksPerRecord <= kThreads, "one partial per thread of the last block");
+    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((record_bytes(r) + per_block - 1) / per_block, 1),
                                         kMaxBlocksPerRecord);
 }
 
@@ -367,10 +404,11 @@ Layout layout(uint64_t n_rec, uint64_t n_blk) {
 
 uint64_t analyze_workspace_bytes(const ckr_stats_record* recs, uint64_t n) {
     uint64_t nr = 0, nb = 0;
+    const uint64_t per_block = bytes_per_block(recs, n);
     for (uint64_t i = 0; i < n; i++)
         if (analyzable(recs[i])) {
             nr++;
-            nb += blocks_for(recs[i]);
+            nb += blocks_for(recs[i], per_block);
         }
     return nr ? layout(nr, nb).total : 0;
 }
@@ -378,6 +416,7 @@ uint64_t analyze_workspace_bytes(const ckr_stats_record* recs, uint64_t n) {
 hipError_t launch_analyze(const ckr_stats_record* recs, uint64_t n, void* ws, hipStream_t s) {
     std::vector<StatsDesc> d;
     uint64_t nb = 0;
+    const uint64_t per_block = bytes_per_block(recs, n);
     for (uint64_t i = 0; i < n; i++) {
         const ckr_stats_record& r = recs[i];
         if (!analyzable(r)) continue;  // TensorAnalyzer.cpp:68, tensor_stats_kernel's default branch
@@ -387,7 +426,7 @@ hipError_t launch_analyze(const ckr_stats_record* recs, uint64_t n, void* ws, hi
         x.dt = r.data_type;
         x.bins = r.histogram_bins;
         x.blk0 = (uint32_t)nb;
-        x.nblk = blocks_for(r);
+        x.nblk = blocks_for(r, per_block);
         const uint64_t es = (uint64_t)ckr_element_size((int)r.data_type);
         const uint64_t mis = reinterpret_cast<uintptr_t>(r.d_ptr) & 15u;
         x.head = (uint32_t)std::min<uint64_t>(mis ? (16 - mis) / es : 0, r.num_elements);
@@ -414,10 +453,9 @@ hipError_t launch_analyze(const ckr_stats_record* recs, uint64_t n, void* ws, hi
         CKR_LAUNCH("stats_desc_store_kernel", s, stats_desc_store_kernel<<<1, 64, 0, s>>>(a, desc));
     }
     const uint32_t nr = (uint32_t)d.size();
-    CKR_LAUNCH("stats_pass1_kernel", s, stats_pass1_kernel<<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, p1));
-    CKR_LAUNCH("stats_mid_kernel", s, stats_mid_kernel<<<nr, kThreads, 0, s>>>(desc, p1, prm));
-    CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
-    CKR_LAUNCH("stats_final_kernel", s, stats_final_kernel<<<nr, kThreads, 0, s>>>(desc, p2, prm));
+    CKR_LAUNCH("stats_pass1_kernel", s, stats_pass1_kernel<<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, p1, prm));
+    if (per_block >= kLongBlock) CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<4><<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
+    else CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<2><<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
     return hipGetLastError();
 }
 

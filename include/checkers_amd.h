@@ -312,7 +312,7 @@ CKR_API int ckr_decode_noalloc(const uint8_t* d_data, const ckr_stream_header* d
                                uint64_t* h_bad_lanes, void* stream);
 
 /* ---- TensorAnalyzer statistics pass over n records ----
- * All records go through four launches (two passes over the data, each with
+ * All records go through two launches (two passes over the data, each with
  * every record's blocks in one grid).  The workspace size depends on each
  * record's pointer, element count and dtype (records with a null pointer, no
  * elements or an unknown dtype are skipped, as the reference skips them);
