@@ -1176,8 +1176,7 @@ namespace {
 constexpr int kUseHostTable = 1;  // compress_device_table: take the host's sorted table instead
 
 // The symbol-0 state chains of every count (ckr::launch_canon_chains), one
-// buffer per device, made and filled on first use on the caller's stream (so
-// that the first encode finds them filled) and kept for the process.
+// buffer per device, made and filled on first use and kept for the process.
 const void* canon_chains(hipStream_t s) {
     static std::mutex mu;
     static std::vector<void*> per_dev;
@@ -1186,9 +1185,21 @@ const void* canon_chains(hipStream_t s) {
     std::lock_guard<std::mutex> lk(mu);
     if ((int)per_dev.size() <= dev) per_dev.resize(dev + 1, nullptr);
     if (!per_dev[dev]) {
+        // a capturing stream can neither allocate nor fill them: the callers have
+        // paths that do without
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
         void* p = nullptr;
         if (hipMalloc(&p, ckr::kChainBytes) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-        if (ckr::launch_canon_chains(p, s) != hipSuccess) { (void)hipGetLastError(); (void)hipFree(p); return nullptr; }
+        // filled before any other stream or thread can see them (once per process)
+        if (ckr::launch_canon_chains(p, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipFree(p);
+            return nullptr;
+        }
         per_dev[dev] = p;
     }
     return per_dev[dev];
@@ -1269,7 +1280,8 @@ int dev_enc_queue_encode(const DevEnc& d, hipStream_t s) {
 }
 
 // The encode and, right behind it with no read-back between them, the redo
-// pass (it ends at once when no unit outgrew its slots).
+// pass (it ends at once when no unit outgrew its slots), which also writes the
+// control and table words to d.pin; where it does not fit, a copy does.
 int dev_enc_queue_encode_redo(DevEnc& d, hipStream_t s) {
     if (int rc = dev_enc_queue_encode(d, s)) return rc;
     const uint32_t lds_limit = (uint32_t)max_lds_per_block();
@@ -1278,8 +1290,10 @@ int dev_enc_queue_encode_redo(DevEnc& d, hipStream_t s) {
         CKR_HIP(ckr::launch_encode_fast_list(d.src, d.g, reinterpret_cast<ckr::EncSym*>(d.ws + L.off_enc),
                                              reinterpret_cast<uint32_t*>(d.ws + L.off_canon), d.fp, lds_limit, d.hdrs,
                                              d.out, d.unit_off, reinterpret_cast<uint64_t*>(d.ws + L.off_status), d.dctl,
-                                             reinterpret_cast<uint32_t*>(d.ws + L.off_redo), s));
+                                             reinterpret_cast<uint32_t*>(d.ws + L.off_redo), s, d.pin, kCtlWords));
         d.redo_queued = true;
+    } else {
+        CKR_HIP(hipMemcpyAsync(d.pin, d.dctl, kCtlWords * 4, hipMemcpyDeviceToHost, s));
     }
     return CKR_OK;
 }
@@ -1366,10 +1380,14 @@ int compress_device_table(const void* src, const ckr::EncodeGeom& g, int ensure_
         (void)hipStreamSynchronize(s);  // the set-up writes the caller's workspace
         return rc;
     }
+    pw[6] = pw[7] = 0;  // the epoch words: no stale report passes for this call's
     rc = dev_enc_queue_encode_redo(d, s);
     if (rc) return rc;
-    CKR_HIP(hipMemcpyAsync(pw, d.dctl, kCtlWords * 4, hipMemcpyDeviceToHost, s));
     CKR_HIP(hipStreamSynchronize(s));
+    if (pw[1] && d.redo_queued) {  // units were coded again: the flags they may have raised
+        CKR_HIP(hipMemcpyAsync(pw, d.dctl, 16, hipMemcpyDeviceToHost, s));
+        CKR_HIP(hipStreamSynchronize(s));
+    }
     bool more = false;
     rc = dev_enc_finish(d, h_table, h_total_out, &more, s);
     if (rc == CKR_OK && more) CKR_HIP(hipStreamSynchronize(s));  // the output complete, as on the other paths
@@ -1919,8 +1937,15 @@ int decode_impl(const uint8_t* d_data, const ckr_stream_header* d_headers, const
     auto* dec = reinterpret_cast<uint32_t*>(ws + L.off_dec);
     auto* bad = reinterpret_cast<unsigned long long*>(ws + L.off_bad);
     const CanonKs ck = canon_ks(g);
-    CKR_HIP(ckr::launch_build_dec_table(ta, dec, bad, s));  // also clears the bad-lane counter
-    if (L.fast) CKR_HIP(canon_launch(h_table, ck, canon, s));
+    // decode table, canonical streams and a cleared bad-lane counter: one launch
+    // where the state chains cover the lane counts (units up to 64 KiB)
+    const void* chains = L.fast && !noalloc && std::max(ck.k0, ck.k1) <= ckr::kChainSteps ? canon_chains(s) : nullptr;
+    if (chains) {
+        CKR_HIP(ckr::launch_dec_setup(ta, dec, canon, bad, ck.k0, ck.k1, ck.k2, ck.cw, chains, s));
+    } else {
+        CKR_HIP(ckr::launch_build_dec_table(ta, dec, bad, s));
+        if (L.fast) CKR_HIP(canon_launch(h_table, ck, canon, s));
+    }
     // the decoders store 32-bit words at the 4-byte columns of the destination:
     // a destination that is only element-aligned receives a copy
     uint8_t* out = static_cast<uint8_t*>(d_dst);

@@ -70,6 +70,11 @@ hipError_t launch_build_enc_table_reset(const TableArg& t, EncSym* d_enc, uint64
 // bad (may be null): a bad-lane counter to clear in the same launch.
 hipError_t launch_build_dec_table(const TableArg& t, uint32_t* d_dec, unsigned long long* bad, hipStream_t s);
 
+// The same and the canonical zero-plane streams of lane counts k0, k1, k2 (at
+// most kChainSteps each) from the state chains, in one launch.
+hipError_t launch_dec_setup(const TableArg& t, uint32_t* d_dec, uint32_t* canon, unsigned long long* bad, uint32_t k0,
+                            uint32_t k1, uint32_t k2, uint32_t cw, const void* chains, hipStream_t s);
+
 hipError_t launch_extract_mantissa(const uint8_t* src, uint64_t n_elems, int es, int spe,
                                    uint8_t* masked, uint8_t* sidecar, hipStream_t s);
 
@@ -141,12 +146,15 @@ struct FastEncParamsHost {
 uint32_t encode_fast_lds_bytes(const FastEncParamsHost& p, uint32_t lds_limit);
 // The fast encoder's redo list (ctl[1] units) coded again: one coder pair per
 // workgroup with slots that hold any lane; false/error when those slots do not
-// fit lds_limit.
+// fit lds_limit.  report (may be null): pinned host memory that receives
+// ctl[0 .. n_report) as they are when the launch begins, in place of a copy
+// behind it.
 bool encode_fast_list_fits(const FastEncParamsHost& p, const EncodeGeom& g, uint32_t lds_limit);
 hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, const EncSym* d_enc, const uint32_t* canon,
                                    const FastEncParamsHost& hp, uint32_t lds_limit, ckr_stream_header* hdrs,
                                    uint8_t* out, uint64_t* unit_off, uint64_t* status, uint32_t* ctl,
-                                   uint32_t* redo_list, hipStream_t s);
+                                   uint32_t* redo_list, hipStream_t s, uint32_t* report = nullptr,
+                                   uint32_t n_report = 0);
 // Several tensors' fast encodes in one launch (same spe, sidecars for all or
 // none, tables the data's own): each job's arguments as launch_encode_fast's,
 // dsl its device slot sizes (sl0, sl1: the largest the launch's LDS holds);

@@ -1664,6 +1664,7 @@ __host__ __device__ constexpr uint32_t ws_lds_bytes(uint32_t pairs, uint32_t can
 // redo_list) coded again with slots large enough for any lane (2 bytes per
 // row), at the offsets that launch published; tickets from ctl[3]; no sidecar,
 // no look-back.  A lane that outgrew even those slots would set ctl[2] bit 1.
+// report (LIST): ctl[0 .. n_report) as they are at the launch, copied there first.
 template <int SPE, bool ESC, bool SIDE, int PAIRS, int NPK, bool LIST>
 __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src, EncodeGeom g,
                                                  const EncSym* __restrict__ d_enc,
@@ -1674,7 +1675,10 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
                                                  uint64_t* __restrict__ status, uint32_t* __restrict__ ctl,
                                                  uint32_t* __restrict__ redo_list,
                                                  uint64_t* __restrict__ phase,
-                                                 const uint32_t* __restrict__ dsl) {
+                                                 const uint32_t* __restrict__ dsl, uint32_t* report,
+                                                 uint32_t n_report) {
+    if (LIST && report && blockIdx.x == 0)  // (see launch_encode_fast_list)
+        for (uint32_t i = threadIdx.x; i < n_report; i += blockDim.x) report[i] = ctl[i];
     if (LIST && __hip_atomic_load(&ctl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;  // nothing to redo
     if (dsl) {  // slot sizes made on the device (table_enc_kernel), within the launch's LDS
         fp.sl0 = dsl[0]; fp.sl1 = dsl[1];
@@ -2064,9 +2068,9 @@ encode_fast_kernel(const uint8_t* __restrict__ src, EncodeGeom g, const EncSym* 
                    const uint32_t* __restrict__ canon, FastEncParams fp, ckr_stream_header* __restrict__ hdrs,
                    uint8_t* __restrict__ sidecar, uint8_t* __restrict__ out, uint64_t* __restrict__ unit_off,
                    uint64_t* __restrict__ status, uint32_t* __restrict__ ctl, uint32_t* __restrict__ redo_list,
-                   uint64_t* __restrict__ phase, const uint32_t* __restrict__ dsl) {
+                   uint64_t* __restrict__ phase, const uint32_t* __restrict__ dsl, uint32_t* report, uint32_t n_report) {
     encode_fast_body<SPE, ESC, SIDE, PAIRS, NPK, LIST>(src, g, d_enc, canon, fp, hdrs, sidecar, out, unit_off, status,
-                                                       ctl, redo_list, phase, dsl);
+                                                       ctl, redo_list, phase, dsl, report, n_report);
 }
 
 // Several tensors' fast encodes in one launch (a shard of small tensors): the
@@ -2084,7 +2088,7 @@ encode_fast_multi_kernel(FastJobs J) {
     fp.sl0 = b.sl0; fp.sl1 = b.sl1; fp.cw = b.cw; fp.canon_bytes = b.canon_bytes;
     fp.stride0 = slot_stride(b.sl0); fp.stride1 = slot_stride(b.sl1);
     encode_fast_body<SPE, false, SIDE, PAIRS, NPK, false>(b.src, b.g, b.enc, b.canon, fp, b.hdrs, b.sidecar, b.out,
-                                                          b.unit_off, b.status, b.ctl, b.redo, nullptr, b.dsl);
+                                                          b.unit_off, b.status, b.ctl, b.redo, nullptr, b.dsl, nullptr, 0u);
 }
 
 uint64_t encode_fast_status_words(uint64_t n_units) { return n_units + 2 * ((n_units + 63) / 64); }
@@ -2131,7 +2135,7 @@ hipError_t launch_encode_fast(const uint8_t* src, const EncodeGeom& g, const Enc
         const uint32_t grid = (uint32_t)std::min<uint64_t>(need, (uint64_t)per_cu * (uint64_t)std::max(ncu, 1));
         CKR_LAUNCH("encode_fast_kernel", s,
                    kern<<<grid, nthreads, lb, s>>>(src, g, d_enc, canon, fp, hdrs, sidecar, out, unit_off, status,
-                                                   ctl, redo_list, phase, dsl));
+                                                   ctl, redo_list, phase, dsl, nullptr, 0u));
         return hipGetLastError();
     };
 #define CKR_FAST_ENC_P(SPE_, ESC_, SIDE_, NPK_)                                                                  \
@@ -2228,7 +2232,7 @@ bool encode_fast_list_fits(const FastEncParamsHost& hp, const EncodeGeom& g, uin
 hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, const EncSym* d_enc, const uint32_t* canon,
                                    const FastEncParamsHost& hp, uint32_t lds_limit, ckr_stream_header* hdrs,
                                    uint8_t* out, uint64_t* unit_off, uint64_t* status, uint32_t* ctl,
-                                   uint32_t* redo_list, hipStream_t s) {
+                                   uint32_t* redo_list, hipStream_t s, uint32_t* report, uint32_t n_report) {
     if (!encode_fast_list_fits(hp, g, lds_limit)) return hipErrorInvalidValue;
     FastEncParams fp;
     fp.sl0 = fp.sl1 = encode_fast_list_slot(g);
@@ -2247,7 +2251,7 @@ hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, cons
         const uint32_t grid = (uint32_t)std::min<uint64_t>(g.n_units, (uint64_t)std::max(ncu, 1));
         CKR_LAUNCH("encode_fast_redo_kernel", s,
                    kern<<<grid, nthreads, lb, s>>>(src, g, d_enc, canon, fp, hdrs, nullptr, out, unit_off, status, ctl,
-                                                   redo_list, nullptr, nullptr));
+                                                   redo_list, nullptr, nullptr, report, n_report));
         return hipGetLastError();
     };
     if (g.spe == 2) return hp.escapes ? run(encode_fast_kernel<2, true, false, 1, ENC_NPK, true>)
@@ -3872,6 +3876,31 @@ __global__ void __launch_bounds__(64 * DF_WAVES) decode_fast_multi_kernel(DecJob
                           b.zero_bytes, blockIdx.x - b.blk0, b.nblk);
 }
 
+// The set-up of one decode in one launch (16 workgroups): as dec_setup_multi_kernel's,
+// the frequency table as a kernel argument.
+__global__ void __launch_bounds__(256) dec_setup_kernel(TableArg t, uint32_t* __restrict__ dec, uint32_t* __restrict__ canon,
+                                                        unsigned long long* bad, uint32_t k0, uint32_t k1, uint32_t k2,
+                                                        uint32_t cw, Chains ch) {
+    __shared__ uint32_t cum[257];
+    __shared__ CanonLds C;
+    for (uint32_t i = threadIdx.x; i < 257; i += 256) cum[i] = t.cum[i];
+    if (blockIdx.x == 0) {
+        const CanonLoad cl = canon_load(t.norm[0], k0, k1, k2, ch);
+        if (threadIdx.x == 0) *bad = 0;
+        canon_put(cl, C);
+    }
+    __syncthreads();
+    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+    uint32_t lo = 0, hi = 256;  // the largest symbol with cum <= j
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (cum[mid] <= j) lo = mid; else hi = mid;
+    }
+    const uint32_t f = t.norm[lo];
+    if (j < cum[256] && f) dec[j] = lo | ((f - 1u) << 8) | (cum[lo] << 20);
+    if (blockIdx.x == 0) canon_write(k0, k1, k2, cw, C, canon);
+}
+
 // The decode set-up of several tensors in one launch, one workgroup per job:
 // its decode table from the frequency table staged in device memory
 // (TableArg's norm, cum), the canonical zero-plane streams from the state
@@ -4774,6 +4803,12 @@ uint32_t encode_fast_max_slot(uint32_t canon_bytes, uint32_t K, uint32_t lds_cap
 }
 hipError_t launch_build_dec_table(const TableArg& t, uint32_t* d_dec, unsigned long long* bad, hipStream_t s) {
     CKR_LAUNCH("build_dec_table_kernel", s, build_dec_table_kernel<<<16, 256, 0, s>>>(t, d_dec, bad));
+    return hipGetLastError();
+}
+
+hipError_t launch_dec_setup(const TableArg& t, uint32_t* d_dec, uint32_t* canon, unsigned long long* bad, uint32_t k0,
+                            uint32_t k1, uint32_t k2, uint32_t cw, const void* chains, hipStream_t s) {
+    CKR_LAUNCH("dec_setup_kernel", s, dec_setup_kernel<<<16, 256, 0, s>>>(t, d_dec, canon, bad, k0, k1, k2, cw, chains_of(chains)));
     return hipGetLastError();
 }
 
