@@ -27,8 +27,10 @@
 // sequence, so first occurrences compare as the reference's do.
 //
 // Rounds run on the device with no host synchronisation inside a batch of
-// eight (one replay of a captured graph).  A build round is up to seven
-// launches, each returning at once when its case does not arise:
+// eight (one replay of a captured graph).  A build round is seven launches (a
+// full round) or the last four of them (a lean one, for rounds that need
+// neither a recount nor a tie-break; run_rounds says which when), each returning
+// at once when its case does not arise:
 //   rp_pairs<COUNT>  (recount rounds: the first, or when the table could pass
 //                    3/4 full) every adjacent pair of live tokens counted,
 //                    through a per-workgroup LDS cache of 2048 pairs in front
@@ -558,7 +560,8 @@ __device__ void commit_rule(RepairCtl* ctl, const RoundArgs& A) {
 }
 
 // The pair of the round a grid kernel works on.  Build: the one committed in
-// ctl (by rp_close or the tie-break).  Apply: rule ctl->round + ri of the
+// ctl (by rp_close or the tie-break); none while a recount or a tie is pending
+// (a lean round, whose launches leave the sequence as it is).  Apply: rule ctl->round + ri of the
 // mapped rules, ri being the round's place in its batch (ctl->round moves once
 // per batch), so that apply rounds need no closing launch.
 struct RoundSel {
@@ -573,7 +576,7 @@ struct Cur {
 __device__ __forceinline__ Cur cur_round(const RepairCtl* ctl, const RoundSel& rs) {
     Cur x;
     if (!rs.rmap) {
-        x.live = !ctl->done && !ctl->skip;
+        x.live = !ctl->done && !ctl->skip && !ctl->recount && !ctl->tie;
         x.a = ctl->a; x.b = ctl->b; x.c = ctl->c;
         x.run = ctl->run_mode != 0;
         return x;
@@ -1223,7 +1226,7 @@ __global__ void __launch_bounds__(RT) rp_write(T* __restrict__ tok, uint32_t* __
 // counts (committed when no tie needs rp_pairs<FIRST>).
 __global__ void __launch_bounds__(CLOSE_T) rp_close(uint32_t nb, RepairCtl* ctl, const uint32_t* __restrict__ bcount,
                                                     RoundArgs A) {
-    if (ctl->done) return;
+    if (ctl->done || ctl->recount || ctl->tie) return;  // (pending: rp_pairs and rp_tie come first)
     __shared__ uint32_t sh[16];
     __shared__ uint32_t s_recount;
     uint32_t occ = 0;
@@ -1445,10 +1448,10 @@ struct RoundGraphKey {
     const void* ws;
     uint64_t n;
     int es, build, device, tok16;
-    uint32_t k, rounds, dlimit, batch;
+    uint32_t k, rounds, dlimit, batch, full;
     bool operator==(const RoundGraphKey& o) const {
         return ws == o.ws && n == o.n && es == o.es && build == o.build && device == o.device && tok16 == o.tok16 &&
-               k == o.k && rounds == o.rounds && dlimit == o.dlimit && batch == o.batch;
+               k == o.k && rounds == o.rounds && dlimit == o.dlimit && batch == o.batch && full == o.full;
     }
 };
 struct RoundGraph {
@@ -1471,11 +1474,11 @@ hipStream_t side_stream(int dev, std::vector<hipStream_t>& v) {
 }
 
 template <typename BatchFn>
-hipGraphExec_t round_graph(const RepairArgs& A, const RepairLayout& L, uint32_t len, BatchFn& batch) {
+hipGraphExec_t round_graph(const RepairArgs& A, const RepairLayout& L, uint32_t len, uint32_t full, BatchFn& batch) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
     const RoundGraphKey key{A.ws, A.n, A.es, A.build, dev, L.tok16 ? 1 : 0, A.k, A.build ? A.max_rules : A.n_rules,
-                            A.recount_each_round ? 1u : 0u, len};
+                            A.recount_each_round ? 1u : 0u, len, full};
     std::lock_guard<std::mutex> lk(g_rg_mu);
     for (const RoundGraph& r : g_rgs)
         if (r.key == key) return r.x;
@@ -1485,7 +1488,7 @@ hipGraphExec_t round_graph(const RepairArgs& A, const RepairLayout& L, uint32_t 
     hipGraph_t g = nullptr;
     hipGraphExec_t x = nullptr;
     if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    const hipError_t e = batch(cs, len);
+    const hipError_t e = batch(cs, len, full);
     const hipError_t e2 = hipStreamEndCapture(cs, &g);
     if (e != hipSuccess || e2 != hipSuccess || !g || hipGraphInstantiate(&x, g, nullptr, nullptr, 0) != hipSuccess) {
         (void)hipGetLastError();
@@ -1572,12 +1575,13 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
                        const_cast<uint32_t*>(R.rmap), sym));
     }
     // One round.  Build: every kernel reads what to do from ctl, so the rounds
-    // are identical launches.  Apply: the grid kernels take the round's place
-    // in its batch and read the rule themselves, rp_find writes in place; no
-    // write or closing launch.
-    auto round = [&](hipStream_t x, uint32_t ri) -> hipError_t {
+    // are identical launches; a lean one is without the counting and the
+    // tie-break.  Apply: the grid kernels take the round's place in its batch
+    // and read the rule themselves, rp_find writes in place; no write or
+    // closing launch.
+    auto round = [&](hipStream_t x, uint32_t ri, bool full) -> hipError_t {
         const RoundSel rs{A.build ? nullptr : R.rmap, R.rounds, ri};
-        if (A.build) {
+        if (A.build && full) {
             CKR_LAUNCH("repair_count_kernel", x, (rp_pairs<T, false><<<gpair, RT, 0, x>>>(tok, len, N, ctl, R, pchunk)));
             CKR_LAUNCH("repair_first_kernel", x, (rp_pairs<T, true><<<gpair, RT, 0, x>>>(tok, len, N, ctl, R, pchunk)));
             CKR_LAUNCH("repair_select_kernel", x, rp_tie<<<1, CLOSE_T, 0, x>>>(ctl, R));
@@ -1599,9 +1603,10 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
         }
         return hipGetLastError();
     };
-    auto batch = [&](hipStream_t x, uint32_t n_rounds) -> hipError_t {
+    // `full` rounds of n_rounds, the first ones, are full.
+    auto batch = [&](hipStream_t x, uint32_t n_rounds, uint32_t full) -> hipError_t {
         for (uint32_t i = 0; i < n_rounds; i++) {
-            const hipError_t er = round(x, i);
+            const hipError_t er = round(x, i, i < full);
             if (er != hipSuccess) return er;
         }
         if (!A.build) CKR_LAUNCH("repair_close_kernel", x, rp_batch_end<<<1, 1, 0, x>>>(ctl, n_rounds));
@@ -1610,19 +1615,40 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
     // Rounds go in batches of kRoundBatch (the last one shorter), each batch
     // one launch of a graph captured once per workspace, shape and batch
     // length and kept (a round is up to 7 launches, whose host cost would
-    // otherwise exceed a small tensor's GPU work).  A build reads the device's
-    // done flag after each batch but the last and stops there once it is set
-    // (rounds past the last rule find the grammar done and return at once).
-    // While ckr_profile_begin is in effect the kernels are launched one by one.
-    for (uint32_t r = 0; r < R.rounds; r += kRoundBatch) {
+    // otherwise exceed a small tensor's GPU work).  While ckr_profile_begin is
+    // in effect the kernels are launched one by one.
+    //
+    // A build reads the device's state after a batch: it stops once the grammar
+    // is done (rounds past the last rule return at once), and else goes on from
+    // the round that the device has reached.  A lean batch is one full round
+    // and lean ones: without the counting and the tie-break, whose three
+    // launches take 5.9 us and return at once in nearly every round of a large
+    // tensor (50 rules of 4 Mi bf16 words built and applied to as many: 2948 to
+    // 2784 us).  A lean round that needs a recount or meets a tie does nothing, nor
+    // do those after it, and the next batch's full round takes it up; after the
+    // k-th such stop the next 16 << k rounds are full ones, so that a tensor
+    // whose rounds tie (few words, or many that are all rare) loses at most the
+    // rest of one batch, whose launches return at once, now and then.
+    auto launch = [&](uint32_t n_rounds, uint32_t full) -> hipError_t {
+        hipGraphExec_t gx = ckr::profiling() ? nullptr : round_graph(A, L, n_rounds, full, batch);
+        return gx ? hipGraphLaunch(gx, s) : batch(s, n_rounds, full);
+    };
+    if (!A.build) {
+        for (uint32_t r = 0; r < R.rounds; r += kRoundBatch)
+            if ((e = launch(std::min(kRoundBatch, R.rounds - r), 0)) != hipSuccess) return e;
+    }
+    uint32_t full_until = A.recount_each_round ? R.rounds : 0, stops = 0;
+    for (uint32_t r = 0; A.build && r < R.rounds;) {
         const uint32_t n_rounds = std::min(kRoundBatch, R.rounds - r);
-        hipGraphExec_t gx = ckr::profiling() ? nullptr : round_graph(A, L, n_rounds, batch);
-        if ((e = gx ? hipGraphLaunch(gx, s) : batch(s, n_rounds)) != hipSuccess) return e;
-        if (!A.build || r + kRoundBatch >= R.rounds) continue;
-        uint32_t done = 0;
-        if ((e = hipMemcpyAsync(&done, &ctl->done, 4, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+        const uint32_t full = r < full_until ? n_rounds : 1;
+        if ((e = launch(n_rounds, full)) != hipSuccess) return e;
+        if (full == n_rounds && r + n_rounds >= R.rounds) break;  // no round of it can have been left out
+        RepairCtl now{};
+        if ((e = hipMemcpyAsync(&now, ctl, sizeof(now), hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
         if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
-        if (done) break;
+        if (now.done || now.err || now.round <= r) break;
+        if (now.round < r + n_rounds) full_until = now.round + (16u << std::min(stops++, 10u));
+        r = now.round;
     }
     // the live tokens counted per block and scanned: the output's offsets, and
     // (apply, whose rounds keep no running count) the compressed length
