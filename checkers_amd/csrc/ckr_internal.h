@@ -350,10 +350,10 @@ struct RepairCtl {
     uint32_t n_cur, occ, done, round;  // live tokens; occurrences found this round
     uint32_t best, ncand, chosen, d;   // d: occupied pair-table slots
     uint32_t a0, a, b, c;              // alphabet size; pair (a, b) → c of this round
-    uint32_t skip, tie, err, max_pair; // tie: several pairs hold the top count
+    uint32_t tie, err, max_pair;       // tie: several pairs hold the top count
     uint32_t recount, recount_next;    // build: count every pair this round / the next
     uint32_t run_mode;                 // a == b: occurrences depend on the run parity
-    uint32_t pad[4];
+    uint32_t pad[5];
 };
 constexpr uint32_t kRepairMaxPrimes = 512;
 // Token ids of the repair sequence lie below these; the values from here up

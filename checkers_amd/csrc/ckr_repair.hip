@@ -26,8 +26,8 @@
 // other array for spans under LMAX).  Positions are monotone in the compacted
 // sequence, so first occurrences compare as the reference's do.
 //
-// Rounds run on the device with no host synchronisation inside a batch of
-// eight (one replay of a captured graph).  A build round is seven launches (a
+// A build's rounds run on the device with no host synchronisation inside a batch
+// of eight (one replay of a captured graph).  A build round is seven launches (a
 // full round) or the last four of them (a lean one, for rounds that need
 // neither a recount nor a tie-break; run_rounds says which when), each returning
 // at once when its case does not arise:
@@ -56,11 +56,10 @@
 //                    number, the table emptied before a recount) and the next
 //                    pair selected from the kept counts, committed when no tie
 //                    needs rp_pairs<FIRST>.
-// An apply round is rp_runs and rp_find alone: the rules are known, so each
-// kernel reads its rule (the batch's base round in ctl plus the round's place
-// in the batch), and rp_find replaces each occurrence as it finds it (see
-// rp_find for why that is safe when no counts are kept); the live count is
-// taken once at the end.
+// An apply round is rp_find alone, behind rp_runs if its rule is of a pair (x, x):
+// the rules are known, so each kernel is told its rule, and rp_find replaces
+// each occurrence as it finds it (see rp_find for why that is safe when no
+// counts are kept); the live count is taken once at the end.
 // Selection: the largest count and the number of pairs holding it; a unique
 // holder is the rule.  Ties: libstdc++ keeps one singly linked list; a node
 // for an empty bucket goes to the list head, a node for a used bucket goes to
@@ -219,14 +218,24 @@ __global__ void __launch_bounds__(RT) alpha_mark_direct(const uint8_t* __restric
     __shared__ uint32_t bm[2048];
     for (int j = threadIdx.x; j < 2048; j += RT) bm[j] = 0;
     __syncthreads();
-    for (uint64_t i = (uint64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (uint64_t)gridDim.x * RT) {
-        const uint32_t v = load_word<ES>(words, i) >> k;
-        const uint32_t bit = 1u << (v & 31);
-        if (!(bm[v >> 5] & bit)) atomicOr(&bm[v >> 5], bit);
+    constexpr int U = 8;  // words loaded together
+    const uint64_t step = (uint64_t)gridDim.x * RT;
+    for (uint64_t i = (uint64_t)blockIdx.x * RT + threadIdx.x; i < n; i += U * step) {
+        uint32_t v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = load_word<ES>(words, i + u * step < n ? i + u * step : i) >> k;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t bit = 1u << (v[u] & 31);
+            if (!(bm[v[u] >> 5] & bit)) atomicOr(&bm[v[u] >> 5], bit);
+        }
     }
     __syncthreads();
+    // (a bit that is there already needs no atomic: most workgroups see the
+    // same words, and their atomics on the same few lines took longer than the
+    // read of the tensor: 28.3 to 11.0 us on 4 Mi bf16 words)
     for (int j = threadIdx.x; j < 2048; j += RT)
-        if (bm[j]) atomicOr(&bitmap[j], bm[j]);
+        if (bm[j] & ~(bm[j] ? ld_relaxed32(&bitmap[j]) : 0u)) atomicOr(&bitmap[j], bm[j]);
 }
 
 // Ranks: rank[v] for the 2^w values (NONE if absent), sym[rank] = v << k.
@@ -237,14 +246,16 @@ __global__ void __launch_bounds__(SCAN_T) alpha_rank_direct(const uint32_t* __re
     const uint32_t t = threadIdx.x;
     const uint32_t b0 = bitmap[2 * t], b1 = bitmap[2 * t + 1];
     uint32_t total;
-    uint32_t base = block_excl_scan(__popc(b0) + __popc(b1), sh, &total);
-    const uint32_t nv = 1u << w;
-    for (uint32_t j = 0; j < 64; j++) {
-        const uint32_t v = 64 * t + j;
-        if (v >= nv) break;
-        const bool present = ((j < 32 ? b0 : b1) >> (j & 31)) & 1u;
-        if (present) { rank[v] = base; sym[base] = (uint64_t)v << k; base++; }
-        else rank[v] = NONE;
+    const uint32_t base = block_excl_scan(__popc(b0) + __popc(b1), sh, &total);
+    __shared__ uint32_t bits[2048], below[2048];  // a word's bits, and the values present before it
+    bits[2 * t] = b0; bits[2 * t + 1] = b1;
+    below[2 * t] = base; below[2 * t + 1] = base + __popc(b0);
+    __syncthreads();
+    for (uint32_t v = t; v < 1u << w; v += SCAN_T) {
+        const uint32_t m = bits[v >> 5], r = below[v >> 5] + __popc(m & ((1u << (v & 31)) - 1u));
+        const bool present = (m >> (v & 31)) & 1u;
+        rank[v] = present ? r : NONE;
+        if (present) sym[r] = (uint64_t)v << k;
     }
     if (t == 0) ctl->a0 = total;
 }
@@ -534,40 +545,47 @@ struct RoundArgs {
     int build;
 };
 
-// Build: record the round's rule (or stop: best count < 2).  Thread 0 only.
-__device__ void commit_rule(RepairCtl* ctl, const RoundArgs& A) {
-    const uint32_t r = ctl->round;
-    const uint32_t best = ctl->best;
+// Build: record the round's rule (or stop: best count < 2), from the state that
+// the caller has in registers.  Thread 0 only.
+struct CommitIn {
+    uint32_t round, n_cur, d, max_pair, a0;  // as in ctl
+    uint32_t best, chosen;                   // the top count, and the slot that holds it
+};
+__device__ __forceinline__ CommitIn commit_in(const RepairCtl& c, uint32_t best, uint32_t chosen) {
+    return CommitIn{c.round, c.n_cur, c.d, c.max_pair, c.a0, best, chosen};
+}
+__device__ void commit_rule(RepairCtl* ctl, const RoundArgs& A, const CommitIn& in) {
+    const uint32_t r = in.round;
+    const uint32_t best = in.best;
     if (r >= A.rounds) { ctl->done = 1; return; }  // the last rule is built: no round r is counted
-    if (best > ctl->max_pair) ctl->max_pair = best;
-    if (ctl->n_cur < 2 || best < 2) { ctl->done = 1; return; }
-    const uint64_t key = A.tab.key[ctl->chosen];
-    const uint32_t a = (uint32_t)(key >> 32), b = (uint32_t)key, c = ctl->a0 + r;
+    if (best > in.max_pair) ctl->max_pair = best;
+    if (in.n_cur < 2 || best < 2) { ctl->done = 1; return; }
+    const uint64_t key = A.tab.key[in.chosen];
+    const uint32_t a = (uint32_t)(key >> 32), b = (uint32_t)key, c = in.a0 + r;
+    const uint64_t lhs = A.sym[a], rhs = A.sym[b];
     const uint64_t rs = (1ull << 63) + r;
     A.rules[r].replacement = rs;
-    A.rules[r].lhs = A.sym[a];
-    A.rules[r].rhs = A.sym[b];
+    A.rules[r].lhs = lhs;
+    A.rules[r].rhs = rhs;
     A.rules[r].frequency = best;
     A.sym[c] = rs;
-    ctl->a = a; ctl->b = b; ctl->c = c; ctl->skip = 0; ctl->tie = 0;
+    ctl->a = a; ctl->b = b; ctl->c = c; ctl->tie = 0;
     ctl->run_mode = a == b ? 1u : 0u;
     // the round's new pairs are (x, c) and (c, x): at most 2 per occurrence
     // of c and 2 per symbol x (the a0 + r + 1 ids so far), plus (c, c)
-    const uint64_t fresh = 2ull * min((uint64_t)best, (uint64_t)ctl->a0 + r + 1u) + 1u;
+    const uint64_t fresh = 2ull * min((uint64_t)best, (uint64_t)in.a0 + r + 1u) + 1u;
     ctl->recount = 0;
-    ctl->recount_next = (uint64_t)ctl->d + fresh > A.dlimit ? 1u : 0u;
-    A.tab.cnt[ctl->chosen] = 0;
+    ctl->recount_next = (uint64_t)in.d + fresh > A.dlimit ? 1u : 0u;
+    A.tab.cnt[in.chosen] = 0;
 }
 
 // The pair of the round a grid kernel works on.  Build: the one committed in
 // ctl (by rp_close or the tie-break); none while a recount or a tie is pending
-// (a lean round, whose launches leave the sequence as it is).  Apply: rule ctl->round + ri of the
-// mapped rules, ri being the round's place in its batch (ctl->round moves once
-// per batch), so that apply rounds need no closing launch.
+// (a lean round, whose launches leave the sequence as it is).  Apply: rule ri of
+// the mapped rules, so that apply rounds need no closing launch.
 struct RoundSel {
     const uint32_t* rmap;  // apply: (a, b, c) per rule; null in build
-    uint32_t rounds;       // apply: rule count
-    uint32_t ri;           // apply: the round's index within its batch
+    uint32_t ri;           // apply: the rule
 };
 struct Cur {
     uint32_t a, b, c;
@@ -576,18 +594,13 @@ struct Cur {
 __device__ __forceinline__ Cur cur_round(const RepairCtl* ctl, const RoundSel& rs) {
     Cur x;
     if (!rs.rmap) {
-        x.live = !ctl->done && !ctl->skip && !ctl->recount && !ctl->tie;
+        x.live = !ctl->done && !ctl->recount && !ctl->tie;
         x.a = ctl->a; x.b = ctl->b; x.c = ctl->c;
         x.run = ctl->run_mode != 0;
         return x;
     }
-    const uint32_t r = ctl->round + rs.ri;
-    x.live = r < rs.rounds;
-    x.a = x.b = x.c = NONE;
-    if (x.live) {
-        x.a = rs.rmap[3 * r]; x.b = rs.rmap[3 * r + 1]; x.c = rs.rmap[3 * r + 2];
-        x.live = x.a != NONE && x.b != NONE;
-    }
+    x.a = rs.rmap[3 * rs.ri]; x.b = rs.rmap[3 * rs.ri + 1]; x.c = rs.rmap[3 * rs.ri + 2];
+    x.live = x.a != NONE && x.b != NONE;
     x.run = x.a == x.b;
     return x;
 }
@@ -604,23 +617,29 @@ __device__ __forceinline__ TopCount top_combine(TopCount x, TopCount y) {
     if (y.best == x.best) x.n += y.n;
     return x;
 }
-__device__ TopCount table_top(RepairCtl* ctl, const PairTab& t) {
+// The thread's first TOP_U slots come from the caller (top_slots), which loads
+// them together with d: the table has 4096 entries or more, so the read needs no
+// bound, and slots from d on are left alone.
+constexpr int TOP_U = 4;
+__device__ __forceinline__ void top_slots(const PairTab& t, uint32_t (&sl)[TOP_U]) {
+#pragma unroll
+    for (int i = 0; i < TOP_U; i++) sl[i] = t.touched[threadIdx.x + i * blockDim.x];
+}
+__device__ TopCount table_top(uint32_t d, const PairTab& t, uint32_t (&sl)[TOP_U]) {
     __shared__ TopCount sw[16];
-    const uint32_t d = ld_relaxed32(&ctl->d), bs = blockDim.x;
+    const uint32_t bs = blockDim.x;
     TopCount r{0, 0, 0};
-    uint32_t j = threadIdx.x;
-    for (; j + 3 * bs < d; j += 4 * bs) {
-        uint32_t sl[4], v[4];
+    for (uint32_t j = threadIdx.x; j < d;) {
+        uint32_t v[TOP_U];
 #pragma unroll
-        for (int i = 0; i < 4; i++) sl[i] = t.touched[j + i * bs];
+        for (int i = 0; i < TOP_U; i++) v[i] = j + i * bs < d ? ld_relaxed32(&t.cnt[sl[i]]) : 0u;
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = ld_relaxed32(&t.cnt[sl[i]]);
+        for (int i = 0; i < TOP_U; i++)
+            if (j + i * bs < d) r = top_combine(r, TopCount{v[i], 1, sl[i]});
+        j += TOP_U * bs;
 #pragma unroll
-        for (int i = 0; i < 4; i++) r = top_combine(r, TopCount{v[i], 1, sl[i]});
-    }
-    for (; j < d; j += bs) {
-        const uint32_t sl = t.touched[j];
-        r = top_combine(r, TopCount{ld_relaxed32(&t.cnt[sl]), 1, sl});
+        for (int i = 0; i < TOP_U; i++)
+            if (j + i * bs < d) sl[i] = t.touched[j + i * bs];
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -641,16 +660,19 @@ __device__ TopCount table_top(RepairCtl* ctl, const PairTab& t) {
 
 // Build: the largest count and its holders over the table's used slots; a
 // unique holder (or none worth a rule) commits, several set up the tie-break
-// (their first occurrences are taken by rp_pairs<FIRST>).
-__device__ void select_round(RepairCtl* ctl, const RoundArgs& A) {
-    const TopCount top = table_top(ctl, A.tab);
+// (their first occurrences are taken by rp_pairs<FIRST>).  `in` is the state in
+// registers, its top count yet to be found.
+__device__ void select_round(RepairCtl* ctl, const RoundArgs& A, CommitIn in, uint32_t (&sl)[TOP_U]) {
+    const TopCount top = table_top(in.d, A.tab, sl);
     const uint32_t ncand = top.best >= 2 ? top.n : 0u;
     if (threadIdx.x == 0) {
         ctl->best = top.best;
         ctl->ncand = ncand;
         ctl->chosen = top.slot;
-        if (top.best >= 2 && ncand > 1 && ctl->n_cur >= 2) ctl->tie = 1;  // first[] is NONE outside a tie
-        else commit_rule(ctl, A);
+        in.best = top.best;
+        in.chosen = top.slot;
+        if (top.best >= 2 && ncand > 1 && in.n_cur >= 2) ctl->tie = 1;  // first[] is NONE outside a tie
+        else commit_rule(ctl, A, in);
     }
     __syncthreads();
 }
@@ -692,7 +714,7 @@ __device__ void break_tie(RepairCtl* ctl, const RoundArgs& A) {
     __syncthreads();
     if (threadIdx.x == 0) {
         ctl->chosen = s_chosen;
-        commit_rule(ctl, A);
+        commit_rule(ctl, A, commit_in(*ctl, best, s_chosen));
     }
     __syncthreads();
 }
@@ -701,7 +723,9 @@ __device__ void break_tie(RepairCtl* ctl, const RoundArgs& A) {
 // selection's question, asked by every workgroup of rp_pairs<FIRST> in a
 // recount round (all get the same answer from the same counts).
 __device__ bool table_tied(RepairCtl* ctl, const PairTab& t) {
-    const TopCount top = table_top(ctl, t);
+    uint32_t sl[TOP_U];
+    top_slots(t, sl);
+    const TopCount top = table_top(ld_relaxed32(&ctl->d), t, sl);
     return top.best >= 2 && top.n > 1 && ctl->n_cur >= 2;
 }
 
@@ -756,7 +780,11 @@ __global__ void __launch_bounds__(RT) rp_pairs(const T* __restrict__ tok, const 
 // (committing a unique pair), then any tie broken and its pair committed.
 __global__ void __launch_bounds__(CLOSE_T) rp_tie(RepairCtl* ctl, RoundArgs A) {
     if (ctl->done) return;
-    if (ctl->recount) select_round(ctl, A);
+    if (ctl->recount) {
+        uint32_t sl[TOP_U];
+        top_slots(A.tab, sl);
+        select_round(ctl, A, commit_in(*ctl, 0, 0), sl);
+    }
     if (ctl->done || !ctl->tie) return;
     break_tie(ctl, A);
 }
@@ -943,9 +971,14 @@ __global__ void __launch_bounds__(RT) rp_find(T* tok, uint32_t* len, uint32_t* b
                                               uint32_t* __restrict__ ucount, uint32_t* __restrict__ lp,
                                               uint32_t* __restrict__ lq, uint32_t* __restrict__ le, uint32_t nids,
                                               uint32_t* __restrict__ hist, RoundSel rs) {
+    const Unit un = unit_of(N, K);
+    const uint32_t lane = threadIdx.x & 63;
+    Win<T> wn;  // the next chunk's window, loaded while this one is worked on (the first, while ctl is read)
+    if (un.c0 < un.c1) wn.load(tok, N, un.c0 * CHUNK + lane * SEG);
     const Cur cr = cur_round(ctl, rs);
     if (!cr.live) return;
-    // count changes: with ids below nids <= HV, two histograms over the ids
+    // count changes: with ids below nids <= HV, two histograms over the ids of
+    // the sequence, which lie below this round's c
     // (hl[t]: occurrences whose left neighbour t loses (t, a) and gains (t, c);
     // hr[t]: right neighbour t, (b, t) to (c, t)) and three counters for the
     // pairs of the run and overlap cases (hs: (c, c), (b, a) to (c, c), (c, a));
@@ -963,7 +996,7 @@ __global__ void __launch_bounds__(RT) rp_find(T* tok, uint32_t* len, uint32_t* b
     const bool direct = nids <= HV;
     if (count) {
         if (direct) {
-            for (uint32_t j = threadIdx.x; j < nids; j += RT) { hl[j] = 0; hr[j] = 0; }
+            for (uint32_t j = threadIdx.x; j < c; j += RT) { hl[j] = 0; hr[j] = 0; }
             if (threadIdx.x < 3) hs[threadIdx.x] = 0;
             __syncthreads();
         } else {
@@ -983,8 +1016,6 @@ __global__ void __launch_bounds__(RT) rp_find(T* tok, uint32_t* len, uint32_t* b
     auto cc = [&]() { if (direct) atomicAdd(&hs[0], 1u); else upd(c, c, 1u); };
     auto ba = [&]() { if (direct) atomicAdd(&hs[1], 1u); else { upd(b, a, DEC); upd(c, c, 1u); } };
     auto ca = [&]() { if (direct) atomicAdd(&hs[2], 1u); else upd(c, a, 1u); };
-    const Unit un = unit_of(N, K);
-    const uint32_t lane = threadIdx.x & 63;
     const uint64_t base = (uint64_t)un.u * K * (CHUNK / 2);  // the unit's slots: at most CHUNK / 2 per chunk
     uint32_t wcount = 0;                                      // slots used (uniform over the wave)
     uint32_t qw = 0;                                          // state entering the chunk
@@ -1008,8 +1039,6 @@ __global__ void __launch_bounds__(RT) rp_find(T* tok, uint32_t* len, uint32_t* b
         qw = all & 1;
         for (uint32_t v = u0; v < un.u; v++) qw = (rstate[v] >> qw) & 1;
     }
-    Win<T> wn;  // the next chunk's window, loaded while this one is worked on
-    if (un.c0 < un.c1) wn.load(tok, N, un.c0 * CHUNK + lane * SEG);
     for (uint32_t ch = un.c0; ch < un.c1; ch++) {
         const uint32_t i0 = ch * CHUNK + lane * SEG;
         const Win<T> w = wn;
@@ -1144,18 +1173,18 @@ __global__ void __launch_bounds__(RT) rp_find(T* tok, uint32_t* len, uint32_t* b
     // the histograms as this workgroup's row (hl | hr | hs), summed over the
     // workgroups and added to the table by rp_write
     __syncthreads();
-    uint32_t* row = hist + (uint64_t)blockIdx.x * (2 * nids + 3);
-    for (uint32_t j = threadIdx.x; j < nids; j += RT) {
+    uint32_t* row = hist + (uint64_t)blockIdx.x * (2 * c + 3);
+    for (uint32_t j = threadIdx.x; j < c; j += RT) {
         row[j] = hl[j];
-        row[nids + j] = hr[j];
+        row[c + j] = hr[j];
     }
-    if (threadIdx.x < 3) row[2 * nids + threadIdx.x] = hs[threadIdx.x];
+    if (threadIdx.x < 3) row[2 * c + threadIdx.x] = hs[threadIdx.x];
 }
 
 // The round's occurrences replaced in place (no two share a position): each
 // wave writes its unit's, whose positions lie in the unit's chunks.  Build
 // rounds that keep counts with ids below HV (merge): the count-change rows that
-// rp_find left (one per workgroup: hl | hr | hs) are summed in tiles of 256
+// rp_find left (one per workgroup: hl | hr | hs, 2 c + 3 entries) are summed in tiles of 256
 // columns x a group of rows, and each tile's sums go to the table, so each
 // pair takes one add per row group rather than one per workgroup.
 template <typename T>
@@ -1163,23 +1192,26 @@ __global__ void __launch_bounds__(RT) rp_write(T* __restrict__ tok, uint32_t* __
                                                uint32_t* __restrict__ back, uint32_t N, uint32_t K, RepairCtl* ctl,
                                                const uint32_t* __restrict__ ucount, const uint32_t* __restrict__ lp,
                                                const uint32_t* __restrict__ lq, const uint32_t* __restrict__ le,
-                                               const uint32_t* __restrict__ hist, uint32_t nids, uint32_t nrows,
-                                               PairTab tab, int merge, RoundSel rs) {
-    const Cur cr = cur_round(ctl, rs);
-    if (!cr.live) return;
-    const T c = (T)cr.c;
+                                               const uint32_t* __restrict__ hist, uint32_t nrows, PairTab tab,
+                                               int merge, RoundSel rs) {
     const Unit un = unit_of(N, K);
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t base = (uint64_t)un.u * K * (CHUNK / 2);
+    // the first 64 entries are loaded with the count and ctl rather than after
+    // them (a unit's part of the list has CHUNK / 2 or more); with that and the
+    // shorter count rows 8.5 to 7.1 us on 4 Mi bf16 words
     const uint32_t m = ucount[un.u];
-    for (uint32_t k = lane; k < m; k += 64) {
-        const uint32_t p = lp[base + k], q = lq[base + k], e = le[base + k];
-        if (p >= q || q >= e || e > N) continue;  // (never: p < q < e <= N)
-        merge_span<T>(tok, len, back, p, q, e, c);
+    uint32_t p = lp[base + lane], q = lq[base + lane], e = le[base + lane];
+    const Cur cr = cur_round(ctl, rs);
+    if (!cr.live) return;
+    const uint32_t a = cr.a, b = cr.b, c = cr.c;
+    for (uint32_t k = lane; k < m;) {
+        if (p < q && q < e && e <= N) merge_span<T>(tok, len, back, p, q, e, (T)c);  // (always: p < q < e <= N)
+        k += 64;
+        if (k < m) { p = lp[base + k]; q = lq[base + k]; e = le[base + k]; }
     }
     if (!merge || ctl->recount_next) return;
-    const uint32_t a = cr.a, b = cr.b;
-    const uint32_t rowlen = 2 * nids + 3, ncb = (rowlen + RT - 1) / RT;
+    const uint32_t rowlen = 2 * c + 3, ncb = (rowlen + RT - 1) / RT;
     const uint32_t ngrp = min(MERGE_RG, nrows), rpt = (nrows + ngrp - 1) / ngrp;
     const uint32_t ntiles = ncb * ngrp;  // tiles of RT columns x rpt rows
     // a workgroup takes up to four tiles at a time (when there are more tiles
@@ -1195,21 +1227,25 @@ __global__ void __launch_bounds__(RT) rp_write(T* __restrict__ tok, uint32_t* __
             uint32_t sum = 0;
             if (col < rowlen) {
                 uint32_t r = r0;
-                for (; r + 4 <= r1; r += 4) {
+                for (; r + 8 <= r1; r += 8) {
                     const uint32_t* h = hist + (uint64_t)r * rowlen + col;
-                    sum += h[0] + h[rowlen] + h[2 * rowlen] + h[3 * rowlen];
+                    uint32_t x[8];
+#pragma unroll
+                    for (int y = 0; y < 8; y++) x[y] = h[y * rowlen];
+#pragma unroll
+                    for (int y = 0; y < 8; y++) sum += x[y];
                 }
                 for (; r < r1; r++) sum += hist[(uint64_t)r * rowlen + col];
             }
             uint64_t k0 = 0, k1 = 0;
             uint32_t v0 = 0u - sum, v1 = sum;
-            if (col < nids) {                       // left neighbour col: (col, a) to (col, c)
+            if (col < c) {                       // left neighbour col: (col, a) to (col, c)
                 k0 = pair_key(col, a); k1 = pair_key(col, c);
-            } else if (col < 2 * nids) {            // right neighbour: (b, t) to (c, t)
-                k0 = pair_key(b, col - nids); k1 = pair_key(c, col - nids);
-            } else if (col == 2 * nids) {           // (c, c) made by runs
+            } else if (col < 2 * c) {            // right neighbour: (b, t) to (c, t)
+                k0 = pair_key(b, col - c); k1 = pair_key(c, col - c);
+            } else if (col == 2 * c) {           // (c, c) made by runs
                 k0 = k1 = pair_key(c, c); v0 = 0;
-            } else if (col == 2 * nids + 1) {       // (b, a) to (c, c)
+            } else if (col == 2 * c + 1) {       // (b, a) to (c, c)
                 k0 = pair_key(b, a); k1 = pair_key(c, c);
             } else {                                // (c, a) after an odd run
                 k0 = k1 = pair_key(c, a); v0 = 0;
@@ -1226,54 +1262,63 @@ __global__ void __launch_bounds__(RT) rp_write(T* __restrict__ tok, uint32_t* __
 // counts (committed when no tie needs rp_pairs<FIRST>).
 __global__ void __launch_bounds__(CLOSE_T) rp_close(uint32_t nb, RepairCtl* ctl, const uint32_t* __restrict__ bcount,
                                                     RoundArgs A) {
-    if (ctl->done || ctl->recount || ctl->tie) return;  // (pending: rp_pairs and rp_tie come first)
-    __shared__ uint32_t sh[16];
-    __shared__ uint32_t s_recount;
+    // one workgroup, so what it waits for is memory's latency, again and again:
+    // all that does not depend on another load is loaded at once, before the
+    // first of it is looked at (4 Mi bf16 words: 10.0 to 8.5 us)
+    const RepairCtl in = *ctl;
+    uint32_t sl[TOP_U];
+    top_slots(A.tab, sl);
     uint32_t occ = 0;
-    if (!ctl->skip) {
-        uint32_t j = threadIdx.x;
-        for (; j + 3 * CLOSE_T < nb; j += 4 * CLOSE_T)
-            occ += bcount[j] + bcount[j + CLOSE_T] + bcount[j + 2 * CLOSE_T] + bcount[j + 3 * CLOSE_T];
-        for (; j < nb; j += CLOSE_T) occ += bcount[j];
-    }
+    uint32_t j = threadIdx.x;
+    for (; j + 3 * CLOSE_T < nb; j += 4 * CLOSE_T)
+        occ += bcount[j] + bcount[j + CLOSE_T] + bcount[j + 2 * CLOSE_T] + bcount[j + 3 * CLOSE_T];
+    for (; j < nb; j += CLOSE_T) occ += bcount[j];
+    if (in.done || in.recount || in.tie) return;  // (pending: rp_pairs and rp_tie come first)
+    __shared__ uint32_t sh[16];
     uint32_t total;
     block_excl_scan(occ, sh, &total);
+    CommitIn next = commit_in(in, 0, 0);
+    next.n_cur -= total;
+    next.round++;
     if (threadIdx.x == 0) {
-        ctl->n_cur -= total;
-        ctl->round++;
-        ctl->best = 0; ctl->ncand = 0; ctl->pick = 0; ctl->skip = 0; ctl->tie = 0; ctl->run_mode = 0;
-        ctl->recount = ctl->recount_next;
+        ctl->n_cur = next.n_cur;
+        ctl->round = next.round;
+        ctl->best = 0; ctl->ncand = 0; ctl->pick = 0; ctl->run_mode = 0;
+        ctl->recount = in.recount_next;
         ctl->recount_next = 0;
-        s_recount = ctl->recount;
     }
-    __syncthreads();
-    if (s_recount) {  // rp_pairs fills the table again
-        const uint32_t d = ctl->d;
-        for (uint32_t j = threadIdx.x; j < d; j += blockDim.x) {
-            const uint32_t s = A.tab.touched[j];
+    if (in.recount_next) {  // rp_pairs fills the table again
+        for (uint32_t k = threadIdx.x; k < in.d; k += blockDim.x) {
+            const uint32_t s = A.tab.touched[k];
             A.tab.key[s] = EMPTY_KEY; A.tab.cnt[s] = 0; A.tab.first[s] = NONE;
         }
-        __syncthreads();
         if (threadIdx.x == 0) ctl->d = 0;
     } else {
-        select_round(ctl, A);
+        select_round(ctl, A, next, sl);
     }
 }
 
-// Apply, after a batch of rounds: the batch's rounds are done.
-__global__ void rp_batch_end(RepairCtl* ctl, uint32_t rounds) { ctl->round += rounds; }
-
 // ------------------------------------------------------------------ output
 // The live tokens as reference symbols, in order: per block of BLK positions
-// the live count, one scan, then the writes.
+// the live count, one scan, then the writes.  A thread's SEG tokens come in
+// 16-byte loads (the array is aligned, and carries 32 tombstones past its end).
+template <typename T>
+__device__ __forceinline__ uint32_t seg_live(const T* __restrict__ tok, uint32_t N, uint32_t i0, T (&t)[SEG]) {
+    uint32_t c = 0;
+    if (i0 >= N) return 0;
+    uint4* v = reinterpret_cast<uint4*>(t);
+#pragma unroll
+    for (int q = 0; q < (int)(SEG * sizeof(T) / 16); q++) v[q] = reinterpret_cast<const uint4*>(tok + i0)[q];
+#pragma unroll
+    for (int j = 0; j < SEG; j++) c += (i0 + j < N && t[j] < tb0<T>()) ? 1u : 0u;
+    return c;
+}
 template <typename T>
 __global__ void __launch_bounds__(RT) seq_count(const T* __restrict__ tok, uint32_t N, uint32_t* __restrict__ bcount) {
     __shared__ uint32_t sh[16];
-    const uint32_t i0 = blockIdx.x * BLK + threadIdx.x * SEG;
-    uint32_t c = 0;
-    for (int j = 0; j < SEG; j++) c += (i0 + j < N && tok[i0 + j] < tb0<T>()) ? 1u : 0u;
+    alignas(16) T t[SEG];
     uint32_t tot;
-    block_excl_scan(c, sh, &tot);
+    block_excl_scan(seg_live<T>(tok, N, blockIdx.x * BLK + threadIdx.x * SEG, t), sh, &tot);
     if (threadIdx.x == 0) bcount[blockIdx.x] = tot;
 }
 
@@ -1283,15 +1328,13 @@ __global__ void __launch_bounds__(RT) seq_write(const T* __restrict__ tok, uint3
                                                 uint64_t* __restrict__ out) {
     __shared__ uint32_t sh[16];
     const uint32_t i0 = blockIdx.x * BLK + threadIdx.x * SEG;
-    uint32_t c = 0;
-    for (int j = 0; j < SEG; j++) c += (i0 + j < N && tok[i0 + j] < tb0<T>()) ? 1u : 0u;
+    alignas(16) T t[SEG];
+    const uint32_t c = seg_live<T>(tok, N, i0, t);
     uint32_t tot;
     uint32_t o = bbase[blockIdx.x] + block_excl_scan(c, sh, &tot);
-    for (int j = 0; j < SEG; j++) {
-        if (i0 + j >= N) break;
-        const T t = tok[i0 + j];
-        if (t < tb0<T>()) out[o++] = sym[t];
-    }
+#pragma unroll
+    for (int j = 0; j < SEG; j++)
+        if (i0 + j < N && t[j] < tb0<T>()) out[o++] = sym[t[j]];
 }
 
 template <typename T>
@@ -1406,11 +1449,12 @@ hipError_t build_alphabet(const uint8_t* words, uint64_t n, int es, uint32_t k, 
     const uint32_t g = grid_for(n, 2048);
     if (L.direct) {
         uint32_t* bitmap = reinterpret_cast<uint32_t*>(P(L.o_bitmap));
+        const uint32_t gm = std::min(g, 512u);  // (each clears and hands on a bitmap of 8 KiB)
         uint32_t* rank = reinterpret_cast<uint32_t*>(P(L.o_rank));
         hipError_t e = fill<uint32_t>(bitmap, 2048, 0u, s);
         if (e != hipSuccess) return e;
-        if (es == 2) CKR_LAUNCH("repair_alpha_kernel", s, alpha_mark_direct<2><<<g, RT, 0, s>>>(words, n, k, bitmap));
-        else CKR_LAUNCH("repair_alpha_kernel", s, alpha_mark_direct<4><<<g, RT, 0, s>>>(words, n, k, bitmap));
+        if (es == 2) CKR_LAUNCH("repair_alpha_kernel", s, alpha_mark_direct<2><<<gm, RT, 0, s>>>(words, n, k, bitmap));
+        else CKR_LAUNCH("repair_alpha_kernel", s, alpha_mark_direct<4><<<gm, RT, 0, s>>>(words, n, k, bitmap));
         CKR_LAUNCH("repair_alpha_kernel", s, alpha_rank_direct<<<1, SCAN_T, 0, s>>>(bitmap, L.w, k, rank, sym, ctl));
         const uint32_t nv = 1u << L.w;
         const size_t lds = nv <= 16384 ? nv * 4 : 0;
@@ -1439,7 +1483,7 @@ hipError_t build_alphabet(const uint8_t* words, uint64_t n, int es, uint32_t k, 
 
 constexpr uint32_t kRoundBatch = 8;
 
-// The captured graphs of a batch of rounds (kRoundBatch, or the last batch's
+// The captured graphs of a batch of build rounds (kRoundBatch, or the last batch's
 // remainder), keyed by what their kernels' arguments derive from (the
 // workspace and its layout's inputs) and the batch length.  A graph is
 // captured on a library stream, instantiated once and kept; at most
@@ -1447,10 +1491,10 @@ constexpr uint32_t kRoundBatch = 8;
 struct RoundGraphKey {
     const void* ws;
     uint64_t n;
-    int es, build, device, tok16;
+    int es, device, tok16;
     uint32_t k, rounds, dlimit, batch, full;
     bool operator==(const RoundGraphKey& o) const {
-        return ws == o.ws && n == o.n && es == o.es && build == o.build && device == o.device && tok16 == o.tok16 &&
+        return ws == o.ws && n == o.n && es == o.es && device == o.device && tok16 == o.tok16 &&
                k == o.k && rounds == o.rounds && dlimit == o.dlimit && batch == o.batch && full == o.full;
     }
 };
@@ -1477,7 +1521,7 @@ template <typename BatchFn>
 hipGraphExec_t round_graph(const RepairArgs& A, const RepairLayout& L, uint32_t len, uint32_t full, BatchFn& batch) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    const RoundGraphKey key{A.ws, A.n, A.es, A.build, dev, L.tok16 ? 1 : 0, A.k, A.build ? A.max_rules : A.n_rules,
+    const RoundGraphKey key{A.ws, A.n, A.es, dev, L.tok16 ? 1 : 0, A.k, A.max_rules,
                             A.recount_each_round ? 1u : 0u, len, full};
     std::lock_guard<std::mutex> lk(g_rg_mu);
     for (const RoundGraph& r : g_rgs)
@@ -1574,46 +1618,48 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
                        L.vcap ? L.vcap - 1 : 0, reinterpret_cast<const uint32_t*>(P(L.o_vrank)), ctl,
                        const_cast<uint32_t*>(R.rmap), sym));
     }
-    // One round.  Build: every kernel reads what to do from ctl, so the rounds
-    // are identical launches; a lean one is without the counting and the
-    // tie-break.  Apply: the grid kernels take the round's place in its batch
-    // and read the rule themselves, rp_find writes in place; no write or
-    // closing launch.
-    auto round = [&](hipStream_t x, uint32_t ri, bool full) -> hipError_t {
-        const RoundSel rs{A.build ? nullptr : R.rmap, R.rounds, ri};
-        if (A.build && full) {
+    // One build round: every kernel reads what to do from ctl, so the rounds are
+    // identical launches; a lean one is without the counting and the tie-break.
+    auto round = [&](hipStream_t x, bool full) -> hipError_t {
+        const RoundSel rs{nullptr, 0};
+        if (full) {
             CKR_LAUNCH("repair_count_kernel", x, (rp_pairs<T, false><<<gpair, RT, 0, x>>>(tok, len, N, ctl, R, pchunk)));
             CKR_LAUNCH("repair_first_kernel", x, (rp_pairs<T, true><<<gpair, RT, 0, x>>>(tok, len, N, ctl, R, pchunk)));
             CKR_LAUNCH("repair_select_kernel", x, rp_tie<<<1, CLOSE_T, 0, x>>>(ctl, R));
         }
         CKR_LAUNCH("repair_runs_kernel", x, rp_runs<T><<<fg.G, RT, 0, x>>>(tok, len, N, fg.K, ctl, bfun, rs));
-        if (A.build)
-            CKR_LAUNCH("repair_find_kernel", x,
-                       (rp_find<T, true><<<fg.G, RT, 0, x>>>(tok, len, back, N, fg.K, ctl, R.tab, bfun, bcount, lp, lq,
-                                                              le, nids, hist, rs)));
-        else
-            CKR_LAUNCH("repair_find_kernel", x,
-                       (rp_find<T, false><<<fg.G, RT, 0, x>>>(tok, len, back, N, fg.K, ctl, R.tab, bfun, bcount, lp,
-                                                               lq, le, nids, hist, rs)));
-        if (A.build) {
-            CKR_LAUNCH("repair_write_kernel", x,
-                       rp_write<T><<<fg.G, RT, 0, x>>>(tok, len, back, N, fg.K, ctl, bcount, lp, lq, le, hist, nids,
-                                                       fg.G, R.tab, merge, rs));
-            CKR_LAUNCH("repair_close_kernel", x, rp_close<<<1, CLOSE_T, 0, x>>>(fg.U, ctl, bcount, R));
-        }
+        CKR_LAUNCH("repair_find_kernel", x,
+                   (rp_find<T, true><<<fg.G, RT, 0, x>>>(tok, len, back, N, fg.K, ctl, R.tab, bfun, bcount, lp, lq,
+                                                          le, nids, hist, rs)));
+        CKR_LAUNCH("repair_write_kernel", x,
+                   rp_write<T><<<fg.G, RT, 0, x>>>(tok, len, back, N, fg.K, ctl, bcount, lp, lq, le, hist, fg.G, R.tab,
+                                                   merge, rs));
+        CKR_LAUNCH("repair_close_kernel", x, rp_close<<<1, CLOSE_T, 0, x>>>(fg.U, ctl, bcount, R));
         return hipGetLastError();
     };
     // `full` rounds of n_rounds, the first ones, are full.
     auto batch = [&](hipStream_t x, uint32_t n_rounds, uint32_t full) -> hipError_t {
         for (uint32_t i = 0; i < n_rounds; i++) {
-            const hipError_t er = round(x, i, i < full);
+            const hipError_t er = round(x, i < full);
             if (er != hipSuccess) return er;
         }
-        if (!A.build) CKR_LAUNCH("repair_close_kernel", x, rp_batch_end<<<1, 1, 0, x>>>(ctl, n_rounds));
-        return hipGetLastError();
+        return hipSuccess;
     };
-    // Rounds go in batches of kRoundBatch (the last one shorter), each batch
-    // one launch of a graph captured once per workspace, shape and batch
+    // An apply's rounds take the rule as an argument and write in place: one
+    // launch a rule, and the run parity ahead of it for the rules (x, x), which
+    // the host can tell (rp_runs returned at once in the others, 3.9 us each).
+    // A launch costs the host less than rp_find takes, so there is no graph.
+    for (uint32_t r = 0; !A.build && r < R.rounds; r++) {
+        const RoundSel rs{R.rmap, r};
+        if (A.h_rules[r].lhs == A.h_rules[r].rhs)
+            CKR_LAUNCH("repair_runs_kernel", s, rp_runs<T><<<fg.G, RT, 0, s>>>(tok, len, N, fg.K, ctl, bfun, rs));
+        CKR_LAUNCH("repair_find_kernel", s,
+                   (rp_find<T, false><<<fg.G, RT, 0, s>>>(tok, len, back, N, fg.K, ctl, R.tab, bfun, bcount, lp, lq, le,
+                                                           nids, hist, rs)));
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    // A build's rounds go in batches of kRoundBatch (the last one shorter), each
+    // batch one launch of a graph captured once per workspace, shape and batch
     // length and kept (a round is up to 7 launches, whose host cost would
     // otherwise exceed a small tensor's GPU work).  While ckr_profile_begin is
     // in effect the kernels are launched one by one.
@@ -1633,10 +1679,6 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
         hipGraphExec_t gx = ckr::profiling() ? nullptr : round_graph(A, L, n_rounds, full, batch);
         return gx ? hipGraphLaunch(gx, s) : batch(s, n_rounds, full);
     };
-    if (!A.build) {
-        for (uint32_t r = 0; r < R.rounds; r += kRoundBatch)
-            if ((e = launch(std::min(kRoundBatch, R.rounds - r), 0)) != hipSuccess) return e;
-    }
     uint32_t full_until = A.recount_each_round ? R.rounds : 0, stops = 0;
     for (uint32_t r = 0; A.build && r < R.rounds;) {
         const uint32_t n_rounds = std::min(kRoundBatch, R.rounds - r);
