@@ -1206,7 +1206,7 @@ const void* canon_chains(hipStream_t s) {
 }
 
 // A tensor's encode with the table built on the device (tensors the fast
-// encoder takes: masked dtypes, units of at most 64 KiB): from its histograms
+// encoder takes: units of at most 64 KiB): from its histograms
 // in device memory, the table by ranks, encode entries, canonical streams and
 // slot sizes, and the encode are queued with no host round trip, and the
 // control words and the table are read back into pinned words.  After the

@@ -1271,9 +1271,9 @@ hipError_t launch_encode_batch(const uint8_t* src, const EncodeGeom& g, uint64_t
 }
 
 // ------------------------------------------------------------------ fast encode (LDS-staged, look-back)
-// Units of at most 64 KiB of masked dtypes, taken in order from a ticket
-// counter; one thread per 32-bit column, coding only the two live lanes of its
-// column (one coder wave per live plane).  Each live lane writes its stream backward into its
+// Units of at most 64 KiB, taken in order from a ticket counter; one thread per
+// 32-bit column and live lane of it (one coder wave per live plane: two of a
+// masked dtype, four of int8 and int32).  Each live lane writes its stream backward into its
 // own LDS slot, so that the stream ends up contiguous and in stream order; the
 // slot stride is chosen so that the 64 threads writing their e-th bytes hit
 // different banks.  The zero-plane lanes are the canonical streams.  When the

@@ -191,7 +191,7 @@ CKR_API int ckr_encode_planes(const void* d_src, uint64_t n_elems, int dtype,
 /* ---- full tensor compression as ANSCompressor::compress_tensor does it for a
  * singleton (histogram → table → encode), in one call.  The table built is
  * returned in h_table (may be NULL).  The workspace (16-byte aligned) as for
- * ckr_encode.  For tensors of masked dtypes with units of at most 64 KiB the
+ * ckr_encode.  For tensors with units of at most 64 KiB the
  * table is built on the device from the histogram in the same launch (the
  * reference's normalisation, by ranks; a table whose correction falls inside
  * a group of equal fractional parts is taken from the host's sort instead),
@@ -528,7 +528,8 @@ CKR_API int ckr_make_contiguous(const void* d_src, int ndim, const int64_t* shap
  * fast kernels — lanes of masked planes coded once per lane count (their
  * streams are identical), units of at most 64 KiB coded and decoded through
  * LDS; mode 0: every lane coded and decoded independently through global
- * memory; mode 2: fast kernels with minimal LDS lane slots, so that nearly
+ * memory (modes 1 to 3 take int8 and int32, which have no masked planes, the same way
+ * as the other dtypes); mode 2: fast kernels with minimal LDS lane slots, so that nearly
  * every unit takes the overflow route back through the general kernels; mode
  * 3: the same minimal slots, the overflowing units coded again by the fast
  * encoder with slots that hold any lane (mode 1's overflow route).  In
