@@ -353,7 +353,8 @@ struct RepairCtl {
     uint32_t tie, err, max_pair;       // tie: several pairs hold the top count
     uint32_t recount, recount_next;    // build: count every pair this round / the next
     uint32_t run_mode;                 // a == b: occurrences depend on the run parity
-    uint32_t pad[5];
+    uint32_t ties;                     // build: tie-breaks so far
+    uint32_t pad[4];
 };
 constexpr uint32_t kRepairMaxPrimes = 512;
 // Token ids of the repair sequence lie below these; the values from here up

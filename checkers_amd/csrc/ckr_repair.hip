@@ -629,17 +629,24 @@ __device__ TopCount table_top(uint32_t d, const PairTab& t, uint32_t (&sl)[TOP_U
     __shared__ TopCount sw[16];
     const uint32_t bs = blockDim.x;
     TopCount r{0, 0, 0};
-    for (uint32_t j = threadIdx.x; j < d;) {
-        uint32_t v[TOP_U];
+    // no load is behind a branch: past d slot 0 is read (one line for all), and
+    // not used; the next slots are on their way with this step's counts (a build
+    // that ends at its first selection, 1 Mi distinct pairs: 3455 us with guarded
+    // loads, 2823 so)
+    for (uint32_t j0 = 0; j0 < d; j0 += TOP_U * bs) {  // (the same steps for every thread)
+        const uint32_t j = j0 + threadIdx.x;
+        uint32_t v[TOP_U], nx[TOP_U] = {};
 #pragma unroll
-        for (int i = 0; i < TOP_U; i++) v[i] = j + i * bs < d ? ld_relaxed32(&t.cnt[sl[i]]) : 0u;
+        for (int i = 0; i < TOP_U; i++) v[i] = ld_relaxed32(&t.cnt[(uint64_t)j + i * bs < d ? sl[i] : 0u]);
+        if ((uint64_t)j0 + TOP_U * bs < d) {  // (a load past the last step would be waited for at the barrier)
 #pragma unroll
-        for (int i = 0; i < TOP_U; i++)
-            if (j + i * bs < d) r = top_combine(r, TopCount{v[i], 1, sl[i]});
-        j += TOP_U * bs;
+            for (int i = 0; i < TOP_U; i++) nx[i] = t.touched[min((uint64_t)j + (TOP_U + i) * bs, t.mask)];
+        }
 #pragma unroll
-        for (int i = 0; i < TOP_U; i++)
-            if (j + i * bs < d) sl[i] = t.touched[j + i * bs];
+        for (int i = 0; i < TOP_U; i++) {
+            if ((uint64_t)j + i * bs < d) r = top_combine(r, TopCount{v[i], 1, sl[i]});
+            sl[i] = nx[i];
+        }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -786,6 +793,7 @@ __global__ void __launch_bounds__(CLOSE_T) rp_tie(RepairCtl* ctl, RoundArgs A) {
         select_round(ctl, A, commit_in(*ctl, 0, 0), sl);
     }
     if (ctl->done || !ctl->tie) return;
+    if (threadIdx.x == 0) ctl->ties++;
     break_tie(ctl, A);
 }
 
@@ -1672,16 +1680,17 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
     // tensor (50 rules of 4 Mi bf16 words built and applied to as many: 2948 to
     // 2784 us).  A lean round that needs a recount or meets a tie does nothing, nor
     // do those after it, and the next batch's full round takes it up; after the
-    // k-th such stop the next 16 << k rounds are full ones, so that a tensor
-    // whose rounds tie (few words, or many that are all rare) loses at most the
-    // rest of one batch, whose launches return at once, now and then.
+    // k-th such stop the next 16 << k rounds are full ones.  Tensors whose
+    // rounds tie (few words, or many that are all rare) tie from the start: the
+    // first batch is two full rounds, and lean batches follow batches without a
+    // tie only.
     auto launch = [&](uint32_t n_rounds, uint32_t full) -> hipError_t {
         hipGraphExec_t gx = ckr::profiling() ? nullptr : round_graph(A, L, n_rounds, full, batch);
         return gx ? hipGraphLaunch(gx, s) : batch(s, n_rounds, full);
     };
-    uint32_t full_until = A.recount_each_round ? R.rounds : 0, stops = 0;
+    uint32_t full_until = A.recount_each_round ? R.rounds : 2, stops = 0, ties = 0;
     for (uint32_t r = 0; A.build && r < R.rounds;) {
-        const uint32_t n_rounds = std::min(kRoundBatch, R.rounds - r);
+        const uint32_t n_rounds = std::min(r == 0 ? 2u : kRoundBatch, R.rounds - r);
         const uint32_t full = r < full_until ? n_rounds : 1;
         if ((e = launch(n_rounds, full)) != hipSuccess) return e;
         if (full == n_rounds && r + n_rounds >= R.rounds) break;  // no round of it can have been left out
@@ -1690,6 +1699,8 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
         if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
         if (now.done || now.err || now.round <= r) break;
         if (now.round < r + n_rounds) full_until = now.round + (16u << std::min(stops++, 10u));
+        else if (now.ties != ties) full_until = std::max(full_until, now.round + kRoundBatch);
+        ties = now.ties;
         r = now.round;
     }
     // the live tokens counted per block and scanned: the output's offsets, and
