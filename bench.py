@@ -289,8 +289,8 @@ def reference_layout_leg(shard, ck, torch, dev):
                encode_GBps=round(nb / enc_ms / 1e6, 3), decode_GBps=round(nb / dec_ms / 1e6, 3),
                ans_ratio=round(nb / r.total, 4), roundtrip_bit_exact=ok,
                note="one unit: 256 lanes, each coding n/256 symbols in order; one thread per lane chain "
-                    "records its state every 1024 rows (lu_chain_kernel), then every segment is coded side "
-                    "by side (lu_code_kernel); the decode follows one chain per lane (decode_long_kernel). "
+                    "records its state every 256 rows (lu_chain_kernel), then every segment is coded side "
+                    "by side (lu_code_kernel); the decode follows one chain per lane (decode_chain_kernel). "
                     "The reference's own encode kernel runs 256 threads, one per lane")
     del e, r, d, dst
     torch.cuda.empty_cache()
