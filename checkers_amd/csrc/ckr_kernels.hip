@@ -1655,15 +1655,17 @@ __host__ __device__ constexpr uint32_t ws_region_bytes(uint32_t stride0, uint32_
     return (R_SLOTS + 32 * nc * stride0 + 32 * nc * stride1 + 15u) & ~15u;
 }
 __host__ __device__ constexpr uint32_t ws_lds_bytes(uint32_t pairs, uint32_t canon_bytes, uint32_t stride0,
-                                                    uint32_t stride1, uint32_t nc = 2) {
+                                                    uint32_t stride1, uint32_t nc = 2, uint32_t sets = 2) {
     return ws_ctl_offset(canon_bytes) + pairs * (uint32_t)sizeof(WsPairCtl) +
-           2 * pairs * ws_region_bytes(stride0, stride1, nc) + 32;
+           sets * pairs * ws_region_bytes(stride0, stride1, nc) + 32;
 }
 
 // LIST: the units a previous launch put on the redo list (ctl[1] of them in
 // redo_list) coded again with slots large enough for any lane (2 bytes per
 // row), at the offsets that launch published; tickets from ctl[3]; no sidecar,
 // no look-back.  A lane that outgrew even those slots would set ctl[2] bit 1.
+// 256 such slots (int8, int32) fill the LDS once, not twice: one slot set, coded
+// and packed in turn.
 // report (LIST): ctl[0 .. n_report) as they are at the launch, copied there first.
 template <int SPE, bool ESC, bool SIDE, int PAIRS, int NPK, bool LIST>
 __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src, EncodeGeom g,
@@ -1687,6 +1689,7 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
     extern __shared__ uint32_t lds[];
     uint8_t* lds8 = reinterpret_cast<uint8_t*>(lds);
     constexpr uint32_t NC = SPE == 0 ? 4 : 2;  // coder waves of a pair, one per live byte of a column
+    constexpr uint32_t SETS = SPE == 0 && LIST ? 1 : 2;  // slot sets of a pair, used in turn
     constexpr uint32_t NT = 64 * (NC + NPK) * PAIRS;
     const uint4* tab = reinterpret_cast<const uint4*>(lds8 + 0);
     uint32_t* chdr = reinterpret_cast<uint32_t*>(lds8 + FE_CHDR);
@@ -1739,9 +1742,9 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
     if (coder) {
         const uint32_t cb = SPE == 0 ? rl : (rl ? 3u : (uint32_t)FL);  // this wave's byte of the column
         for (uint32_t i = 0;; i++) {
-            const uint32_t s = i & 1;
+            const uint32_t s = i % SETS;
             const uint64_t t_wait = phase ? wall_clock64() : 0;
-            if (i >= 2) ws_wait_ge(&pc.freed[s], i >> 1);  // set s given back
+            if (i >= SETS) ws_wait_ge(&pc.freed[s], i / SETS);  // set s given back
             if (rl == 0) {
                 if (j == 0) {  // ticket
                     if (LIST) {
@@ -1764,7 +1767,7 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
             const uint64_t ubase = (uint64_t)u * g.unit;
             const uint32_t len = (uint32_t)((g.n_bytes - ubase < g.unit) ? (g.n_bytes - ubase) : g.unit);
             const uint8_t* usrc = src + ubase;
-            const uint32_t rb = reg0 + (2 * pr + s) * rbytes;
+            const uint32_t rb = reg0 + (SETS * pr + s) * rbytes;
             const uint32_t endw = slot_end(rb, rl);
             EncLane c{L, 0u, 0u, endw};
             const uint32_t K = len > col ? (len - col + 255) / 256 : 0u;
@@ -1825,15 +1828,15 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
         ws_wait_ge(&pc.pbar, bar);
     };
     for (uint32_t i = 0;; i++) {
-        const uint32_t s = i & 1;
-        ws_wait_ge(&pc.coded[s], NC * ((i >> 1) + 1));
+        const uint32_t s = i % SETS;
+        ws_wait_ge(&pc.coded[s], NC * (i / SETS + 1));
         const uint32_t u = __builtin_amdgcn_readfirstlane(ws_load(&pc.unit[s]));
         if (u >= g.n_units) break;
         const uint64_t t_seen = phase ? wall_clock64() : 0;
         const uint64_t ubase = (uint64_t)u * g.unit;
         const uint32_t len = (uint32_t)((g.n_bytes - ubase < g.unit) ? (g.n_bytes - ubase) : g.unit);
         const uint8_t* usrc = src + ubase;
-        const uint32_t rb = reg0 + (2 * pr + s) * rbytes;
+        const uint32_t rb = reg0 + (SETS * pr + s) * rbytes;
         uint2* lrec = reinterpret_cast<uint2*>(lds8 + rb + R_REC);  // per lane {LDS address of unit byte 0, lane end}
         static_assert(R_REC + 512 * NC <= R_SLOTS - 516, "exchange words below the guard of the lowest slot");
         uint8_t* bmap_w = lds8 + rb + R_MAP;                           // 64-byte block → lane (1025)
@@ -2216,17 +2219,20 @@ hipError_t launch_encode_fast_multi(const FastJob* jobs, uint32_t n, uint32_t ld
                               : run(encode_fast_multi_kernel<1, false, 1, ENC_NPK>, 64u * (2 + ENC_NPK)));
 }
 
-// The redo list of a launch_encode_fast launch (ctl[1] units, queued once the
-// host has seen that there are some): one coder pair per workgroup with slots
-// of 2 bytes per row (any lane fits), one workgroup per CU.
+// The redo list of a launch_encode_fast launch (ctl[1] units): one coder pair
+// (int8, int32: one unit's four coder waves and one slot set) per workgroup with
+// slots of 2 bytes per row (any lane fits), one workgroup per CU.
 static uint32_t encode_fast_list_slot(const EncodeGeom& g) {
     return (uint32_t)(2 * ((g.unit + 255) / 256) + 8 + 3) & ~3u;
 }
 
-bool encode_fast_list_fits(const FastEncParamsHost& hp, const EncodeGeom& g, uint32_t lds_limit) {
-    if (g.spe == 0) return false;  // 256 such slots, twice, never fit: the general kernels redo those units
+static uint32_t encode_fast_list_lds(const FastEncParamsHost& hp, const EncodeGeom& g) {
     const uint32_t st = slot_stride(encode_fast_list_slot(g));
-    return ws_lds_bytes(1, hp.canon_bytes, st, st) <= lds_limit;
+    return g.spe ? ws_lds_bytes(1, hp.canon_bytes, st, st) : ws_lds_bytes(1, hp.canon_bytes, st, st, 4, 1);
+}
+
+bool encode_fast_list_fits(const FastEncParamsHost& hp, const EncodeGeom& g, uint32_t lds_limit) {
+    return encode_fast_list_lds(hp, g) <= lds_limit;
 }
 
 hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, const EncSym* d_enc, const uint32_t* canon,
@@ -2238,13 +2244,12 @@ hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, cons
     fp.sl0 = fp.sl1 = encode_fast_list_slot(g);
     fp.cw = hp.cw; fp.canon_bytes = hp.canon_bytes;
     fp.stride0 = slot_stride(fp.sl0); fp.stride1 = slot_stride(fp.sl1);
-    const uint32_t lb = ws_lds_bytes(1, fp.canon_bytes, fp.stride0, fp.stride1);
+    const uint32_t lb = encode_fast_list_lds(hp, g);
     int dev = 0, ncu = 0;
     hipError_t e;
     if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
     if ((e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
-    auto run = [&](auto kern) -> hipError_t {
-        const uint32_t nthreads = 64u * (2 + ENC_NPK);
+    auto run = [&](auto kern, uint32_t nthreads = 64u * (2 + ENC_NPK)) -> hipError_t {
         hipError_t r = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)lb);
         if (r != hipSuccess) return r;
@@ -2254,6 +2259,9 @@ hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, cons
                                                    redo_list, nullptr, nullptr, report, n_report));
         return hipGetLastError();
     };
+    if (g.spe == 0)
+        return hp.escapes ? run(encode_fast_kernel<0, true, false, 1, 2 * ENC_NPK, true>, 64u * (4 + 2 * ENC_NPK))
+                          : run(encode_fast_kernel<0, false, false, 1, 2 * ENC_NPK, true>, 64u * (4 + 2 * ENC_NPK));
     if (g.spe == 2) return hp.escapes ? run(encode_fast_kernel<2, true, false, 1, ENC_NPK, true>)
                                       : run(encode_fast_kernel<2, false, false, 1, ENC_NPK, true>);
     return hp.escapes ? run(encode_fast_kernel<1, true, false, 1, ENC_NPK, true>)
