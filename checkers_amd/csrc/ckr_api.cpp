@@ -1176,33 +1176,57 @@ namespace {
 constexpr int kUseHostTable = 1;  // compress_device_table: take the host's sorted table instead
 
 // The symbol-0 state chains of every count (ckr::launch_canon_chains), one
-// buffer per device, made and filled on first use and kept for the process.
-const void* canon_chains(hipStream_t s) {
+// buffer per device, kept for the process; made (8.4 MB, filled on a stream of
+// the library's own) by the first call with make set.  Null: none to use, the
+// callers have paths that do without.  The host never waits here: until the
+// fill is known to be complete, the caller's stream is made to wait for it.
+const void* canon_chains(hipStream_t s, bool make = true) {
+    struct PerDevice {
+        void* p = nullptr;
+        hipStream_t fill = nullptr;    // while the fill may still run
+        hipEvent_t filled = nullptr;
+    };
     static std::mutex mu;
-    static std::vector<void*> per_dev;
+    static std::vector<PerDevice> per_dev;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
     std::lock_guard<std::mutex> lk(mu);
-    if ((int)per_dev.size() <= dev) per_dev.resize(dev + 1, nullptr);
-    if (!per_dev[dev]) {
-        // a capturing stream can neither allocate nor fill them: the callers have
-        // paths that do without
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        void* p = nullptr;
-        if (hipMalloc(&p, ckr::kChainBytes) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-        // filled before any other stream or thread can see them (once per process)
-        if (ckr::launch_canon_chains(p, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
-            (void)hipGetLastError();
-            (void)hipFree(p);
-            return nullptr;
-        }
-        per_dev[dev] = p;
+    if ((int)per_dev.size() <= dev) per_dev.resize(dev + 1);
+    PerDevice& c = per_dev[dev];
+    if (c.p && !c.filled) return c.p;
+    if (!c.p && !make) return nullptr;
+    // a capturing stream can neither have them made nor wait for their fill
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
     }
-    return per_dev[dev];
+    const void* r = nullptr;
+    auto settle = [&]() {  // the stream and the event are not needed any more
+        if (c.filled) (void)hipEventDestroy(c.filled);
+        if (c.fill) (void)hipStreamDestroy(c.fill);
+        c.filled = nullptr;
+        c.fill = nullptr;
+    };
+    if (!c.p) {
+        void* p = nullptr;
+        if (hipMalloc(&p, ckr::kChainBytes) == hipSuccess &&
+            hipStreamCreateWithFlags(&c.fill, hipStreamNonBlocking) == hipSuccess &&
+            hipEventCreateWithFlags(&c.filled, hipEventDisableTiming) == hipSuccess &&
+            ckr::launch_canon_chains(p, c.fill) == hipSuccess && hipEventRecord(c.filled, c.fill) == hipSuccess) {
+            c.p = p;
+        } else {
+            settle();
+            if (p) (void)hipFree(p);
+        }
+    }
+    if (c.p) {
+        const hipError_t q = hipEventQuery(c.filled);
+        if (q == hipSuccess) settle();
+        if (q == hipSuccess || (q == hipErrorNotReady && hipStreamWaitEvent(s, c.filled, 0) == hipSuccess)) r = c.p;
+    }
+    (void)hipGetLastError();
+    return r;
 }
 
 // A tensor's encode with the table built on the device (tensors the fast
@@ -1938,8 +1962,11 @@ int decode_impl(const uint8_t* d_data, const ckr_stream_header* d_headers, const
     auto* bad = reinterpret_cast<unsigned long long*>(ws + L.off_bad);
     const CanonKs ck = canon_ks(g);
     // decode table, canonical streams and a cleared bad-lane counter: one launch
-    // where the state chains cover the lane counts (units up to 64 KiB)
-    const void* chains = L.fast && !noalloc && std::max(ck.k0, ck.k1) <= ckr::kChainSteps ? canon_chains(s) : nullptr;
+    // where the state chains cover the lane counts (units up to 64 KiB).  A
+    // decode that the host does not wait for queues its work and nothing else:
+    // it takes the chains only if they exist.
+    const void* chains = L.fast && !noalloc && std::max(ck.k0, ck.k1) <= ckr::kChainSteps
+                             ? canon_chains(s, h_bad_lanes != nullptr) : nullptr;
     if (chains) {
         CKR_HIP(ckr::launch_dec_setup(ta, dec, canon, bad, ck.k0, ck.k1, ck.k2, ck.cw, chains, s));
     } else {
