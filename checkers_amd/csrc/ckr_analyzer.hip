@@ -402,13 +402,15 @@ Layout layout(uint64_t n_rec, uint64_t n_blk) {
 
 }  // namespace
 
+// Enough for the most blocks that each record takes in any list, so that a
+// workspace for a list also serves a part of it, or smaller records: with fewer
+// bytes in all a record takes more blocks.
 uint64_t analyze_workspace_bytes(const ckr_stats_record* recs, uint64_t n) {
     uint64_t nr = 0, nb = 0;
-    const uint64_t per_block = bytes_per_block(recs, n);
     for (uint64_t i = 0; i < n; i++)
         if (analyzable(recs[i])) {
             nr++;
-            nb += blocks_for(recs[i], per_block);
+            nb += blocks_for(recs[i], kMinBytesPerBlock);
         }
     return nr ? layout(nr, nb).total : 0;
 }

@@ -317,7 +317,8 @@ CKR_API int ckr_decode_noalloc(const uint8_t* d_data, const ckr_stream_header* d
  * All records go through two launches (two passes over the data, each with
  * every record's blocks in one grid).  The workspace size depends on each
  * record's pointer, element count and dtype (records with a null pointer, no
- * elements or an unknown dtype are skipped, as the reference skips them);
+ * elements or an unknown dtype are skipped, as the reference skips them); one
+ * sized for a list also serves any part of it, and smaller records;
  * data pointers must be aligned to their element size. */
 CKR_API uint64_t ckr_analyze_workspace_bytes(const ckr_stats_record* h_records, uint64_t n);
 CKR_API int ckr_analyze(const ckr_stats_record* h_records, uint64_t n,
