@@ -33,13 +33,18 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kHistCopies = 16;  // 8, 16, 32 within 2%; 64 (a copy per lane) 35% slower
 // Loads in flight per thread.  Pass 2 with 4 takes 103 VGPRs, so half the waves
-// fit; with 2, held to 64 VGPRs, all 8 per SIMD.  For 144 records of 1.53 GB in
-// all the whole call takes 592 us with 2 and 650 with 4 (721 with 4, 128 KiB
-// blocks and closing kernels of their own); for four records of 1G elements
-// (long loops per thread) 4742 us with 2 and 4650 with 4.  So 4 from
-// kLongBlock bytes per block (about 4 GB a call) on.
+// fit; with 2, held to 64 VGPRs, all 8 per SIMD.  2 is the better one for most
+// calls, whose blocks fill the device (144 records of 1.53 GB in all: 592 us with
+// 2, 650 with 4; four records of 64 Mi fp32, 1 MiB per block: 371 and 428) or
+// are short (one of 1 Mi: 36.3 and 40.9).  4 where the loops are long: from
+// kLongBlock bytes per block of all calls on (four records of 1 Gi elements: 4742
+// us with 2, 4650 with 4), and from kLongBlockFew where one or two records leave
+// two waves per SIMD at most, which 2 loads each do not keep the memory busy with
+// (one record of 256 Mi fp32: 716 and 594; of 64 Mi, 169 and 163; of 16 Mi,
+// 256 KiB per block, 69.7 and 71.4).
 constexpr int kUnroll1 = 4;
-constexpr uint64_t kLongBlock = 2 << 20;
+constexpr uint64_t kLongBlock = 2 << 20, kLongBlockFew = 512 << 10;
+constexpr uint64_t kFewBlocks = 512;  // two per CU
 // At most 256 workgroups per record, so that pass 2's closing global atomics
 // (one per histogram bin and workgroup) stay few (four records of 1G elements:
 // 2048 workgroups per record 5.18 ms per call; 512, 4.95; 256, 4.70; 128, 6.34).
@@ -417,7 +422,7 @@ uint64_t analyze_workspace_bytes(const ckr_stats_record* recs, uint64_t n) {
 
 hipError_t launch_analyze(const ckr_stats_record* recs, uint64_t n, void* ws, hipStream_t s) {
     std::vector<StatsDesc> d;
-    uint64_t nb = 0;
+    uint64_t nb = 0, longest = 0;  // blocks; the most bytes of one
     const uint64_t per_block = bytes_per_block(recs, n);
     for (uint64_t i = 0; i < n; i++) {
         const ckr_stats_record& r = recs[i];
@@ -437,6 +442,7 @@ hipError_t launch_analyze(const ckr_stats_record* recs, uint64_t n, void* ws, hi
         x.mm = r.d_minmax;
         x.fp = r.d_fingerprint;
         nb += x.nblk;
+        longest = std::max(longest, record_bytes(r) / x.nblk);
         d.push_back(x);
     }
     if (d.empty()) return hipSuccess;
@@ -456,7 +462,7 @@ hipError_t launch_analyze(const ckr_stats_record* recs, uint64_t n, void* ws, hi
     }
     const uint32_t nr = (uint32_t)d.size();
     CKR_LAUNCH("stats_pass1_kernel", s, stats_pass1_kernel<<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, p1, prm));
-    if (per_block >= kLongBlock) CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<4><<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
+    if (per_block >= kLongBlock || (nb <= kFewBlocks && longest >= kLongBlockFew)) CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<4><<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
     else CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<2><<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
     return hipGetLastError();
 }
