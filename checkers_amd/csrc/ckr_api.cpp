@@ -249,8 +249,20 @@ hipError_t canon_launch(const ckr_freq_table* t, const CanonKs& ck, uint32_t* ca
     return hipSuccess;
 }
 
+// int8 and int32 in short units stay with the general kernels: the fast encoder
+// hands a unit's offset on to the next one and steps over its 256 short lanes 16
+// bytes at a time, which a short unit has no coding to hide behind.  Compress of 4
+// MB of int8 (int32) in 256-byte units: 157 us (152) general, 5271 (3377) fast; in
+// 1 KiB units 92 (89) and 161 (220); 2 KiB 84 (81) and 94 (108); 4 KiB 85 (81) and
+// 70 (73); 8 KiB 97 (91) and 64 (65).  The fewer the units, the shorter those that
+// the fast encoder leads with (1 MB in 1 KiB units 68 (67) and 71 (84), in 2 KiB
+// units 69 (66) and 61 (60); 16 MB in 4 KiB units 142 (114) and 154 (160)).
+bool long_unmasked_units(const ckr::EncodeGeom& g) {
+    const uint64_t K = (g.unit + 255) / 256;
+    return K >= 32 || (K >= 8 && g.n_units <= 64 * K);
+}
 bool use_fast_encode(const ckr::EncodeGeom& g) {
-    return g_fast_paths && g.n_units > 0 && (g.unit + 255) / 256 <= kFastMaxK;
+    return g_fast_paths && g.n_units > 0 && (g.unit + 255) / 256 <= kFastMaxK && (g.spe || long_unmasked_units(g));
 }
 // Units above 64 KiB (up to the dedup limit): the two-pass kernels.
 bool use_seg_encode(const ckr::EncodeGeom& g) { return use_dedup(g) && (g.unit + 255) / 256 > kFastMaxK; }
@@ -370,7 +382,11 @@ DecodeLayout decode_layout(const ckr::EncodeGeom& g) {
     DecodeLayout L{};
     const CanonKs ck = canon_ks(g);
     L.fast = g_fast_paths != 0 && g.spe > 0 && g.n_units > 0 && use_dedup(g);
-    L.fast_any = L.fast || (g_fast_paths != 0 && g.spe == 0 && g.n_units > 0 && (g.unit + 255) / 256 <= kDedupMaxK);
+    // int8 and int32: from 3 KiB units on (a lane's set-up outweighs fewer rows:
+    // 16 MB of int8 in 1 KiB units 52 us general, 68 fast; 2 KiB 46, 52; 4 KiB 57,
+    // 42; one unit of 1000 bytes 26, 32; of 3 KiB 35, 35; of 6 KiB 48, 30)
+    const uint64_t K = (g.unit + 255) / 256;
+    L.fast_any = L.fast || (g_fast_paths != 0 && g.spe == 0 && g.n_units > 0 && K >= 12 && K <= kDedupMaxK);
     uint64_t o = 0;
     L.off_canon = o; o = align_up(o + (L.fast ? 3ull * (4 + 2 * ck.cw) * 4 : 0), kAlign);
     L.off_dec = o;   o = align_up(o + 4096 * 4, kAlign);

@@ -532,7 +532,7 @@ CKR_API int ckr_make_contiguous(const void* d_src, int ndim, const int64_t* shap
  * streams are identical), units of at most 64 KiB coded and decoded through
  * LDS; mode 0: every lane coded and decoded independently through global
  * memory (modes 1 to 3 take int8 and int32, which have no masked planes, the same way
- * as the other dtypes); mode 2: fast kernels with minimal LDS lane slots, so that nearly
+ * as the other dtypes, units of fewer than 32 rows of 256 bytes aside); mode 2: fast kernels with minimal LDS lane slots, so that nearly
  * every unit takes the overflow route back through the general kernels; mode
  * 3: the same minimal slots, the overflowing units coded again by the fast
  * encoder with slots that hold any lane (mode 1's overflow route).  In
