@@ -1965,10 +1965,11 @@ int decode_prepare(const uint8_t* d_data, const ckr_stream_header* d_headers, co
 // counted: the caller reads the bad-lane count (h_bad_lanes, or
 // ckr_decode_many's check), so that the fast decoder also compares the
 // zero-plane lanes' bytes, which do not enter the output.
+// all_units: of all the decodes that share the device with this one (0: none do).
 int decode_impl(const uint8_t* d_data, const ckr_stream_header* d_headers, const uint64_t* d_unit_offsets,
                 const ckr_freq_table* h_table, uint64_t n_elems, int dtype, uint64_t unit_bytes,
                 const uint8_t* d_sidecar, void* d_dst, void* d_workspace, uint64_t workspace_bytes,
-                uint64_t* h_bad_lanes, void* stream, bool noalloc, bool counted) {
+                uint64_t* h_bad_lanes, void* stream, bool noalloc, bool counted, uint64_t all_units = 0) {
     if (h_bad_lanes) *h_bad_lanes = 0;
     DecPrep p;
     if (int rc = decode_prepare(d_data, d_headers, d_unit_offsets, h_table, n_elems, dtype, unit_bytes, d_sidecar, d_dst,
@@ -2011,7 +2012,7 @@ int decode_impl(const uint8_t* d_data, const ckr_stream_header* d_headers, const
     hipError_t de = use_long_units(g)
                         ? ckr::launch_decode_long(d_data, d_headers, d_unit_offsets, dec, g, d_sidecar, out, bad, s)
                         : ckr::launch_decode(d_data, d_headers, d_unit_offsets, dec, g, d_sidecar, out, bad,
-                                             L.fast ? canon : nullptr, ck.cw, L.fast_any, s, counted);
+                                             L.fast ? canon : nullptr, ck.cw, L.fast_any, s, counted, all_units);
     if (tmp) {
         if (de == hipSuccess) de = hipMemcpyAsync(d_dst, tmp, g.n_bytes, hipMemcpyDeviceToDevice, s);
         (void)hipFreeAsync(tmp, s);
@@ -2105,11 +2106,14 @@ int ckr_decode_many(ckr_decode_job* jobs, uint64_t n, uint64_t unit_bytes, int c
     // effect every job goes on the caller's stream, so that a launch's
     // profiling events bracket its own kernel.
     bool small = true;
+    uint64_t all_units = 0;  // of small jobs side by side
     for (uint64_t i = 0; i < n && small; i++) {
         ckr::EncodeGeom g;
         make_geom(jobs[i].n_elems, jobs[i].dtype, unit_bytes, &g);
         small = g.n_bytes <= kManySmallJobBytes;
+        all_units += g.n_units;
     }
+    if (!small || n == 1 || g_prof_on) all_units = 0;
     std::vector<hipStream_t> pool{s};
     if (n > 1 && !g_prof_on) {
         if (small) pool = {s, a->s2, a->sx[0], a->sx[1]};
@@ -2221,7 +2225,7 @@ int ckr_decode_many(ckr_decode_job* jobs, uint64_t n, uint64_t unit_bytes, int c
         hipStream_t js = pool[i % pool.size()];
         int rc = decode_impl(jb.d_data, jb.d_headers, jb.d_unit_offsets, jb.h_table, jb.n_elems, jb.dtype, unit_bytes,
                              jb.d_sidecar, jb.d_dst, jb.d_workspace, jb.workspace_bytes, nullptr, js, false,
-                             check != 0);
+                             check != 0, all_units);
         if (rc == CKR_OK && check) {
             ckr::EncodeGeom g;
             make_geom(jb.n_elems, jb.dtype, unit_bytes, &g);

@@ -327,10 +327,12 @@ uint32_t decode_fast_lds_bytes();
 // their canonical streams (their headers are checked either way); those bytes
 // do not enter the output, so only a caller that reads the bad-lane count
 // needs them read.
+// all_units: the units of all launches that share the device with this one
+// (small tensors on several streams; 0: it has the device to itself).
 hipError_t launch_decode(const uint8_t* data, const ckr_stream_header* hdrs, const uint64_t* unit_off,
                          const uint32_t* d_dec, const EncodeGeom& g, const uint8_t* sidecar, uint8_t* dst,
                          unsigned long long* bad, const uint32_t* canon, uint32_t cw, bool fast_ok, hipStream_t s,
-                         bool zero_bytes = true);
+                         bool zero_bytes = true, uint64_t all_units = 0);
 
 // Analyzer (ckr_analyzer.hip): every record in one grid per pass.
 struct StatsParams {     // per record, device resident between passes

@@ -4874,7 +4874,7 @@ hipError_t launch_decode_fast_multi(DecJob* jobs, uint32_t n, hipStream_t s) {
 hipError_t launch_decode(const uint8_t* data, const ckr_stream_header* hdrs, const uint64_t* unit_off,
                          const uint32_t* d_dec, const EncodeGeom& g, const uint8_t* sidecar, uint8_t* dst,
                          unsigned long long* bad, const uint32_t* canon, uint32_t cw, bool fast_ok, hipStream_t s,
-                         bool zero_bytes) {
+                         bool zero_bytes, uint64_t all_units) {
     const uint32_t grid = (uint32_t)((g.n_units + 3) / 4);
     if (grid == 0) return hipSuccess;
     hipError_t e;
@@ -4891,8 +4891,18 @@ hipError_t launch_decode(const uint8_t* data, const ckr_stream_header* hdrs, con
                 (void)hipGetLastError();
                 return hipSuccess;  // LDS too small on this device: the general kernel takes every unit
             }
-            // persistent: the blocks that fit at once, never more than units
-            const uint32_t fg = (uint32_t)std::min<uint64_t>(g.n_units, (uint64_t)per_cu * (uint64_t)std::max(ncu, 1));
+            // persistent: the blocks that fit at once, never more than units; beside
+            // other launches the tensor's share of them, at least as many as its units
+            // fill (the others would wait for the CUs that nearly empty blocks hold: a
+            // shard of six bf16 tensors and an int32 one 203 us with every launch
+            // spread over all CUs, 172 so).  A tensor with most of the units is spread
+            // as if alone (1024 units of fp32 and a small int32 tensor: 111 us, with
+            // one block less 123, as some SIMDs then have two waves).
+            const uint64_t fit = (uint64_t)per_cu * (uint64_t)std::max(ncu, 1);
+            const uint64_t upb = g.spe ? DF_WAVES : DF_WAVES / 2;  // units that fill a block
+            const uint64_t need = 4 * g.n_units < 3 * all_units
+                                      ? std::max((g.n_units + upb - 1) / upb, fit * g.n_units / all_units) : g.n_units;
+            const uint32_t fg = (uint32_t)std::min({need, g.n_units, fit});
             if constexpr (std::is_same_v<decltype(kern), decltype(&decode_fast_unmasked_kernel)>)
                 CKR_LAUNCH("decode_fast_kernel", s, kern<<<fg, 64 * DF_WAVES, lb, s>>>(data, hdrs, unit_off, d_dec, g, dst, bad));
             else
