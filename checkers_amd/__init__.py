@@ -33,7 +33,7 @@ EXPORTED = [  # every symbol include/checkers_amd.h declares
     "ckr_decode_noalloc", "ckr_analyze_workspace_bytes",
     "ckr_analyze", "ckr_profile_begin", "ckr_profile_end", "ckr_set_fast_paths",
     "ckr_repair_masked_bits", "ckr_repair_bucket_count", "ckr_repair_workspace_bytes",
-    "ckr_repair_build", "ckr_repair_apply",
+    "ckr_repair_build", "ckr_repair_apply", "ckr_repair_graphs_made",
     "ckr_fingerprint_weights", "ckr_cluster", "ckr_ckpt_write", "ckr_ckpt_set_slice_bytes",
     "ckr_ckpt_slice_bytes", "ckr_ckpt_reserve", "ckr_ckpt_pool_bytes", "ckr_ckpt_release",
     "ckr_ckpt_open", "ckr_ckpt_count",
@@ -162,6 +162,7 @@ def lib():
         "ckr_repair_workspace_bytes": (u64, [u64, i32, i32, ctypes.c_uint32]),
         "ckr_repair_build": (i32, [vp, u64, i32, i32, ctypes.c_uint32, vp, vp, vp, vp, vp, vp, u64, vp]),
         "ckr_repair_apply": (i32, [vp, u64, i32, i32, vp, ctypes.c_uint32, vp, vp, vp, u64, vp]),
+        "ckr_repair_graphs_made": (u64, []),
         "ckr_fingerprint_weights": (i32, [vp, u64, vp]),
         "ckr_cluster": (i32, [vp, vp, u64, vp, vp]),
         "ckr_ckpt_write": (i32, [ctypes.c_char_p, i32, vp, u64, u64, i32, vp, vp]),

@@ -2477,6 +2477,8 @@ int ckr_repair_build(const void* d_words, uint64_t n_elems, int dtype, int maske
                       h_out_tokens, h_max_pair_frequency, d_seq_out, d_workspace, workspace_bytes, stream);
 }
 
+uint64_t ckr_repair_graphs_made(void) { return ckr::repair_graphs_made(); }
+
 int ckr_repair_apply(const void* d_words, uint64_t n_elems, int dtype, int masked_bits,
                      const ckr_repair_rule* h_rules, uint32_t n_rules, uint64_t* h_out_tokens, uint64_t* d_seq_out,
                      void* d_workspace, uint64_t workspace_bytes, void* stream) {

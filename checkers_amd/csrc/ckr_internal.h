@@ -393,5 +393,6 @@ struct RepairArgs {
     RepairLayout layout;
 };
 hipError_t repair_launch(const RepairArgs& a, hipStream_t s);
+uint64_t repair_graphs_made();  // graphs of build rounds captured so far
 
 }  // namespace ckr

@@ -1491,11 +1491,11 @@ hipError_t build_alphabet(const uint8_t* words, uint64_t n, int es, uint32_t k, 
 
 constexpr uint32_t kRoundBatch = 8;
 
-// The captured graphs of a batch of build rounds (kRoundBatch, or the last batch's
-// remainder), keyed by what their kernels' arguments derive from (the
-// workspace and its layout's inputs) and the batch length.  A graph is
-// captured on a library stream, instantiated once and kept; at most
-// kMaxRoundGraphs are kept (the oldest goes).
+// The captured graphs of a batch of build rounds, keyed by what their kernels'
+// arguments derive from (the workspace and its layout's inputs), the batch length
+// and its full rounds: at most six per workspace and rule limit, whatever the
+// data (run_rounds).  A graph is captured on a library stream, instantiated once
+// and kept; at most kMaxRoundGraphs are kept (the oldest goes).
 struct RoundGraphKey {
     const void* ws;
     uint64_t n;
@@ -1514,6 +1514,7 @@ struct RoundGraph {
 constexpr size_t kMaxRoundGraphs = 64;
 std::mutex g_rg_mu;
 std::vector<RoundGraph> g_rgs;
+uint64_t g_rg_made = 0;
 
 // A library stream per device, made on first use (graph capture).
 hipStream_t side_stream(int dev, std::vector<hipStream_t>& v) {
@@ -1554,6 +1555,7 @@ hipGraphExec_t round_graph(const RepairArgs& A, const RepairLayout& L, uint32_t 
         g_rgs.erase(g_rgs.begin());
     }
     g_rgs.push_back({key, g, x});
+    g_rg_made++;
     return x;
 }
 
@@ -1666,11 +1668,10 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
                                                            nids, hist, rs)));
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    // A build's rounds go in batches of kRoundBatch (the last one shorter), each
-    // batch one launch of a graph captured once per workspace, shape and batch
-    // length and kept (a round is up to 7 launches, whose host cost would
-    // otherwise exceed a small tensor's GPU work).  While ckr_profile_begin is
-    // in effect the kernels are launched one by one.
+    // A build's rounds go in batches, each one launch of a graph captured once and
+    // kept (a round is up to 7 launches, whose host cost would otherwise exceed a
+    // small tensor's GPU work).  While ckr_profile_begin is in effect the kernels
+    // are launched one by one.
     //
     // A build reads the device's state after a batch: it stops once the grammar
     // is done (rounds past the last rule return at once), and else goes on from
@@ -1684,13 +1685,22 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
     // rounds tie (few words, or many that are all rare) tie from the start: the
     // first batch is two full rounds, and lean batches follow batches without a
     // tie only.
+    //
+    // Graphs have one of three lengths, so that the data decides which are launched
+    // but not which there are: the first batch's (all rounds of a build of no more
+    // than kRoundBatch, which is read back once, at its end: 5 rules of 1000 words
+    // 252 us against 268 in two batches), kRoundBatch, and what the rule limit
+    // leaves over of whole batches.  Behind a stop another number may be left: those
+    // rounds are launched one by one (at least 35 us each on the device, 25 to launch).
+    const uint32_t first = R.rounds <= kRoundBatch ? R.rounds : 2, over = (R.rounds - first) % kRoundBatch;
     auto launch = [&](uint32_t n_rounds, uint32_t full) -> hipError_t {
-        hipGraphExec_t gx = ckr::profiling() ? nullptr : round_graph(A, L, n_rounds, full, batch);
+        const bool kept = n_rounds == first || n_rounds == kRoundBatch || n_rounds == over;
+        hipGraphExec_t gx = !kept || ckr::profiling() ? nullptr : round_graph(A, L, n_rounds, full, batch);
         return gx ? hipGraphLaunch(gx, s) : batch(s, n_rounds, full);
     };
-    uint32_t full_until = A.recount_each_round ? R.rounds : 2, stops = 0, ties = 0;
+    uint32_t full_until = A.recount_each_round ? R.rounds : first, stops = 0, ties = 0;
     for (uint32_t r = 0; A.build && r < R.rounds;) {
-        const uint32_t n_rounds = std::min(r == 0 ? 2u : kRoundBatch, R.rounds - r);
+        const uint32_t n_rounds = r == 0 ? first : std::min(kRoundBatch, R.rounds - r);
         const uint32_t full = r < full_until ? n_rounds : 1;
         if ((e = launch(n_rounds, full)) != hipSuccess) return e;
         if (full == n_rounds && r + n_rounds >= R.rounds) break;  // no round of it can have been left out
@@ -1716,6 +1726,11 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
 }
 
 }  // namespace
+
+uint64_t repair_graphs_made() {
+    std::lock_guard<std::mutex> lk(g_rg_mu);
+    return g_rg_made;
+}
 
 hipError_t repair_launch(const RepairArgs& A, hipStream_t s) {
     return A.layout.tok16 ? run_rounds<uint16_t>(A, s) : run_rounds<uint32_t>(A, s);

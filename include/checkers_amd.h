@@ -363,6 +363,9 @@ CKR_API int ckr_repair_build(const void* d_words, uint64_t n_elems, int dtype, i
 CKR_API int ckr_repair_apply(const void* d_words, uint64_t n_elems, int dtype, int masked_bits,
                              const ckr_repair_rule* h_rules, uint32_t n_rules, uint64_t* h_out_tokens,
                              uint64_t* d_seq_out, void* d_workspace, uint64_t workspace_bytes, void* stream);
+/* No counterpart in the reference: how many graphs of build rounds the process
+ * has captured (at most six per workspace, tensor size and rule limit). */
+CKR_API uint64_t ckr_repair_graphs_made(void);
 
 /* ---- fingerprint weights and clusters (host) ----
  * ckr_fingerprint_weights ← TensorAnalyzer::compute_fingerprint_weights

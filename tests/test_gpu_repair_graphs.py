@@ -1,0 +1,42 @@
+"""Builds on one workspace: the data decides how many rounds run and in which one a
+lean batch stops, not which graphs exist, and the rules equal the oracle's behind
+every length of the last batch."""
+import numpy as np
+import pytest
+
+import oracle as oc
+
+pytestmark = pytest.mark.gpu
+
+PAIRS = 40
+
+
+def _ties_in(rng, rnd):
+    """40 pairs of words of their own, each rarer than the one before but for the one
+    after `rnd`, shuffled: the rules take them in order, and only that round ties
+    (what the shuffle makes adjacent occurs far less often)."""
+    counts = 200 - 3 * np.arange(PAIRS)
+    counts[rnd + 1] = counts[rnd]
+    which = rng.permutation(np.repeat(np.arange(PAIRS), counts))
+    return (np.stack([2 * which + 1, 2 * which + 2], 1).reshape(-1).astype(np.uint16)) << 7
+
+
+@pytest.mark.parametrize("max_rules", [3, 8, 9, 10, 13, 30])
+def test_graphs_per_workspace(max_rules, gpu):
+    import torch
+
+    import checkers_amd as ck
+    n = int(_ties_in(np.random.default_rng(0), 5).size) + 3
+    k = ck.repair_masked_bits(1, None)
+    rp = ck.Repairer(n, 1, None, max_rules)
+    before = ck.lib().ckr_repair_graphs_made()
+    for rnd in (1, 3, 4, 5, 6, 7, 8, 9, 12, 14, 15, 21, 25):
+        w = _ties_in(np.random.default_rng(rnd), rnd)
+        words = np.concatenate([w, np.full(n - w.size, 500 << 7, np.uint16)])
+        raw = words.view(np.uint8)
+        ref = oc.repair_build(raw, n, 2, k, max_rules, want_seq=True)
+        got = rp.build(torch.from_numpy(raw.copy()).to(gpu), want_seq=True)
+        assert got["rules"] == ref["rules"] and got["out_len"] == ref["out_len"]
+        assert np.array_equal(got["seq"], ref["seq"])
+    made = ck.lib().ckr_repair_graphs_made() - before
+    assert made <= 6, made
