@@ -1526,27 +1526,34 @@ hipStream_t side_stream(int dev, std::vector<hipStream_t>& v) {
     return v[dev];
 }
 
+// Launches the batch's graph on s; false: there is none, and nothing was launched.
+// The lock is held until it is launched: another thread's capture may drop the
+// oldest graph, which waits for what runs but not for what is about to.
 template <typename BatchFn>
-hipGraphExec_t round_graph(const RepairArgs& A, const RepairLayout& L, uint32_t len, uint32_t full, BatchFn& batch) {
+bool round_graph_launch(const RepairArgs& A, const RepairLayout& L, uint32_t len, uint32_t full, BatchFn& batch,
+                        hipStream_t s, hipError_t* launched) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return false; }
     const RoundGraphKey key{A.ws, A.n, A.es, dev, L.tok16 ? 1 : 0, A.k, A.max_rules,
                             A.recount_each_round ? 1u : 0u, len, full};
     std::lock_guard<std::mutex> lk(g_rg_mu);
     for (const RoundGraph& r : g_rgs)
-        if (r.key == key) return r.x;
+        if (r.key == key) {
+            *launched = hipGraphLaunch(r.x, s);
+            return true;
+        }
     static std::vector<hipStream_t> cap;  // one capture stream per device
     hipStream_t cs = side_stream(dev, cap);
-    if (!cs) return nullptr;
+    if (!cs) return false;
     hipGraph_t g = nullptr;
     hipGraphExec_t x = nullptr;
-    if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) { (void)hipGetLastError(); return false; }
     const hipError_t e = batch(cs, len, full);
     const hipError_t e2 = hipStreamEndCapture(cs, &g);
     if (e != hipSuccess || e2 != hipSuccess || !g || hipGraphInstantiate(&x, g, nullptr, nullptr, 0) != hipSuccess) {
         (void)hipGetLastError();
         if (g) (void)hipGraphDestroy(g);
-        return nullptr;  // the rounds are then launched one by one
+        return false;  // the rounds are then launched one by one
     }
     if (g_rgs.size() >= kMaxRoundGraphs) {
         (void)hipDeviceSynchronize();  // the oldest graph may still run somewhere
@@ -1556,7 +1563,8 @@ hipGraphExec_t round_graph(const RepairArgs& A, const RepairLayout& L, uint32_t 
     }
     g_rgs.push_back({key, g, x});
     g_rg_made++;
-    return x;
+    *launched = hipGraphLaunch(x, s);
+    return true;
 }
 
 template <typename T>
@@ -1695,8 +1703,9 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
     const uint32_t first = R.rounds <= kRoundBatch ? R.rounds : 2, over = (R.rounds - first) % kRoundBatch;
     auto launch = [&](uint32_t n_rounds, uint32_t full) -> hipError_t {
         const bool kept = n_rounds == first || n_rounds == kRoundBatch || n_rounds == over;
-        hipGraphExec_t gx = !kept || ckr::profiling() ? nullptr : round_graph(A, L, n_rounds, full, batch);
-        return gx ? hipGraphLaunch(gx, s) : batch(s, n_rounds, full);
+        hipError_t le = hipSuccess;
+        if (kept && !ckr::profiling() && round_graph_launch(A, L, n_rounds, full, batch, s, &le)) return le;
+        return batch(s, n_rounds, full);
     };
     uint32_t full_until = A.recount_each_round ? R.rounds : first, stops = 0, ties = 0;
     for (uint32_t r = 0; A.build && r < R.rounds;) {
