@@ -840,7 +840,10 @@ int encode_impl(const void* d_src, uint64_t n_elems, int dtype, const ckr_freq_t
         for (int s2 = 0; s2 < 256; s2++)
             if ((h_planes[s2] || h_planes[256 + s2]) && !h_table->norm_freq[s2]) escapes = true;
     }
-    bool fast = use_fast_encode(g);
+    // int8 and int32 with no total to read back: the general kernels, which the
+    // call only queues (the fast encoder's control words have to be read), so that
+    // it can be captured
+    bool fast = use_fast_encode(g) && (g.spe || h_total_out || defer);
     ckr::FastEncParamsHost fp{};
     if (fast) {
         fp.escapes = escapes;

@@ -166,7 +166,9 @@ CKR_API int ckr_build_tables_device(const uint32_t* d_hists, uint64_t n, int ens
  * The table is given on the host.  The workspace must hold
  * ckr_encode_workspace_bytes(...) bytes; d_out must hold
  * ckr_encode_max_output_bytes(...) bytes.  If h_total_out is not NULL the
- * call synchronises `stream` and stores C there. ---- */
+ * call synchronises `stream` and stores C there.  If it is NULL, int8 and int32
+ * are only queued (and may be captured into a graph); the other dtypes'
+ * encoders still read their control words back. ---- */
 CKR_API uint64_t ckr_num_units(uint64_t n_elems, int dtype, uint64_t unit_bytes);
 CKR_API uint64_t ckr_encode_max_output_bytes(uint64_t n_elems, int dtype, uint64_t unit_bytes);
 CKR_API uint64_t ckr_encode_workspace_bytes(uint64_t n_elems, int dtype, uint64_t unit_bytes);
