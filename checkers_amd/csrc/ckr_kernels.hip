@@ -717,7 +717,7 @@ __global__ void __launch_bounds__(256) masked_hist_multi_kernel(HistJobs jobs) {
     else masked_hist_share<0, 16>(sh, j.src, j.n_bytes, j.es, j.hist, nullptr, j.head_n, b, j.nblk);
 }
 
-// Histograms and encode set-ups of up to kMaxHistJobs masked tensors in one
+// Histograms and encode set-ups of up to kMaxHistJobs tensors in one
 // grid (launch_hist_table).  Job k's workgroups (blk0 .. blk0 + nblk): the
 // first clears the job's histogram words and done counter, then opens the
 // job's gate with the launch's epoch (no earlier launch used that value, so
@@ -725,7 +725,7 @@ __global__ void __launch_bounds__(256) masked_hist_multi_kernel(HistJobs jobs) {
 // LDS, adds its sums once the gate is open, and takes a done ticket; the one
 // that takes the last ticket builds the table in the same LDS
 // (table_enc_body).  Every workgroup also clears a share of the job's
-// look-back status words.  Words of hist: 768 counts, gate (768-769), done
+// look-back status words.  Words of hist: 768 counts (int8 and int32: 256), gate (768-769), done
 // counter (770), gate time-out stamp (772-773).
 struct HistTableJob {
     HistJob h;
@@ -1348,13 +1348,14 @@ __device__ __forceinline__ uint4 enc_entry_of(uint32_t w) {
 //
 // Instruction issue bounds the coder waves (a wave issues one instruction in
 // about 4.2 cycles whether or not it depends on the one before; v_mul_hi_u32
-// takes 6.5), so the row's instruction count is its time: 12 a row here
-// (address, 2 for n, 3 window shifts, 5 for the state, and half of the 5 of
-// enc_flush) against 20 with two comparisons per row and a selector that
-// tracked the pending bytes.  Measured: a 64 KiB unit coded in 12.7 us instead
+// takes 6.5), so the row's instruction count is its time: 12 vector instructions
+// a row here (address, 2 for n, 3 window shifts, 4 for the state, and half of the 4
+// that move the position and flush; 13 with bf16's sidecar bytes) against 20 with
+// two comparisons per row and a selector that tracked the pending bytes.  Measured: a 64 KiB unit coded in 12.7 us instead
 // of 14.8; the encode of a 436 MB bf16 layer 231 -> 202 us, of a 67 MB fp32
 // tensor 57 -> 52, pass 2 of a 1 GiB fp32 tensor in 1 MiB units 761 -> 650 and
-// pass 1 288 -> 246.  The packer waves are then as slow as the coders.
+// pass 1 288 -> 246.  The packer waves (15.5 us a unit with the look-back) then set
+// the pace.
 struct EncLane {
     uint32_t x, hi, lo, a;
 };
@@ -1596,16 +1597,17 @@ __device__ __forceinline__ void enc_full_rows(EncLane& c, const uint8_t* ucol, u
 //
 // LDS layout (bytes): table 256 x 16 (see enc_quad) | canonical headers 12 x
 // u32 | canonical bytes 3 x canon_bytes | pair control blocks | 2 x WS regions
-// | 32 bytes of read padding.  A region holds one set: the packers' lane
+// | 32 bytes of read padding (int8 and int32: one group of four coder waves, no
+// canonical streams, and one region in list mode).  A region holds one set: the packers' lane
 // records (per lane {LDS address of unit byte 0 as if it were in the lane, end
 // of the lane in the unit}, 8 bytes) and block map (u8 lane per 64 bytes of
 // packed output), then the rank-0 slots (64 x stride0) and the rank-1 slots
-// (64 x stride1).  The records and the map are only written once both coders
-// are done with the set, so they
+// (64 x stride1), or four times 64 slots of one size.  The records and the map are
+// only written once all coders are done with the set, so they
 // double as the guard under the slots: a lane's dwords are flushed downward
 // from the end of its slot, and a lane that outgrows its slot keeps flushing
-// into the slots below it (lanes of the same unit, whose bytes are then redone
-// by the general kernels) and, for the lowest slot, into the lane tables (at
+// into the slots below it (lanes of the same unit, whose bytes are then redone)
+// and, for the lowest slot, into the lane tables (at
 // most 2 bytes per symbol, 256 symbols: 516 bytes), never out of its region.
 static constexpr uint32_t FE_TABSZ = 4096, FE_CHDR = FE_TABSZ, FE_CBYTES = FE_TABSZ + 48;
 // Rows per load group of the fast encoder's coders, entries of their table ring.
@@ -3973,11 +3975,11 @@ static constexpr uint32_t LU_CH = 130;    // chains per unit: 64 columns x 2 liv
 // The chain of one lane (byte SH / 8 of its column) over the 32 ng rows at
 // in32, from the top down: groups of 32 rows, the next two groups' loads in
 // flight while one is coded, and each row's table entry read 7 rows ahead.
-// record(s) at the entry of every segment.  A row is 9.5 VALU instructions and
+// record(s) at the entry of every segment.  A row is 8.6 VALU instructions and
 // one LDS read, all on one wave: instruction issue (about 4.2 cycles each) is
 // what bounds the chain.  A 33.5 MB bf16 tensor (131072 rows): 4.90 ms with
-// enc_step's earlier form (15 instructions) and entries 4 rows ahead in the
-// source but sunk to their use, 4.18 with 9.5 instructions, 3.2 with this ring.
+// two comparisons per row and entries 4 rows ahead in the source but sunk to their
+// use, 4.18 without the comparisons, 3.2 with this ring.
 template <bool ESC, uint32_t SH, typename R>
 __device__ __forceinline__ void lu_chain_rows(uint32_t& x, uint32_t& e, const uint32_t* in32, uint32_t ng, R&& record) {
     constexpr int TR = 8;
@@ -4488,11 +4490,13 @@ static constexpr uint32_t DL_LDS = DL_TAB_BYTES + 4 * DL_RING_BYTES + 64;
 static constexpr uint32_t DL_ROWS = 16;  // rows per group
 static constexpr uint32_t DL_AHEAD = 2;  // groups of sidecar bytes loaded ahead (zero-plane lanes)
 static constexpr uint32_t DL_PUT_AFTER = 2;
-// A group takes at most 2 DL_ROWS bytes of a lane, and its last pair's (4 at most)
-// are counted in the next: chunk ch is entered at 64 ch + 2 DL_ROWS + 3 at most, ch + 1
-// two groups later at the earliest, when the registers of the chunk fetched on
-// entering ch are free again; that chunk, ch + 2, is in the ring before a window
-// (12 bytes with its dwords) reaches it.
+// A step counts at most 2 DL_ROWS bytes of a lane (the group's, but for its last
+// pair's 4 at most, and the last pair's of the group before), and the step before the
+// one that enters chunk ch was at 64 ch - 1 at most: ch is entered at 64 ch + 2
+// DL_ROWS - 1 at most, so that ch + 1, at 64 ch + 64 or more, is entered DL_PUT_AFTER
+// steps later at the earliest, when the registers of the chunk fetched on entering
+// ch are free again (one byte to spare); that chunk, ch + 2, is in the ring before a
+// window (12 bytes with its dwords) reaches it.
 static_assert(2 * DL_ROWS * DL_PUT_AFTER <= 64, "one chunk in flight per lane");
 static_assert(2 * DL_ROWS * (DL_PUT_AFTER + 1) + 4 + 12 <= 128, "a chunk must be in the ring before it is read");
 static_assert(2 * DL_ROWS + 4 + 12 <= DL_LANE - 256, "windows of a group end within the copy of the ring's start");
