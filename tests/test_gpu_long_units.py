@@ -50,3 +50,40 @@ def test_lanes_of_rare_symbols(dt, gpu):
     dst, bad = ck.decode(enc)
     torch.cuda.synchronize()
     assert bad == 0 and np.array_equal(dst.cpu().numpy(), dg.raw_bytes(raw))
+
+
+def test_more_units_than_cus_fp32_with_raw_units(gpu):
+    """Above one unit per CU (decode_long_kernel), fp32, under a table made for other
+    data: units of its frequent bytes are coded, units of rare ones (12 bits each,
+    beside zero planes at 5) are stored raw, the ragged last one among them."""
+    import torch
+    import checkers_amd as ck
+    units = 259
+    n = (units - 1) * (UNIT // 4) + 70_003
+    h = np.full(256, 1, np.uint32)
+    h[0] = 128
+    h[0x30:0x40] = 232
+    t, s = ck.build_table(h)
+    assert s == 4096
+    g = torch.Generator(device=gpu)
+    g.manual_seed(5)
+    b = torch.randint(0, 256, (n, 4), generator=g, device=gpu, dtype=torch.uint8)
+    cheap = torch.randint(0x30, 0x40, (n, 2), generator=g, device=gpu, dtype=torch.uint8)
+    raw_unit = torch.arange(n, device=gpu) // (UNIT // 4) % 3 == 0  # (unit 258 is one)
+    b[:, 2:] = torch.where(raw_unit[:, None], (b[:, 2:] & 63) + 0x80, cheap)
+    src = b.reshape(-1)
+    e = ck.Encoder(n, ck.F32, UNIT)
+    enc = e.encode(src, t)
+    torch.cuda.synchronize()
+    off = enc.unit_offsets[: units + 1].cpu().numpy()
+    size = np.diff(off)
+    length = np.full(units, UNIT)
+    length[-1] = n * 4 - (units - 1) * UNIT
+    assert (size[::3] == length[::3]).all() and (size[1::3] < UNIT).all() and (size[2::3] < UNIT).all()
+    d = ck.Decoder(n, ck.F32, UNIT)
+    dst = torch.zeros(n * 4, dtype=torch.uint8, device=gpu)
+    ck.profile_begin()
+    bad = d.decode(enc.data, enc.headers, enc.unit_offsets, enc.table, enc.sidecar, dst)
+    prof = ck.profile_end()
+    assert "decode_long_kernel" in prof and "decode_chain_kernel" not in prof
+    assert bad == 0 and torch.equal(dst, src)
