@@ -388,7 +388,7 @@ struct RepairArgs {
     const uint64_t* h_primes;         // build: library bucket counts covering [2, n], ascending
     uint32_t n_primes;
     uint64_t* d_seq_out;
-    bool recount_each_round;          // build: every pair recounted each round
+    uint32_t recount;                 // build: 0 when the table is 3/4 full; 1 each round; 2 at 1/16 (tests)
     uint8_t* ws;
     RepairLayout layout;
 };

@@ -1500,10 +1500,10 @@ struct RoundGraphKey {
     const void* ws;
     uint64_t n;
     int es, device, tok16;
-    uint32_t k, rounds, dlimit, batch, full;
+    uint32_t k, rounds, recount, batch, full;
     bool operator==(const RoundGraphKey& o) const {
         return ws == o.ws && n == o.n && es == o.es && device == o.device && tok16 == o.tok16 &&
-               k == o.k && rounds == o.rounds && dlimit == o.dlimit && batch == o.batch && full == o.full;
+               k == o.k && rounds == o.rounds && recount == o.recount && batch == o.batch && full == o.full;
     }
 };
 struct RoundGraph {
@@ -1535,7 +1535,7 @@ bool round_graph_launch(const RepairArgs& A, const RepairLayout& L, uint32_t len
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return false; }
     const RoundGraphKey key{A.ws, A.n, A.es, dev, L.tok16 ? 1 : 0, A.k, A.max_rules,
-                            A.recount_each_round ? 1u : 0u, len, full};
+                            A.recount, len, full};
     std::lock_guard<std::mutex> lk(g_rg_mu);
     for (const RoundGraph& r : g_rgs)
         if (r.key == key) {
@@ -1592,7 +1592,9 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
     R.rounds = A.build ? A.max_rules : A.n_rules;
     // rounds keep their counts while the table stays at most 3/4 full (limit 0:
     // every round recounts)
-    R.dlimit = A.recount_each_round ? 0u : (uint32_t)std::min<uint64_t>(L.pair_cap - L.pair_cap / 4, 0xFFFFFFFFull);
+    R.dlimit = A.recount == 1 ? 0u
+                              : (uint32_t)std::min<uint64_t>(A.recount ? L.pair_cap / 16 : L.pair_cap - L.pair_cap / 4,
+                                                             0xFFFFFFFFull);
     hipError_t e;
 
     CKR_LAUNCH("repair_init_kernel", s, ctl_init<<<1, 1, 0, s>>>(ctl, (uint32_t)A.n));
@@ -1707,7 +1709,7 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
         if (kept && !ckr::profiling() && round_graph_launch(A, L, n_rounds, full, batch, s, &le)) return le;
         return batch(s, n_rounds, full);
     };
-    uint32_t full_until = A.recount_each_round ? R.rounds : first, stops = 0, ties = 0;
+    uint32_t full_until = A.recount == 1 ? R.rounds : first, stops = 0, ties = 0;
     for (uint32_t r = 0; A.build && r < R.rounds;) {
         const uint32_t n_rounds = r == 0 ? first : std::min(kRoundBatch, R.rounds - r);
         const uint32_t full = r < full_until ? n_rounds : 1;

@@ -542,7 +542,8 @@ CKR_API int ckr_make_contiguous(const void* d_src, int ndim, const int64_t* shap
  * 3: the same minimal slots, the overflowing units coded again by the fast
  * encoder with slots that hold any lane (mode 1's overflow route).  In
  * mode 0 the prefix-mask repair build also recounts every pair each round
- * instead of keeping the counts up to date.  The output bytes are identical in
+ * instead of keeping the counts up to date, in modes 2 and 3 whenever its pair
+ * table is 1/16 full instead of 3/4.  The output bytes are identical in
  * every mode; tests use this to cover all routes.  Process-wide; returns the
  * previous mode. ---- */
 CKR_API int ckr_set_fast_paths(int mode);

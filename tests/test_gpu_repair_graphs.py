@@ -40,3 +40,34 @@ def test_graphs_per_workspace(max_rules, gpu):
         assert np.array_equal(got["seq"], ref["seq"])
     made = ck.lib().ckr_repair_graphs_made() - before
     assert made <= 6, made
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("max_rules", [13, 30, 38])
+def test_recounts_within_lean_batches(max_rules, mode, gpu):
+    """Words without a tie among the pairs, so that lean batches run from the third
+    round on; in mode 2 the table's limit is passed every few rounds, the rest of the
+    batch leaves the sequence alone and the next full round counts again."""
+    import torch
+
+    import checkers_amd as ck
+    w = _ties_in(np.random.default_rng(3), PAIRS - 2)
+    raw = np.ascontiguousarray(w).view(np.uint8)
+    ref = oc.repair_build(raw, w.size, 2, ck.repair_masked_bits(1, None), max_rules, want_seq=True)
+    rp = ck.Repairer(w.size, 1, None, max_rules)
+    src = torch.from_numpy(raw.copy()).to(gpu)
+    old = ck.set_fast_paths(mode)
+    try:
+        for _ in range(2):
+            got = rp.build(src, want_seq=True)
+            assert got["rules"] == ref["rules"] and got["out_len"] == ref["out_len"]
+            assert np.array_equal(got["seq"], ref["seq"])
+        ck.profile_begin()  # (kernels one by one: what ran can be counted)
+        got = rp.build(src)
+        prof = ck.profile_end()
+    finally:
+        ck.set_fast_paths(old)
+    assert got["rules"] == ref["rules"]
+    lean = prof["repair_find_kernel"][0] - prof["repair_count_kernel"][0]
+    stopped = prof["repair_find_kernel"][0] - max_rules
+    assert lean > 0 and (stopped > 0 if mode == 2 else stopped == 0), prof
