@@ -32,19 +32,21 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kHistCopies = 16;  // 8, 16, 32 within 2%; 64 (a copy per lane) 35% slower
-// Loads in flight per thread.  Pass 2 with 4 takes 103 VGPRs, so half the waves
-// fit; with 2, held to 64 VGPRs, all 8 per SIMD.  2 is the better one for most
+// Loads in flight per thread.  Pass 2 with 4 takes 82 VGPRs (5 waves per SIMD);
+// with 2, held to 64 VGPRs, all 8 fit.  2 is the better one for most
 // calls, whose blocks fill the device (144 records of 1.53 GB in all: 592 us with
-// 2, 650 with 4; four records of 64 Mi fp32, 1 MiB per block: 371 and 428) or
-// are short (one of 1 Mi: 36.3 and 40.9).  4 where the loops are long: from
-// kLongBlock bytes per block of all calls on (four records of 1 Gi elements: 4742
-// us with 2, 4650 with 4), and from kLongBlockFew where one or two records leave
-// two waves per SIMD at most, which 2 loads each do not keep the memory busy with
-// (one record of 256 Mi fp32: 716 and 594; of 64 Mi, 169 and 163; of 16 Mi,
-// 256 KiB per block, 69.7 and 71.4).
+// 2, 650 with 4; four records of 64 Mi fp32, 1 MiB per block: 371 and 428; six of
+// 256 Mi bf16, 2 MiB per block of 1536: 1141 and 1229) or are short (one of 1 Mi:
+// 36.3 and 40.9).  4 where the loops are long and the blocks few, which 2 loads
+// each do not keep the memory busy with: kLongBlock bytes in the longest of up to
+// five blocks per CU (one record of 512 Mi fp32 beside 800 of 1 MB: 1717 us with 2,
+// 1505 with 4; three of 512 Mi bf16: 1342 and 1261), kLongBlockFew in up to two per
+// CU (one record of 256 Mi fp32: 719 and 612; of 64 Mi, 169 and 156; of 16 Mi, 256
+// KiB per block, 69.7 and 71.4), and in calls of about 4 GB and more (four records
+// of 1 Gi elements: 4742 us with 2, 4650 with 4).
 constexpr int kUnroll1 = 4;
 constexpr uint64_t kLongBlock = 2 << 20, kLongBlockFew = 512 << 10;
-constexpr uint64_t kFewBlocks = 512;  // two per CU
+constexpr uint64_t kSomeBlocks = 5 * 256, kFewBlocks = 2 * 256;
 // At most 256 workgroups per record, so that pass 2's closing global atomics
 // (one per histogram bin and workgroup) stay few (four records of 1G elements:
 // 2048 workgroups per record 5.18 ms per call; 512, 4.95; 256, 4.70; 128, 6.34).
@@ -216,7 +218,7 @@ __device__ __forceinline__ bool last_block(uint32_t* done, uint32_t nblk) {
 // The sum of one vector's elements in fp32 (at most 16 terms), then into the
 // fp64 total.
 template <uint32_t DT>
-__device__ void pass1_share(const StatsDesc& d, uint32_t lb, float& mn, float& mx, double& sm) {
+__device__ __forceinline__ void pass1_share(const StatsDesc& d, uint32_t lb, float& mn, float& mx, double& sm) {
     float part = 0.f;
     for_share<DT, kUnroll1>(
         d, lb,
@@ -283,8 +285,11 @@ __global__ void __launch_bounds__(kThreads) stats_pass1_kernel(StatsDesc* __rest
 
 // Central powers as the reference forms them (float d = x - mean), summed in
 // fp32 over one vector's elements, then into fp64 totals.
+// Inlined whatever its size: as a call (the compiler's choice for one of the five
+// dtypes) the LDS histogram was reached by flat atomics and the totals lay in
+// scratch, int8 with 4 loads 1131 us for 256 Mi elements against 323.
 template <uint32_t DT, int kUnroll2>
-__device__ void pass2_share(const StatsDesc& d, uint32_t lb, const StatsParams& q, uint32_t* sh, double& a2,
+__device__ __forceinline__ void pass2_share(const StatsDesc& d, uint32_t lb, const StatsParams& q, uint32_t* sh, double& a2,
                             double& a3, double& a4) {
     const uint32_t c = threadIdx.x & (kHistCopies - 1);
     const float mean = q.mean;
@@ -462,7 +467,9 @@ hipError_t launch_analyze(const ckr_stats_record* recs, uint64_t n, void* ws, hi
     }
     const uint32_t nr = (uint32_t)d.size();
     CKR_LAUNCH("stats_pass1_kernel", s, stats_pass1_kernel<<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, p1, prm));
-    if (per_block >= kLongBlock || (nb <= kFewBlocks && longest >= kLongBlockFew)) CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<4><<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
+    const bool long_loops = per_block >= kLongBlock || (nb <= kSomeBlocks && longest >= kLongBlock) ||
+                            (nb <= kFewBlocks && longest >= kLongBlockFew);
+    if (long_loops) CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<4><<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
     else CKR_LAUNCH("stats_pass2_kernel", s, stats_pass2_kernel<2><<<(uint32_t)nb, kThreads, 0, s>>>(desc, nr, prm, p2));
     return hipGetLastError();
 }

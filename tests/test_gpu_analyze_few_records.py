@@ -9,15 +9,17 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("sizes,dtype", [
     ([33_554_432 + 5], "float32"), ([33_550_000], "float32"), ([67_108_864 * 2 + 3], "bfloat16"),
     ([34_000_001, 33_999_999], "float32"), ([40_000_000, 5, 5], "float32"), ([9_000_000, 70_000_000], "bfloat16"),
+    ([134_300_000] + [77] * 900, "float32"), ([140_000_001], "int8"), ([33_600_003], "int32"),
 ])
 def test_long_shares(sizes, dtype, gpu):
     import torch
     import checkers_amd as ck
     dt = getattr(torch, dtype)
-    tag = ck.F32 if dt == torch.float32 else ck.BF16
+    tag = {"float32": ck.F32, "bfloat16": ck.BF16, "int8": ck.I8, "int32": ck.I32}[dtype]
     g = torch.Generator(device=gpu)
     g.manual_seed(len(sizes))
-    xs = [(torch.randn(n, generator=g, device=gpu) * 0.1 + 0.05).to(dt) for n in sizes]
+    scale = 0.1 if dt.is_floating_point else 30.0
+    xs = [(torch.randn(n, generator=g, device=gpu) * scale + scale / 2).to(dt) for n in sizes]
     a = ck.Analyzer(xs, [tag] * len(xs), 256)
     for _ in range(2):
         a.run()
