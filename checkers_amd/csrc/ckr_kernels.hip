@@ -4903,9 +4903,9 @@ hipError_t launch_decode(const uint8_t* data, const ckr_stream_header* hdrs, con
             // as if alone (1024 units of fp32 and a small int32 tensor: 111 us, with
             // one block less 123, as some SIMDs then have two waves).
             const uint64_t fit = (uint64_t)per_cu * (uint64_t)std::max(ncu, 1);
-            const uint64_t upb = g.spe ? DF_WAVES : DF_WAVES / 2;  // units that fill a block
-            const uint64_t need = 4 * g.n_units < 3 * all_units
-                                      ? std::max((g.n_units + upb - 1) / upb, fit * g.n_units / all_units) : g.n_units;
+            const uint64_t need = g.spe && 4 * g.n_units < 3 * all_units
+                                      ? std::max((g.n_units + DF_WAVES - 1) / DF_WAVES, fit * g.n_units / all_units)
+                                      : g.n_units;
             const uint32_t fg = (uint32_t)std::min({need, g.n_units, fit});
             if constexpr (std::is_same_v<decltype(kern), decltype(&decode_fast_unmasked_kernel)>)
                 CKR_LAUNCH("decode_fast_kernel", s, kern<<<fg, 64 * DF_WAVES, lb, s>>>(data, hdrs, unit_off, d_dec, g, dst, bad));
