@@ -1194,6 +1194,10 @@ int ckr_encode_planes(const void* d_src, uint64_t n_elems, int dtype, const ckr_
 namespace {
 constexpr int kUseHostTable = 1;  // compress_device_table: take the host's sorted table instead
 
+// The state chains have a row per coded symbol up to kChainSteps: the streams of
+// longer lanes are made on the host (canon_launch).
+bool chains_cover(const CanonKs& ck) { return std::max(ck.k0, ck.k1) <= ckr::kChainSteps; }
+
 // The symbol-0 state chains of every count (ckr::launch_canon_chains), one
 // buffer per device, kept for the process; made (8.4 MB, filled on a stream of
 // the library's own) by the first call with make set.  Null: none to use, the
@@ -1992,8 +1996,7 @@ int decode_impl(const uint8_t* d_data, const ckr_stream_header* d_headers, const
     // where the state chains cover the lane counts (units up to 64 KiB).  A
     // decode that the host does not wait for queues its work and nothing else:
     // it takes the chains only if they exist.
-    const void* chains = L.fast && !noalloc && std::max(ck.k0, ck.k1) <= ckr::kChainSteps
-                             ? canon_chains(s, h_bad_lanes != nullptr) : nullptr;
+    const void* chains = L.fast && !noalloc && chains_cover(ck) ? canon_chains(s, h_bad_lanes != nullptr) : nullptr;
     if (chains) {
         CKR_HIP(ckr::launch_dec_setup(ta, dec, canon, bad, ck.k0, ck.k1, ck.k2, ck.cw, chains, s));
     } else {
@@ -2132,8 +2135,8 @@ int ckr_decode_many(ckr_decode_job* jobs, uint64_t n, uint64_t unit_bytes, int c
         a->bad_jobs = n;
     }
     // A shard of small tensors that the fast decoder takes whole (masked
-    // dtypes of one kind or two, 4-byte aligned destinations; empty jobs have
-    // nothing to decode): one set-up
+    // dtypes of one kind or two, units of at most 64 KiB, 4-byte aligned
+    // destinations; empty jobs have nothing to decode): one set-up
     // launch for every job's decode table, canonical streams and bad-lane
     // counter, from the frequency tables uploaded in one copy, then one decode
     // launch over every job's units per dtype class, all on the caller's
@@ -2148,7 +2151,7 @@ int ckr_decode_many(ckr_decode_job* jobs, uint64_t n, uint64_t unit_bytes, int c
             all = decode_prepare(jb.d_data, jb.d_headers, jb.d_unit_offsets, jb.h_table, jb.n_elems, jb.dtype,
                                  unit_bytes, jb.d_sidecar, jb.d_dst, jb.d_workspace, jb.workspace_bytes, pp[i]) == CKR_OK &&
                   (pp[i].g.n_units == 0 ||
-                   (pp[i].L.fast && !use_long_units(pp[i].g) && aligned_to(jb.d_dst, 4)));
+                   (pp[i].L.fast && chains_cover(canon_ks(pp[i].g)) && aligned_to(jb.d_dst, 4)));
         }
         const void* chains = all ? canon_chains(s) : nullptr;
         if (all && chains) {

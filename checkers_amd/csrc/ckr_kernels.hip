@@ -4826,6 +4826,7 @@ hipError_t launch_build_dec_table(const TableArg& t, uint32_t* d_dec, unsigned l
 
 hipError_t launch_dec_setup(const TableArg& t, uint32_t* d_dec, uint32_t* canon, unsigned long long* bad, uint32_t k0,
                             uint32_t k1, uint32_t k2, uint32_t cw, const void* chains, hipStream_t s) {
+    if (std::max({k0, k1, k2}) > kChainSteps) return hipErrorInvalidValue;
     CKR_LAUNCH("dec_setup_kernel", s, dec_setup_kernel<<<16, 256, 0, s>>>(t, d_dec, canon, bad, k0, k1, k2, cw, chains_of(chains)));
     return hipGetLastError();
 }
@@ -4836,7 +4837,10 @@ hipError_t launch_dec_setup_multi(const DecSetupJob* jobs, uint32_t n, const voi
     for (uint32_t j0 = 0; j0 < n; j0 += kMaxDecJobs) {
         DecSetupJobs J{};
         J.n = std::min<uint32_t>(kMaxDecJobs, n - j0);
-        for (uint32_t k = 0; k < J.n; k++) J.j[k] = jobs[j0 + k];
+        for (uint32_t k = 0; k < J.n; k++) {
+            J.j[k] = jobs[j0 + k];
+            if (std::max({J.j[k].k0, J.j[k].k1, J.j[k].k2}) > kChainSteps) return hipErrorInvalidValue;
+        }
         CKR_LAUNCH("dec_setup_multi_kernel", s, dec_setup_multi_kernel<<<16 * J.n, 256, 0, s>>>(J, chains_of(chains)));
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
