@@ -1490,6 +1490,11 @@ hipError_t build_alphabet(const uint8_t* words, uint64_t n, int es, uint32_t k, 
 }
 
 constexpr uint32_t kRoundBatch = 8;
+// The next pair's count from which a batch is lean: below it ties are common, and a
+// lean batch that a tie stops costs another batch and read-back (10 rules of 3000
+// bf16 words: 478 us with full rounds only, 504 lean from the third round on, 438
+// by this rule; of 2 Mi words, whose counts are large, 513 and 464).
+constexpr uint32_t kLeanCount = 64;
 
 // The captured graphs of a batch of build rounds, keyed by what their kernels'
 // arguments derive from (the workspace and its layout's inputs), the batch length
@@ -1694,7 +1699,7 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
     // k-th such stop the next 16 << k rounds are full ones.  Tensors whose
     // rounds tie (few words, or many that are all rare) tie from the start: the
     // first batch is two full rounds, and lean batches follow batches without a
-    // tie only.
+    // tie only, while the counts are kLeanCount or more.
     //
     // Graphs have one of three lengths, so that the data decides which are launched
     // but not which there are: the first batch's (all rounds of a build of no more
@@ -1709,10 +1714,10 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
         if (kept && !ckr::profiling() && round_graph_launch(A, L, n_rounds, full, batch, s, &le)) return le;
         return batch(s, n_rounds, full);
     };
-    uint32_t full_until = A.recount == 1 ? R.rounds : first, stops = 0, ties = 0;
+    uint32_t full_until = A.recount == 1 ? R.rounds : first, stops = 0, ties = 0, best = ~0u;
     for (uint32_t r = 0; A.build && r < R.rounds;) {
         const uint32_t n_rounds = r == 0 ? first : std::min(kRoundBatch, R.rounds - r);
-        const uint32_t full = r < full_until ? n_rounds : 1;
+        const uint32_t full = r < full_until || best < kLeanCount ? n_rounds : 1;
         if ((e = launch(n_rounds, full)) != hipSuccess) return e;
         if (full == n_rounds && r + n_rounds >= R.rounds) break;  // no round of it can have been left out
         RepairCtl now{};
@@ -1722,6 +1727,7 @@ hipError_t run_rounds(const RepairArgs& A, hipStream_t s) {
         if (now.round < r + n_rounds) full_until = now.round + (16u << std::min(stops++, 10u));
         else if (now.ties != ties) full_until = std::max(full_until, now.round + kRoundBatch);
         ties = now.ties;
+        best = now.best;
         r = now.round;
     }
     // the live tokens counted per block and scanned: the output's offsets, and

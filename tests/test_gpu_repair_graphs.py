@@ -71,3 +71,24 @@ def test_recounts_within_lean_batches(max_rules, mode, gpu):
     lean = prof["repair_find_kernel"][0] - prof["repair_count_kernel"][0]
     stopped = prof["repair_find_kernel"][0] - max_rules
     assert lean > 0 and (stopped > 0 if mode == 2 else stopped == 0), prof
+
+
+def test_small_counts_take_full_rounds(gpu):
+    """Top counts below 64, where ties are common: no lean round is tried, so that a
+    tie costs no extra batch."""
+    import torch
+
+    import checkers_amd as ck
+    rng = np.random.default_rng(2)
+    counts = 60 - np.arange(20)
+    counts[6] = counts[5]
+    which = rng.permutation(np.repeat(np.arange(20), counts))
+    w = np.stack([2 * which + 1, 2 * which + 2], 1).reshape(-1).astype(np.uint16) << 7
+    raw = np.ascontiguousarray(w).view(np.uint8)
+    ref = oc.repair_build(raw, w.size, 2, ck.repair_masked_bits(1, None), 18)
+    rp = ck.Repairer(w.size, 1, None, 18)
+    ck.profile_begin()
+    got = rp.build(torch.from_numpy(raw.copy()).to(gpu))
+    prof = ck.profile_end()
+    assert got["rules"] == ref["rules"]
+    assert prof["repair_find_kernel"][0] == prof["repair_count_kernel"][0] == 18
