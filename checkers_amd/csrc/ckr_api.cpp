@@ -1199,15 +1199,17 @@ constexpr int kUseHostTable = 1;  // compress_device_table: take the host's sort
 bool chains_cover(const CanonKs& ck) { return std::max(ck.k0, ck.k1) <= ckr::kChainSteps; }
 
 // The symbol-0 state chains of every count (ckr::launch_canon_chains), one
-// buffer per device, kept for the process; made (8.4 MB, filled on a stream of
-// the library's own) by the first call with make set.  Null: none to use, the
-// callers have paths that do without.  The host never waits here: until the
-// fill is known to be complete, the caller's stream is made to wait for it.
+// buffer per device, kept for the process; made (8.4 MB) by the first call with
+// make set, and filled on its stream.  Null: none to use, the callers have paths
+// that do without.  The host never waits here, and no stream for another's work:
+// until the fill is known to be complete the chains serve the stream that it went
+// to only.  (A stream of the library's own for the fill made every later launch of
+// the process slower, the decode's set-up 4.5 to 5.4 us: a second queue in use.)
 const void* canon_chains(hipStream_t s, bool make = true) {
     struct PerDevice {
         void* p = nullptr;
-        hipStream_t fill = nullptr;    // while the fill may still run
-        hipEvent_t filled = nullptr;
+        hipEvent_t filled = nullptr;  // while the fill may still run, on
+        hipStream_t on = nullptr;
     };
     static std::mutex mu;
     static std::vector<PerDevice> per_dev;
@@ -1224,32 +1226,30 @@ const void* canon_chains(hipStream_t s, bool make = true) {
         (void)hipGetLastError();
         return nullptr;
     }
-    const void* r = nullptr;
-    auto settle = [&]() {  // the stream and the event are not needed any more
-        if (c.filled) (void)hipEventDestroy(c.filled);
-        if (c.fill) (void)hipStreamDestroy(c.fill);
-        c.filled = nullptr;
-        c.fill = nullptr;
-    };
     if (!c.p) {
         void* p = nullptr;
         if (hipMalloc(&p, ckr::kChainBytes) == hipSuccess &&
-            hipStreamCreateWithFlags(&c.fill, hipStreamNonBlocking) == hipSuccess &&
             hipEventCreateWithFlags(&c.filled, hipEventDisableTiming) == hipSuccess &&
-            ckr::launch_canon_chains(p, c.fill) == hipSuccess && hipEventRecord(c.filled, c.fill) == hipSuccess) {
+            ckr::launch_canon_chains(p, s) == hipSuccess && hipEventRecord(c.filled, s) == hipSuccess) {
             c.p = p;
-        } else {
-            settle();
-            if (p) (void)hipFree(p);
+            c.on = s;
+            return p;
         }
+        (void)hipGetLastError();
+        if (c.filled) (void)hipEventDestroy(c.filled);
+        c.filled = nullptr;
+        if (p) (void)hipFree(p);
+        return nullptr;
     }
-    if (c.p) {
-        const hipError_t q = hipEventQuery(c.filled);
-        if (q == hipSuccess) settle();
-        if (q == hipSuccess || (q == hipErrorNotReady && hipStreamWaitEvent(s, c.filled, 0) == hipSuccess)) r = c.p;
+    const hipError_t q = hipEventQuery(c.filled);
+    if (q == hipSuccess) {
+        (void)hipEventDestroy(c.filled);
+        c.filled = nullptr;
+        return c.p;
     }
     (void)hipGetLastError();
-    return r;
+    // (the wait costs nothing where s is that stream; its handle may be a later one's)
+    return q == hipErrorNotReady && s == c.on && hipStreamWaitEvent(s, c.filled, 0) == hipSuccess ? c.p : nullptr;
 }
 
 // A tensor's encode with the table built on the device (tensors the fast

@@ -12,6 +12,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _run():
+    import threading
+    import time
+
     import torch
     import checkers_amd as ck
     x = torch.randn(100_003, device="cuda") * 1e-3
@@ -44,16 +47,32 @@ def _run():
     assert torch.cuda.mem_get_info()[0] == free, "the call allocated"
     assert torch.equal(dst, x.view(torch.uint8))
 
-    # counting decodes make the chains and use them, on two streams
-    other = torch.cuda.Stream()
-    other.wait_stream(torch.cuda.current_stream())
+    # a counting decode on another thread makes the chains behind long work; one on
+    # this thread and another stream neither waits for that nor uses them
+    i8 = ck.compress(torch.ones(1000, dtype=torch.int8, device="cuda"), ck.I8, 256)
+    dst.zero_()
     out2 = torch.zeros_like(dst)
     d2 = ck.Decoder(x.numel(), ck.F32, 65536)
+    busy, other, bad = torch.cuda.Stream(), torch.cuda.Stream(), []
+    assert ck.decode(i8)[1] == 0  # (this thread's read-back buffer, by a dtype without chains)
     torch.cuda.synchronize()
-    bad = d.decode(*args), d2.decode(*args[:-1], out2, stream=other)
+    with torch.cuda.stream(busy):
+        for _ in range(200):
+            big.mul_(1.0)
+        before = torch.cuda.Event()
+        before.record()
+    free = torch.cuda.mem_get_info()[0]
+    th = threading.Thread(target=lambda: bad.append(d.decode(*args, stream=busy)), daemon=True)
+    th.start()
+    while torch.cuda.mem_get_info()[0] == free and not before.query():
+        time.sleep(0.001)
+    made_early = not before.query()
+    assert d2.decode(*args[:-1], out2, stream=other) == 0
+    waited = before.query()
+    th.join(30)
+    assert made_early and not waited, "a call waited for another stream's work"
     torch.cuda.synchronize()
-    assert bad == (0, 0) and torch.equal(dst, x.view(torch.uint8)) and torch.equal(out2, x.view(torch.uint8))
-    assert torch.cuda.mem_get_info()[0] < free
+    assert bad == [0] and torch.equal(dst, x.view(torch.uint8)) and torch.equal(out2, x.view(torch.uint8))
     for _ in range(3):
         dst.zero_()
         assert d.decode(*args) == 0 and torch.equal(dst, x.view(torch.uint8))
