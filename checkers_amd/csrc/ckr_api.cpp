@@ -256,10 +256,12 @@ hipError_t canon_launch(const ckr_freq_table* t, const CanonKs& ck, uint32_t* ca
 // 1 KiB units 92 (89) and 161 (220); 2 KiB 84 (81) and 94 (108); 4 KiB 85 (81) and
 // 70 (73); 8 KiB 97 (91) and 64 (65).  The fewer the units, the shorter those that
 // the fast encoder leads with (1 MB in 1 KiB units 68 (67) and 71 (84), in 2 KiB
-// units 69 (66) and 61 (60); 16 MB in 4 KiB units 142 (114) and 154 (160)).
+// units 69 (66) and 61 (60); 16 MB in 4 KiB units 142 (114) and 154 (160)).  A
+// unit alone waits for no other: 1000 bytes 58 (57) and 42 (70 where the ranks
+// leave the table to the sort), 300 bytes 56 (54) and 64..75 (124..141).
 bool long_unmasked_units(const ckr::EncodeGeom& g) {
     const uint64_t K = (g.unit + 255) / 256;
-    return K >= 32 || (K >= 8 && g.n_units <= 64 * K);
+    return K >= 32 || (K >= 8 && g.n_units <= 64 * K) || (K >= 4 && g.n_units == 1);
 }
 bool use_fast_encode(const ckr::EncodeGeom& g) {
     return g_fast_paths && g.n_units > 0 && (g.unit + 255) / 256 <= kFastMaxK && (g.spe || long_unmasked_units(g));

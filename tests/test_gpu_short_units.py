@@ -15,12 +15,12 @@ pytestmark = pytest.mark.gpu
     (256, 40, False, False), (256, 3000, False, False), (1024, 300, False, False), (1792, 90, False, False),
     (2048, 512, True, False), (2048, 513, False, False), (2816, 100, True, False), (3072, 100, True, True),
     (4096, 1024, True, True), (4096, 1025, False, True), (7936, 1985, False, True), (8192, 2100, True, True),
-    (65536, 0, False, False),  # one unit of a few bytes
+    (65536, 0, True, False), (1024, 0, True, False), (768, 0, False, False),  # one unit of a few bytes
 ])
 def test_routes(dt, unit, units, fast_enc, fast_dec, gpu):
     import torch
     import checkers_amd as ck
-    nb = max(units - 1, 0) * unit + (unit // 2 + 4 if units else 1252)
+    nb = max(units - 1, 0) * unit + (unit // 2 + 4 if units else min(unit, 1252))
     rng = np.random.default_rng(units)
     raw = np.minimum(rng.geometric(0.1, nb), 255).astype(np.uint8)
     n = nb // (4 if dt == dg.I32 else 1)
