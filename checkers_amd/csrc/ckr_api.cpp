@@ -1255,7 +1255,7 @@ const void* canon_chains(hipStream_t s, bool make = true) {
 }
 
 // A tensor's encode with the table built on the device (tensors the fast
-// encoder takes, small int8 and int32 ones aside): from its histograms
+// encoder takes): from its histograms
 // in device memory, the table by ranks, encode entries, canonical streams and
 // slot sizes, and the encode are queued with no host round trip, and the
 // control words and the table are read back into pinned words.  After the
@@ -1281,18 +1281,19 @@ struct DevEnc {
     bool redo_queued = false;  // the list-mode redo pass follows the encode on its stream
 };
 
-// Small tensors without zero planes take the host's table: few symbols' counts
-// differ, so that the ranks leave the table to the sort in most of them (of int8
-// and int32 distributions of 1 to 64 KB 50 to 90%, of 100 to 250 KB 35 to 70%) and
-// the tensor is then counted and coded twice.  Compress of 3000 bytes of int8: 41
-// us by ranks, 85 where they fail, 54 by the host's table.
+// A shard with small tensors without zero planes takes the host's tables: few of
+// such a tensor's symbol counts differ, so that the ranks leave the table to the
+// sort in most of them (of int8 and int32 distributions of 1 to 64 KB 50 to 90%, of
+// 100 to 250 KB 35 to 70%), and each is then coded again behind the shard (three
+// bf16 tensors of up to 200 KB with four int32 tensors of 3000 elements: 333 us
+// against 276).
 constexpr uint64_t kUnmaskedHostTableBytes = 256 << 10;
 
 // Whether the device table can serve this tensor, and its encode parameters
 // (dctl: null for the workspace's own control words).
 bool dev_enc_setup(DevEnc& d, const void* src, const ckr::EncodeGeom& g, uint8_t* ws, uint8_t* out,
                    ckr_stream_header* hdrs, uint64_t* unit_off, uint8_t* side, uint32_t* dctl, uint32_t* pin) {
-    if (g_fast_paths != 1 || !use_fast_encode(g) || (g.spe == 0 && g.n_bytes <= kUnmaskedHostTableBytes)) return false;
+    if (g_fast_paths != 1 || !use_fast_encode(g)) return false;
     d.src = static_cast<const uint8_t*>(src);
     d.g = g;
     d.L = encode_layout(g);
@@ -1337,7 +1338,8 @@ int dev_enc_queue_encode(const DevEnc& d, hipStream_t s) {
 
 // The encode and, right behind it with no read-back between them, the redo
 // pass (it ends at once when no unit outgrew its slots), which also writes the
-// control and table words to d.pin; where it does not fit, a copy does.
+// control and table words, and an ambiguous table's histograms, to d.pin
+// (kCtlWords + 768 words); where it does not fit, copies do.
 int dev_enc_queue_encode_redo(DevEnc& d, hipStream_t s) {
     if (int rc = dev_enc_queue_encode(d, s)) return rc;
     const uint32_t lds_limit = (uint32_t)max_lds_per_block();
@@ -1346,10 +1348,12 @@ int dev_enc_queue_encode_redo(DevEnc& d, hipStream_t s) {
         CKR_HIP(ckr::launch_encode_fast_list(d.src, d.g, reinterpret_cast<ckr::EncSym*>(d.ws + L.off_enc),
                                              reinterpret_cast<uint32_t*>(d.ws + L.off_canon), d.fp, lds_limit, d.hdrs,
                                              d.out, d.unit_off, reinterpret_cast<uint64_t*>(d.ws + L.off_status), d.dctl,
-                                             reinterpret_cast<uint32_t*>(d.ws + L.off_redo), s, d.pin, kCtlWords));
+                                             reinterpret_cast<uint32_t*>(d.ws + L.off_redo), s, d.pin, kCtlWords,
+                                             reinterpret_cast<uint32_t*>(d.ws + L.off_hist)));
         d.redo_queued = true;
     } else {
         CKR_HIP(hipMemcpyAsync(d.pin, d.dctl, kCtlWords * 4, hipMemcpyDeviceToHost, s));
+        CKR_HIP(hipMemcpyAsync(d.pin + kCtlWords, d.ws + d.L.off_hist, 768 * 4, hipMemcpyDeviceToHost, s));
     }
     return CKR_OK;
 }
@@ -1416,11 +1420,14 @@ int dev_enc_finish(const DevEnc& d, ckr_freq_table* h_table, uint64_t* h_total, 
 }
 
 // ckr_compress through the device table: histogram, queue, one synchronisation.
-// check_outputs: the output buffers' checks, made while the histogram runs.
+// check_outputs: the output buffers' checks, made while the histogram runs.  With
+// kUseHostTable *hists is the tensor's histograms (768 words, in pinned memory) if
+// they have been counted.
 int compress_device_table(const void* src, const ckr::EncodeGeom& g, int ensure_full_alphabet, uint8_t* d_out,
                           ckr_stream_header* d_headers, uint64_t* d_unit_offsets, uint8_t* d_sidecar, uint8_t* ws,
                           ckr_freq_table* h_table, uint64_t* h_total_out, hipStream_t s,
-                          const std::function<int()>& check_outputs) {
+                          const std::function<int()>& check_outputs, const uint32_t** hists) {
+    static_assert(kCtlWords + 768 <= kPinnedWords, "control words and histograms in one read-back");
     uint32_t* pw = pinned_words();
     if (!pw) return fail(CKR_E_HIP, "[ckr] pinned host buffer unavailable");
     DevEnc d;
@@ -1447,6 +1454,7 @@ int compress_device_table(const void* src, const ckr::EncodeGeom& g, int ensure_
     bool more = false;
     rc = dev_enc_finish(d, h_table, h_total_out, &more, s);
     if (rc == CKR_OK && more) CKR_HIP(hipStreamSynchronize(s));  // the output complete, as on the other paths
+    if (rc == kUseHostTable) *hists = pw + kCtlWords;
     return rc;
 }
 }  // namespace
@@ -1476,9 +1484,10 @@ int ckr_compress(const void* d_src, uint64_t n_elems, int dtype, uint64_t unit_b
     if ((rc = st.make(d_src, g.n_bytes, s))) return rc;
     // the fast encoder's tensors: the table on the device, no host round trip
     // before the encode (mode 1; modes 2 and 3 size the slots on the host)
+    const uint32_t* counted = nullptr;  // the histograms, where the ranks left the table to the sort
     if (g_fast_paths == 1 && use_fast_encode(g)) {
         rc = compress_device_table(st.p, g, ensure_full_alphabet, d_out, d_headers, d_unit_offsets, d_sidecar,
-                                   static_cast<uint8_t*>(d_workspace), h_table, h_total_out, s, check_outputs);
+                                   static_cast<uint8_t*>(d_workspace), h_table, h_total_out, s, check_outputs, &counted);
         if (rc != kUseHostTable) {
             st.release(s);
             return rc;
@@ -1488,20 +1497,23 @@ int ckr_compress(const void* d_src, uint64_t n_elems, int dtype, uint64_t unit_b
         st.release(s);
         return rc;
     }
-    uint32_t* d_hist = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(d_workspace) + L.off_hist);
-    const int es = ckr_element_size(dtype);
-    hipError_t he = ckr::launch_masked_hist(static_cast<const uint8_t*>(st.p), n_elems * (uint64_t)es, es, g.spe, d_hist,
-                                            d_hist + 256, s);
-    uint32_t* pw = pinned_words();
-    if (he == hipSuccess && pw) he = hipMemcpyAsync(pw, d_hist, 768 * 4, hipMemcpyDeviceToHost, s);
-    if (he == hipSuccess && pw) he = hipStreamSynchronize(s);
-    if (he != hipSuccess || !pw) {
-        st.release(s);
-        return pw ? fail(CKR_E_HIP, "[ckr] histogram failed: %s", hipGetErrorString(he))
-                  : fail(CKR_E_HIP, "[ckr] pinned host buffer unavailable");
+    if (!counted) {
+        uint32_t* d_hist = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(d_workspace) + L.off_hist);
+        const int es = ckr_element_size(dtype);
+        hipError_t he = ckr::launch_masked_hist(static_cast<const uint8_t*>(st.p), n_elems * (uint64_t)es, es, g.spe,
+                                                d_hist, d_hist + 256, s);
+        uint32_t* pw = pinned_words();
+        if (he == hipSuccess && pw) he = hipMemcpyAsync(pw, d_hist, 768 * 4, hipMemcpyDeviceToHost, s);
+        if (he == hipSuccess && pw) he = hipStreamSynchronize(s);
+        if (he != hipSuccess || !pw) {
+            st.release(s);
+            return pw ? fail(CKR_E_HIP, "[ckr] histogram failed: %s", hipGetErrorString(he))
+                      : fail(CKR_E_HIP, "[ckr] pinned host buffer unavailable");
+        }
+        counted = pw;
     }
     uint32_t hh[768];
-    std::memcpy(hh, pw, sizeof(hh));
+    std::memcpy(hh, counted, sizeof(hh));
     ckr_freq_table local;
     ckr_freq_table* t = h_table ? h_table : &local;
     rc = ckr_build_table(hh, ensure_full_alphabet, t, nullptr);
@@ -1715,7 +1727,8 @@ int ckr_compress_many(ckr_compress_job* jobs, uint64_t n, uint64_t unit_bytes, i
         }
         bool all = true;
         for (uint64_t i = 0; i < n && all; i++)
-            all = dev_enc_setup(dv[i], staged[i].p, geo[i], static_cast<uint8_t*>(jobs[i].d_workspace), jobs[i].d_out,
+            all = (geo[i].spe || geo[i].n_bytes > kUnmaskedHostTableBytes) &&
+                  dev_enc_setup(dv[i], staged[i].p, geo[i], static_cast<uint8_t*>(jobs[i].d_workspace), jobs[i].d_out,
                                 jobs[i].d_headers, jobs[i].d_unit_offsets, jobs[i].d_sidecar,
                                 a->d_tslots + kCtlWords * i, a->tslots + kCtlWords * i);
         chains = all ? canon_chains(a->s2) : nullptr;

@@ -148,13 +148,13 @@ uint32_t encode_fast_lds_bytes(const FastEncParamsHost& p, uint32_t lds_limit);
 // workgroup with slots that hold any lane; false/error when those slots do not
 // fit lds_limit.  report (may be null): pinned host memory that receives
 // ctl[0 .. n_report) as they are when the launch begins, in place of a copy
-// behind it.
+// behind it, and then, if the table's words say that it is ambiguous, hist's 768.
 bool encode_fast_list_fits(const FastEncParamsHost& p, const EncodeGeom& g, uint32_t lds_limit);
 hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, const EncSym* d_enc, const uint32_t* canon,
                                    const FastEncParamsHost& hp, uint32_t lds_limit, ckr_stream_header* hdrs,
                                    uint8_t* out, uint64_t* unit_off, uint64_t* status, uint32_t* ctl,
                                    uint32_t* redo_list, hipStream_t s, uint32_t* report = nullptr,
-                                   uint32_t n_report = 0);
+                                   uint32_t n_report = 0, uint32_t* hist = nullptr);
 // Several tensors' fast encodes in one launch (same spe, sidecars for all or
 // none, tables the data's own): each job's arguments as launch_encode_fast's,
 // dsl its device slot sizes (sl0, sl1: the largest the launch's LDS holds);

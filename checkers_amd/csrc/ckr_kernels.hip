@@ -1668,7 +1668,9 @@ __host__ __device__ constexpr uint32_t ws_lds_bytes(uint32_t pairs, uint32_t can
 // no look-back.  A lane that outgrew even those slots would set ctl[2] bit 1.
 // 256 such slots (int8, int32) fill the LDS once, not twice: one slot set, coded
 // and packed in turn.
-// report (LIST): ctl[0 .. n_report) as they are at the launch, copied there first.
+// report (LIST): ctl[0 .. n_report) as they are at the launch, copied there first,
+// and behind them, where the ranks left the table to the sort, the 768 histogram
+// words at sidecar (which list mode has no other use for), for the host's table.
 template <int SPE, bool ESC, bool SIDE, int PAIRS, int NPK, bool LIST>
 __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src, EncodeGeom g,
                                                  const EncSym* __restrict__ d_enc,
@@ -1681,8 +1683,12 @@ __device__ __forceinline__ void encode_fast_body(const uint8_t* __restrict__ src
                                                  uint64_t* __restrict__ phase,
                                                  const uint32_t* __restrict__ dsl, uint32_t* report,
                                                  uint32_t n_report) {
-    if (LIST && report && blockIdx.x == 0)  // (see launch_encode_fast_list)
+    if (LIST && report && blockIdx.x == 0) {  // (see launch_encode_fast_list)
         for (uint32_t i = threadIdx.x; i < n_report; i += blockDim.x) report[i] = ctl[i];
+        if (sidecar && ctl[8 + 257])
+            for (uint32_t i = threadIdx.x; i < 768; i += blockDim.x)
+                report[n_report + i] = reinterpret_cast<const uint32_t*>(sidecar)[i];
+    }
     if (LIST && __hip_atomic_load(&ctl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;  // nothing to redo
     if (dsl) {  // slot sizes made on the device (table_enc_kernel), within the launch's LDS
         fp.sl0 = dsl[0]; fp.sl1 = dsl[1];
@@ -2240,7 +2246,8 @@ bool encode_fast_list_fits(const FastEncParamsHost& hp, const EncodeGeom& g, uin
 hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, const EncSym* d_enc, const uint32_t* canon,
                                    const FastEncParamsHost& hp, uint32_t lds_limit, ckr_stream_header* hdrs,
                                    uint8_t* out, uint64_t* unit_off, uint64_t* status, uint32_t* ctl,
-                                   uint32_t* redo_list, hipStream_t s, uint32_t* report, uint32_t n_report) {
+                                   uint32_t* redo_list, hipStream_t s, uint32_t* report, uint32_t n_report,
+                                   uint32_t* hist) {
     if (!encode_fast_list_fits(hp, g, lds_limit)) return hipErrorInvalidValue;
     FastEncParams fp;
     fp.sl0 = fp.sl1 = encode_fast_list_slot(g);
@@ -2257,8 +2264,8 @@ hipError_t launch_encode_fast_list(const uint8_t* src, const EncodeGeom& g, cons
         if (r != hipSuccess) return r;
         const uint32_t grid = (uint32_t)std::min<uint64_t>(g.n_units, (uint64_t)std::max(ncu, 1));
         CKR_LAUNCH("encode_fast_redo_kernel", s,
-                   kern<<<grid, nthreads, lb, s>>>(src, g, d_enc, canon, fp, hdrs, nullptr, out, unit_off, status, ctl,
-                                                   redo_list, nullptr, nullptr, report, n_report));
+                   kern<<<grid, nthreads, lb, s>>>(src, g, d_enc, canon, fp, hdrs, reinterpret_cast<uint8_t*>(hist), out,
+                                                   unit_off, status, ctl, redo_list, nullptr, nullptr, report, n_report));
         return hipGetLastError();
     };
     if (g.spe == 0)

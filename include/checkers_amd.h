@@ -193,10 +193,10 @@ CKR_API int ckr_encode_planes(const void* d_src, uint64_t n_elems, int dtype,
 /* ---- full tensor compression as ANSCompressor::compress_tensor does it for a
  * singleton (histogram → table → encode), in one call.  The table built is
  * returned in h_table (may be NULL).  The workspace (16-byte aligned) as for
- * ckr_encode.  For tensors with units of at most 64 KiB (int8 and int32: above
- * 256 KiB) the table is built on the device from the histogram in the same launch (the
- * reference's normalisation, by ranks; a table whose correction falls inside
- * a group of equal fractional parts is taken from the host's sort instead),
+ * ckr_encode.  For tensors with units of at most 64 KiB the table is built on
+ * the device from the histogram in the same launch (the reference's
+ * normalisation, by ranks; a table whose correction falls inside a group of
+ * equal fractional parts is taken from the host's sort instead),
  * and the output buffers are checked while that launch runs: a bad output
  * buffer is reported once it has finished, with only the workspace written.
  * ---- */
