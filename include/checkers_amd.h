@@ -536,12 +536,14 @@ CKR_API int ckr_make_contiguous(const void* d_src, int ndim, const int64_t* shap
  * fast kernels — lanes of masked planes coded once per lane count (their
  * streams are identical), units of at most 64 KiB coded and decoded through
  * LDS; mode 0: every lane coded and decoded independently through global
- * memory (modes 1 to 3 take int8 and int32, which have no masked planes, the same way
- * as the other dtypes, units of fewer than 32 rows of 256 bytes aside); mode 2: fast kernels with minimal LDS lane slots, so that nearly
- * every unit takes the overflow route back through the general kernels; mode
- * 3: the same minimal slots, the overflowing units coded again by the fast
- * encoder with slots that hold any lane (mode 1's overflow route).  In
- * mode 0 the prefix-mask repair build also recounts every pair each round
+ * memory (modes 1 to 3 take int8 and int32, which have no masked planes, the
+ * same way as the other dtypes, but for short units, ckr_encode without
+ * h_total_out, encodes in units above 64 KiB and decodes above 1 MiB, which
+ * stay with these kernels); mode 2: fast kernels with minimal LDS lane slots,
+ * so that nearly every unit takes the overflow route back through the general
+ * kernels; mode 3: the same minimal slots, the overflowing units coded again
+ * by the fast encoder with slots that hold any lane (mode 1's overflow route).
+ * In mode 0 the prefix-mask repair build also recounts every pair each round
  * instead of keeping the counts up to date, in modes 2 and 3 whenever its pair
  * table is 1/16 full instead of 3/4.  The output bytes are identical in
  * every mode; tests use this to cover all routes.  Process-wide; returns the
